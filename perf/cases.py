@@ -64,7 +64,7 @@ def listed():
         # the workload the engine is quoted on (16 orbitals, 12 modes, 7^3 boxes), whole pass over a grid
         dict(name="eph_main", **_eph_case("eph_k", 16, 4, 9, 7, (20, 20, 20), (20, 20, 20), 0.3)),
         # a wide window (hot carriers, optics): five and more bands per k; reduced Fourier precision
-        dict(name="eph_wide", **_eph_case("eph_k", 16, 4, 7, 5, (16, 16, 16), (8, 8, 8), 1.0, "bf16x3")),
+        dict(name="eph_wide", **_eph_case("eph_k", 16, 4, 7, 5, (16, 16, 16), (8, 8, 8), 1.8, "bf16x3")),
         # one tile of 16 q of the outer-q loop (self-energies at chosen q, phonon linewidths)
         dict(name="eph_outer_q", **_eph_case("eph_q", 16, 4, 9, 7, (24, 24, 24), (12, 12, 12), 0.3, ntile=16)),
         # scattering rates and rows at three temperatures from an e-ph payload
