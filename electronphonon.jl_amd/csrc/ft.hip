@@ -161,7 +161,10 @@ __global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, con
     if constexpr (kSep) {
         ax = ft_axes(irvec, nr, red);
         use_tab = ax.total <= FT_TAB_MAX;
-        if (use_tab) ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+        if (use_tab) {
+            ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+            __syncthreads();  // a column's rows are written by 256 / TN waves and read by each of them
+        }
     }
 
     // The phase column this thread generates is fixed for the whole kernel; its R rows are uniform
@@ -446,7 +449,10 @@ __global__ __launch_bounds__(256) void ft_bf16x3_kernel(int64_t ndata, int nr, c
     }
     const FtAxes ax = ft_axes(irvec, nr, red);
     const bool use_tab = ax.total <= FT_TAB_MAX;
-    if (use_tab) ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+    if (use_tab) {
+        ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+        __syncthreads();  // a column's rows are written by 256 / TN waves and read by each of them
+    }
 
     const int pj = tid % TN;
     const int prl0 = __builtin_amdgcn_readfirstlane(tid / TN);
