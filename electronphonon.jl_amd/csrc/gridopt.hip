@@ -94,8 +94,8 @@ __global__ __launch_bounds__(256) void gridopt_stage1_kernel(int64_t nd, int n1,
         dd = j + nb * (i + nb * rest);
     }
     const cplx<float> *o = op + d;
-#pragma unroll 1
-    for (int c = 0; c < np; c++)
+    {
+        const int c = blockIdx.y;  // the np face rows are independent: small operators get np times the workgroups
 #pragma unroll 1
         for (int b = 0; b < np; b++) {
             float sr[P], si[P];
@@ -124,6 +124,7 @@ __global__ __launch_bounds__(256) void gridopt_stage1_kernel(int64_t nd, int n1,
 #pragma unroll
             for (int p = 0; p < P; p++) pl.op1[p][dd + nd * (b + np * c)] = cplx<float>{sr[p], si[p]};
         }
+    }
 }
 
 // Stages 2 and 3 with the window projection, for the k of one k1 plane. One thread per row d'
@@ -550,7 +551,7 @@ extern "C" int ephip_gridopt_stage1_planes(int64_t nd, int32_t n1, int32_t n2, i
     static const K kern[GO_PLANES_MAX] = {gridopt_stage1_kernel<1>, gridopt_stage1_kernel<2>, gridopt_stage1_kernel<3>,
                                           gridopt_stage1_kernel<4>, gridopt_stage1_kernel<5>, gridopt_stage1_kernel<6>,
                                           gridopt_stage1_kernel<7>, gridopt_stage1_kernel<8>};
-    kern[nplanes - 1]<<<(unsigned)((nd + 255) / 256), 256, 0, as_stream(stream)>>>(
+    kern[nplanes - 1]<<<dim3((unsigned)((nd + 255) / 256), (unsigned)np), 256, 0, as_stream(stream)>>>(
         nd, n1, n2, n3, np, r1min, rmap, static_cast<const cplx<float> *>(op), ldop, pl, nb);
     EPHIP_LAUNCHED();
     return EPHIP_OK;

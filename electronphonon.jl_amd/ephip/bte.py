@@ -551,7 +551,9 @@ def run_transport(model, kgrid, qgrid, window, params: ElectronTransportParams, 
     core.synchronize(backend)
     t["setup"] = time.perf_counter() - t0
     t0 = time.perf_counter()
-    loop = eph.OuterKLoop(st, nk_batch=nk_batch, precision=precision)
+    # without the general staged kernels: the FP64 rates and conductivities keep the digits that the FP32 elements
+    # of the direct kernels give (another order of the FP32 sums moves them by 3e-8)
+    loop = eph.OuterKLoop(st, nk_batch=nk_batch, precision=precision, staged=False)
     calc = BoltzmannCalculator(params, smearing=smearing, occupation_method=occupation_method)
     run_boltzmann(loop, calc)
     core.synchronize(backend)

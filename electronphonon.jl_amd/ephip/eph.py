@@ -476,7 +476,10 @@ class OuterKLoop:
 
     def __init__(self, st: OuterQSetup, nk_batch: int | None = 128, precision: int = L.PREC_FP32,
                  nk_batch_cap: int = 512, fuse_rotation: bool = True, fuse_projection: bool = True,
-                 gridopt: bool = True, gridopt_mfma: bool = True, with_ep: bool = False):
+                 gridopt: bool = True, gridopt_mfma: bool = True, with_ep: bool = False, staged: bool = True):
+        """``gridopt``: the staged transforms (GridOpt) of the shapes that csrc/gridopt.hip covers. ``staged``: with
+        it, those of every other shape (csrc/staged.hip). Both evaluate the same sums in FP32; they differ in the
+        order of the additions, about 3e-8 of a scattering rate."""
         torch = _torch()
         self.st = st
         if nk_batch is None:  # memory-adaptive width (plan_batch), the e-ph tensor already resident
@@ -504,40 +507,49 @@ class OuterKLoop:
             else None
         # kR->kq as the staged transform over the uniform q grid with the rotations and g2 fused (FP32)
         self.gridopt_q = _GridOptKQ.build(st) if (gridopt and nw == 16 and nm <= 16 and st.nbw <= 4) else None
+        # the same transforms for the shapes that the two do not cover (other nw, more modes, wider windows)
+        staged = bool(staged and gridopt)
+        self.staged_k = _GridOptKR.build(st, ks_host, self.nd_el, general=True) if (
+            staged and self.gridopt is None) else None
+        self.staged_q = _GridOptKQ.build(st, general=True) if (staged and self.gridopt_q is None) else None
+        if self.gridopt is not None and not self.gridopt.mfma and nw != 16 and staged and self.gridopt.box > 3:
+            self.gridopt.use_general()
+        self.rr = self.gridopt if self.gridopt is not None else self.staged_k
+        self.kq = self.gridopt_q if self.gridopt_q is not None else self.staged_q
         # split-BF16: the contractions that are not staged run on pre-packed operands. The "el" tensor is
         # split once (same bytes as complex64) and its complex64 copy released; the q-grid phase table is
         # built once; k phases and unit operands are packed per batch.
-        self.packed = precision == L.PREC_BF16X3 and (self.gridopt is None or self.gridopt_q is None)
+        self.packed = precision == L.PREC_BF16X3 and (self.rr is None or self.kq is None)
         # split-BF16 with nw = 16, nm = 12, nbw <= 4: kR->kq and the rotations run as one kernel that
         # writes g2 only (no g(k, q) staging buffer)
         self.fused = (bool(fuse_rotation) and self.packed and nw == 16 and nm == 12 and st.nbw <= 4
-                      and self.gridopt_q is None)
+                      and self.kq is None)
         # split-BF16 with nw = 16: RR->kR and the k-side window projection run as one kernel on the "el"
         # operand packed with j fastest; g(k, Rp) is never stored
         self.fused_proj = (bool(fuse_projection) and self.packed and nw == 16 and self.nd_el % 192 == 0
-                           and self.gridopt is None)
+                           and self.rr is None)
         # arithmetic each contraction runs in: the staged kernels are FP32 whatever ``precision`` asks for
         self.precision_requested = precision
         self.stage_precision = {
-            "RR->kR": L.PREC_FP32 if self.gridopt is not None else precision,
-            "kR->kq": L.PREC_FP32 if self.gridopt_q is not None else precision,
+            "RR->kR": L.PREC_FP32 if self.rr is not None else precision,
+            "kR->kq": L.PREC_FP32 if self.kq is not None else precision,
         }
         self.precision_overridden = any(p != precision for p in self.stage_precision.values())
         import ctypes
         self.qgrid_c = (ctypes.c_int32 * 3)(*map(int, st.qgrid))  # for the on-the-fly q phases
-        if self.gridopt is not None:
+        if self.rr is not None:
             self.el_obj = None   # the complex64 "el" tensor stays: stage 1 streams it
         elif self.fused_proj:
             self.apk_el = core.ft_pack_operand_swapped(self.epmat_el, self.nd_el, self.nre, nw, self.nd_el)
         elif self.packed:
             self.apk_el = core.ft_pack_operand(self.epmat_el, self.nd_el, self.nre, self.nd_el)
         if self.packed:
-            if self.gridopt is None:
+            if self.rr is None:
                 self.epmat_el = None
                 self.el_obj = None
                 self.bpk_k = torch.empty(core.ft_stages(self.nre) * self.nk_batch * 64, dtype=torch.bfloat16,
                                          device=dev)
-            if self.gridopt_q is None:
+            if self.kq is None:
                 self.bpk_q = core.ft_pack_phases(self.irvec_ep_dev, st.ph.xq)
         # units of every surviving k, in k order
         bmin = st.el.filt.band_min.cpu().numpy()
@@ -560,23 +572,23 @@ class OuterKLoop:
         max_units = int((self.k_unit_start[w:] - self.k_unit_start[:len(ks) + 1 - w]).max()) if len(ks) else 1
         self.max_units = max_units
         nd2 = nw * nm
-        self.G = None if (self.fused_proj or self.gridopt is not None) else torch.empty(
+        self.G = None if (self.fused_proj or self.rr is not None) else torch.empty(
             (self.nk_batch, self.nd_el), dtype=torch.complex64, device=dev)
         self.A = torch.empty((max_units, nd2 * self.nrp), dtype=torch.complex64, device=dev)
         self.col_index = torch.empty((max_units, self.cs), dtype=torch.int32, device=dev)
         self.ikq = torch.empty((max_units, self.cs), dtype=torch.int32, device=dev)
         self.count = torch.empty(max_units, dtype=torch.int32, device=dev)
-        self.Gq = None if (self.fused or self.gridopt_q is not None) else torch.empty(
+        self.Gq = None if (self.fused or self.kq is not None) else torch.empty(
             (max_units, self.cs, nd2), dtype=torch.complex64, device=dev)
-        if self.gridopt_q is not None:
-            self.line_off = torch.empty((max_units, self.gridopt_q.nlines + 1), dtype=torch.int32, device=dev)
+        if self.kq is not None:
+            self.line_off = torch.empty((max_units, self.kq.nlines + 1), dtype=torch.int32, device=dev)
         self.g2 = torch.empty((max_units, self.cs, st.nbw * nm), dtype=torch.float32, device=dev)
         # the complex elements behind g2 (the EPDataQBatched eps), from the staged or the unfused rotation kernels
         if with_ep and self.fused:
             raise ValueError("with_ep: the fused split-BF16 kR->kq kernel writes g2 only; use gridopt=True or "
                              "fuse_rotation=False")
         self.ep = torch.empty((max_units, self.cs, st.nbw * nm), dtype=torch.complex64, device=dev) if with_ep else None
-        if self.packed and self.gridopt_q is None:
+        if self.packed and self.kq is None:
             self.apk_units = torch.empty(max_units * core.ft_stages(self.nrp) * nd2 * 64, dtype=torch.bfloat16,
                                          device=dev)
         self.uph = st.ph.u.contiguous()
@@ -629,8 +641,8 @@ class OuterKLoop:
         starts = [int(i0) for i0 in starts]
         if warmup and starts:
             self.run_kbatch(starts[0], n)
-        if self.gridopt is not None:
-            self.gridopt.invalidate()
+        if self.rr is not None:
+            self.rr.invalidate()
         timer, self.ft_timer = self.ft_timer, None
         graph = torch.cuda.CUDAGraph()
         torch.cuda.synchronize()
@@ -639,8 +651,8 @@ class OuterKLoop:
                 payloads = [self.run_kbatch(i0, n, calculators) for i0 in starts]
         finally:
             self.ft_timer = timer
-            if self.gridopt is not None:
-                self.gridopt.invalidate()
+            if self.rr is not None:
+                self.rr.invalidate()
         return BatchGraph(graph, starts, n, payloads)
 
     def run_pipelined(self, starts, n: int, calculators=()):
@@ -684,9 +696,9 @@ class OuterKLoop:
         nu = u1 - u0
         # 1. RR->kR Fourier over Re for the batch
         xk_b = self.xk_surv[i0:i0 + n]
-        if self.gridopt is not None:  # staged RR->kR with the projection fused: writes the unit operators A
+        if self.rr is not None:  # staged RR->kR with the projection fused: writes the unit operators A
             self._timed("RR->kR", 8.0 * self.nd_el * self.nre * n,
-                        lambda: self.gridopt.run(self, i0, n, u0, u1, A, stream))
+                        lambda: self.rr.run(self, i0, n, u0, u1, A, stream))
         elif self.fused_proj:  # RR->kR with the projection in its epilogue: writes the unit operators A
             bpk = core.ft_pack_phases(st.irvec_el_dev, xk_b, out=self.bpk_k)
             self._timed("RR->kR", 8.0 * self.nd_el * self.nre * n, lambda: L.call(
@@ -700,7 +712,7 @@ class OuterKLoop:
         else:
             self._timed("RR->kR", 8.0 * self.nd_el * self.nre * n,
                         lambda: core.fourier_batched(self.el_obj, xk_b, out=self.G[:n], precision=self.precision))
-        if not self.fused_proj and self.gridopt is None:
+        if not self.fused_proj and self.rr is None:
             # projection; the unit's column in G is its k position minus i0 (base pointer shifted by -i0 columns)
             g_base = L.ptr(self.G) - i0 * self.G.stride(0) * 8
             L.call("ephip_eph_project_kR", nw, nm, self.nrp, nu, g_base, self.G.stride(0),
@@ -721,8 +733,8 @@ class OuterKLoop:
                L.ptr(self.count), stream)
         # 3. kR->kq batched Fourier over Rp at the kept q
         nd2 = nw * nm
-        if self.gridopt_q is not None:
-            self._timed("kR->kq", None, lambda: self.gridopt_q.run(self, nu, A, stream))
+        if self.kq is not None:
+            self._timed("kR->kq", None, lambda: self.kq.run(self, nu, A, stream))
         elif self.fused:
             core.ft_pack_operand(A, nd2, self.nrp, nd2, nu, nd2 * self.nrp, out=self.apk_units)
             self._timed("kR->kq", None, lambda: L.call(
@@ -743,7 +755,7 @@ class OuterKLoop:
                 L.ptr(self.irvec_ep_dev), L.ptr(st.ph.xq), nu, self.nq, L.ptr(self.count), L.ptr(self.col_index),
                 self.cs, L.ptr(self.Gq), nd2, self.cs * nd2, self.precision, stream))
         # 4. rotations + g2 (already done by the fused kernels)
-        if not self.fused and self.gridopt_q is None:
+        if not self.fused and self.kq is None:
             L.call("ephip_eph_rotate_kq_g2", nw, nm, st.nbw, nu, self.cs, L.ptr(self.count),
                    L.ptr(self.col_index), L.ptr(self.ikq), L.ptr(self.Gq), nd2, self.cs * nd2, L.ptr(st.el.U),
                    L.ptr(st.el.filt.band_min), L.ptr(st.el.filt.band_max), L.ptr(self.uph), L.ptr(self.omega),
@@ -768,8 +780,8 @@ class OuterKLoop:
         nd2 = nw * nm
         slots = st.nbw * kept if kept_slots is None else kept_slots
         rot = 8.0 * (nw * nm + nm * nm) * slots
-        if self.gridopt is not None:
-            go = self.gridopt
+        if self.rr is not None:
+            go = self.rr
             planes = go.line_plane[go.line_of_k[i0:i0 + n]]
             per_plane = np.bincount(go.line_plane[go.line_of_k], minlength=int(planes.max()) + 1)
             # stage 2 per line: n2 n3 complex multiply-adds, or in the folded form h pairs (one multiply-add's
@@ -780,11 +792,11 @@ class OuterKLoop:
                                        + go.n3 * n + nu)
         else:
             f_rr = 8.0 * self.nd_el * self.nre * n
-        if self.gridopt_q is not None:
-            gq = self.gridopt_q
+        if self.kq is not None:
+            gq = self.kq
             n2n3 = int((gq.rmap.view(gq.np, gq.n1, 8) >= 0).any(1).sum().item())  # (c, b) columns present
             from . import tune as T
-            mfma_kq = T.get_variant(T.KIND_GRIDOPT_KQ) == 1
+            mfma_kq = T.get_variant(T.KIND_GRIDOPT_KQ) == 1 and not gq.general
             # stage 1: nrp complex multiply-adds per (unit, q1) and row in the workgroup, or by the pre-pass
             # np^2 sums of np terms (h pairs when r1 spans -h .. h) per (unit, q1) and row
             s1 = self.nrp
@@ -845,7 +857,7 @@ class OuterKLoop:
             return res
         if self.packed:
             # the fused RR->kR + projection kernel has its own variants; tile shapes apply to the unfused one
-            if self.gridopt is not None:
+            if self.rr is not None:
                 res = {}
             elif self.fused_proj and len(T.PROJ_TUNE) == 1:
                 T.set_variant(T.KIND_FUSED_PROJ, T.PROJ_TUNE[0])
@@ -856,10 +868,12 @@ class OuterKLoop:
             else:
                 res = {"packed": T.tune_fourier(T.KIND_PACKED_BF16, lambda: self.run_kbatch(0, n), reps=reps,
                                                 variants=T.PACKED_VARIANTS)}
-            if self.fused and self.gridopt_q is None:
+            if self.fused and self.kq is None:
                 res["fused"] = T.tune_fourier(T.KIND_FUSED_ROT, lambda: self.run_kbatch(0, n), reps=reps,
                                               variants=T.FUSED_TUNE)
             return res
+        if self.rr is not None and self.kq is not None:
+            return {}   # both contractions staged, in forms without variants
         return T.tune_fourier(T.KIND_FP32_WIDE, lambda: self.run_kbatch(0, n), reps=reps)
 
     def run(self, k_start: int = 0, k_stop: int | None = None, calculators=()):
@@ -878,26 +892,34 @@ class _GridOptKR:
 
     N1_MAX, N23_MAX, KLINE_MAX, NBW_MAX = 32, 8, 64, 4
     PLANES = 8
+    LINE_UNITS = 128   # units of a line piece of the general form (ephip_staged_project)
+    # boxes of 27 R stay with the direct kernels: the staged ones are 1.0 to 5.5 times as fast there (7.1 -> 2.4 ms
+    # at 10 orbitals, 9 modes; 3.7 -> 3.6 at 16, 12), but their other order of the FP32 additions would move the FP64
+    # rates that consumers form from these payloads by 3e-8, where results are held to 1e-9
+    SMALL_BOX = 3
 
     @classmethod
-    def build(cls, st, ks, nd, mfma=True):
+    def build(cls, st, ks, nd, mfma=True, general=False):
         r = np.asarray(st.irvec_el_dev.cpu().numpy(), dtype=np.int64)
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         kg = np.asarray(st.kgrid, dtype=np.int64)
         if (len(ks) == 0 or n[0] > cls.N1_MAX or n[1] > cls.N23_MAX or n[2] > cls.N23_MAX
-                or st.nbw > cls.NBW_MAX):
+                or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and n.max() <= cls.SMALL_BOX)):
             return None
-        return cls(st, ks, nd, r, lo, n, kg, mfma)
+        return cls(st, ks, nd, r, lo, n, kg, mfma, general)
 
-    def __init__(self, st, ks, nd, r, lo, n, kg, mfma):
+    def __init__(self, st, ks, nd, r, lo, n, kg, mfma, general=False):
         torch = _torch()
         dev = st.el.xk.device
         self.nd = nd
         # stages 2/3 on the matrix cores for nw = 16 (op1 rows in natural order); otherwise the VALU form,
         # whose lane reduction wants op1 rows j-fastest
         self.mfma = bool(mfma) and st.nw == 16
-        self._nb = 1 if self.mfma else st.nw
+        # any other nw, and windows wider than NBW_MAX: MFMA stages 2/3 of every plane of a group in one launch
+        self.general = bool(general)
+        self._nb = 1 if (self.mfma or self.general) else st.nw
+        self.box = int(n.max())
         self.n1, self.n2, self.n3 = (int(x) for x in n)
         self.np = max(self.n2, self.n3, 3)
         self.rmin = [int(x) for x in lo]
@@ -909,8 +931,9 @@ class _GridOptKR:
         starts = np.concatenate([[0], change, [len(ks)]]).astype(np.int64)
         # a (k1, k2) line with more than KLINE_MAX surviving k (k3 grids above 64) is cut into pieces of at
         # most KLINE_MAX k; each piece forms its own stage-2 sums (the same k2 phases)
-        if np.diff(starts).max() > self.KLINE_MAX:
-            pieces = [np.arange(a, b, self.KLINE_MAX) for a, b in zip(starts[:-1], starts[1:])]
+        kline = max(1, min(self.KLINE_MAX, self.LINE_UNITS // st.nbw)) if self.general else self.KLINE_MAX
+        if np.diff(starts).max() > kline:
+            pieces = [np.arange(a, b, kline) for a, b in zip(starts[:-1], starts[1:])]
             starts = np.concatenate(pieces + [[len(ks)]]).astype(np.int64)
         self.line_start_host = starts
         self.line_start = torch.from_numpy(starts.astype(np.int32)).to(dev)
@@ -927,13 +950,18 @@ class _GridOptKR:
         self.plane_x1 = {p: float(x1[starts[l]]) for p, l in zip(self.planes, first_line)}
         self.plane_pos = {p: i for i, p in enumerate(self.planes)}
         self.cache = []  # [group, {plane: buffer}, buffers], most recent last, at most two
+        self.next_k = 0  # the general form: one past the last batch's k
+
+    def use_general(self):
+        """Take the general form (ephip_staged_project) in place of the VALU projection."""
+        self.general, self._nb = True, 1
 
     def folded(self) -> bool:
         """The MFMA projection kernel's folded stage-2 sums apply: the Re box spans -h .. h along axis 2
         (odd np) and tuner kind 8 is at its default."""
         from . import tune as T
-        return (self.mfma and self.np % 2 == 1 and self.np <= 7 and self.rmin[1] == -(self.np // 2)
-                and T.get_variant(T.KIND_KQ_FOLD) == 0)
+        return ((self.mfma or self.general) and self.np % 2 == 1 and self.np <= 7 and self.rmin[1] == -(self.np // 2)
+                and (self.general or T.get_variant(T.KIND_KQ_FOLD) == 0))
 
     def invalidate(self):
         """Forget which k1 planes the cached stage-1 buffers hold (the buffers are kept for reuse): the next
@@ -972,9 +1000,38 @@ class _GridOptKR:
             self.ph2 = torch.empty((loop.nk_batch, self.np), dtype=torch.complex64, device=dev)  # lines <= k
         return self.ucol, self.ph2, self.ph3
 
+    def _run_general(self, loop, i0, n, u0, u1, A, stream, l_first, l_last):
+        """Stage 1 and one projection launch per group of PLANES planes. Planes are kept between batches that
+        advance through the k list; a batch that starts before the last one's end recomputes what it needs."""
+        import ctypes as C
+        st = loop.st
+        if i0 < self.next_k:
+            self.invalidate()
+        self.next_k = i0 + n
+        ucol, ph2, ph3 = self._tables(loop, A.device)
+        L.call("ephip_gridopt_kR_tables", st.nw, self.np, self.rmin[1], self.rmin[2], L.ptr(loop.xk_surv), i0,
+               i0 + n, l_first, l_last, L.ptr(self.line_start), u1 - u0, L.ptr(loop.unit_state[u0:u1]),
+               L.ptr(loop.unit_band[u0:u1]), L.ptr(st.el.U), L.ptr(ucol), L.ptr(ph2), L.ptr(ph3), stream)
+        planes = self.line_plane[l_first:l_last]
+        cut = np.concatenate([[0], np.flatnonzero(np.diff(planes)) + 1, [len(planes)]])
+        lines = [(int(planes[a]), l_first + int(a), l_first + int(b)) for a, b in zip(cut[:-1], cut[1:])]
+        while lines:
+            g = self.plane_pos[lines[0][0]] // self.PLANES
+            part = [x for x in lines if self.plane_pos[x[0]] // self.PLANES == g]
+            lines = lines[len(part):]
+            m = len(part)
+            op1 = (C.c_void_p * m)(*[L.ptr(self._plane_buffer(p, loop.epmat_el, stream)) for p, _, _ in part])
+            la, lz = (C.c_int32 * m)(*[x[1] for x in part]), (C.c_int32 * m)(*[x[2] for x in part])
+            L.call("ephip_staged_project", st.nw, self.nd // st.nw, self.np, self.rmin[1], m, C.addressof(op1),
+                   C.addressof(la), C.addressof(lz), i0, i0 + n, l_first, L.ptr(self.line_start),
+                   self.max_line_units, L.ptr(loop.k_unit_start_dev), L.ptr(loop.unit_kpos), L.ptr(ucol), L.ptr(ph2),
+                   L.ptr(ph3), L.ptr(A), A.stride(0), stream)
+
     def run(self, loop, i0, n, u0, u1, A, stream):
         st = loop.st
         l_first, l_last = int(self.line_of_k[i0]), int(self.line_of_k[i0 + n - 1]) + 1
+        if self.general:
+            return self._run_general(loop, i0, n, u0, u1, A, stream, l_first, l_last)
         if self.mfma:
             ucol, ph2, ph3 = self._tables(loop, A.device)
             L.call("ephip_gridopt_kR_tables", st.nw, self.np, self.rmin[1], self.rmin[2], L.ptr(loop.xk_surv), i0,
@@ -1010,18 +1067,25 @@ class _GridOptKQ:
     prepass_default = False  # where stage 1 runs in new instances (in each workgroup, or by the pre-pass)
 
     @classmethod
-    def build(cls, st):
+    def build(cls, st, general=False):
         r = np.asarray(st.epmat.irvec_dev().cpu().numpy(), dtype=np.int64)
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         m = np.asarray(st.qgrid, dtype=np.int64)
         if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535:
             return None
-        return cls(st, r, lo, n, m)
+        if general and (st.nw > 32 or st.nm > 48 or n.max() <= _GridOptKR.SMALL_BOX):
+            return None
+        return cls(st, r, lo, n, m, general)
 
-    def __init__(self, st, r, lo, n, m):
+    def __init__(self, st, r, lo, n, m, general=False):
         torch = _torch()
         dev = st.el.xk.device
+        self.general = general   # ephip_staged_kq: any nw, nm and window width
+        # expected kept q of one (unit, q1) slab and window bands per kept q
+        widths = (st.el.filt.band_max - st.el.filt.band_min + 1)[st.el.filt.band_min > 0]
+        self.cols = widths.shape[0] / max(1, st.el.xk.shape[0]) * int(m[1]) * int(m[2])
+        self.width = float(widths.double().mean()) if widths.shape[0] else 1.0
         self.n1 = int(n[0])
         self.np = max(int(n[1]), int(n[2]), 3)
         self.pmin = [int(x) for x in lo]
@@ -1039,6 +1103,13 @@ class _GridOptKQ:
                 self.dense = (ctypes.c_int32 * 3)(s1, s2, s3)
         self.m = [int(x) for x in m]
         self.nlines = self.m[0] * self.m[1]
+        if general:   # phases of the q grid along each axis
+            ne = (self.np + 1) & ~1
+            self.phases = []
+            for mi, ni, nei, pi in zip(self.m, (self.n1, self.np, self.np), (self.n1, ne, ne), self.pmin):
+                e = torch.empty((mi, nei), dtype=torch.complex64, device=dev)
+                L.call("ephip_staged_phases", mi, ni, nei, pi, L.ptr(e), L.stream_handle())
+                self.phases.append(e)
         self.prepass = _GridOptKQ.prepass_default  # stage 1 by the pre-pass (OuterKLoop.tune picks per workload)
         import ctypes
         self.qgrid_c = (ctypes.c_int32 * 3)(*self.m)
@@ -1048,12 +1119,14 @@ class _GridOptKQ:
         and tuner kind 8 is at its default."""
         from . import tune as T
         h = self.np // 2
+        if self.general:
+            return self.np % 2 == 1 and self.n1 == self.np and all(p == -h for p in self.pmin)
         return (self.np % 2 == 1 and self.pmin[1] == -h and self.pmin[2] == -h
                 and T.get_variant(T.KIND_KQ_FOLD) == 0)
 
     def can_prepass(self) -> bool:
         """The stage-1 pre-pass applies: a cube box with odd np <= 7 (n1 = np) and m1 <= 64."""
-        return self.n1 == self.np and self.np % 2 == 1 and self.np <= 7 and self.m[0] <= 64
+        return not self.general and self.n1 == self.np and self.np % 2 == 1 and self.np <= 7 and self.m[0] <= 64
 
     def prepass_folded(self) -> bool:
         return self.pmin[0] == -(self.np // 2)
@@ -1070,6 +1143,14 @@ class _GridOptKQ:
             b1 = self.b1
         L.call("ephip_kq_line_offsets", nu, L.ptr(loop.count), L.ptr(loop.col_index), loop.cs, self.m[2],
                self.nlines, L.ptr(loop.line_off), stream)
+        if self.general:
+            L.call("ephip_staged_kq", st.nw, st.nm, st.nbw, nu, self.n1, self.np, *self.pmin, L.ptr(self.rmap),
+                   C.addressof(self.qgrid_c), *map(L.ptr, self.phases), L.ptr(A), A.stride(0), st.nw * st.nm,
+                   L.ptr(loop.line_off), L.ptr(loop.col_index), L.ptr(loop.ikq), loop.cs, L.ptr(st.el.U),
+                   L.ptr(st.el.filt.band_min), L.ptr(st.el.filt.band_max), L.ptr(loop.uph), L.ptr(loop.omega),
+                   C.addressof(self.dense) if self.dense is not None else None, self.cols, self.width, L.ptr(loop.g2),
+                   L.ptr(loop.ep) if loop.ep is not None else None, stream)
+            return
         L.call("ephip_gridopt_kq_rotate", st.nw, st.nm, st.nbw, nu, self.n1, self.np, self.pmin[0], self.pmin[1],
                self.pmin[2], L.ptr(self.rmap), C.addressof(self.qgrid_c), L.ptr(A), A.stride(0),
                st.nw * st.nm, L.ptr(loop.line_off), L.ptr(loop.col_index), L.ptr(loop.ikq), loop.cs,

@@ -329,6 +329,33 @@ int ephip_gridopt_kq_rotate(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits,
                             const int64_t *bmin, const int64_t *bmax, const void *uph, const double *omega,
                             const int32_t *dense_strides, float *g2, void *ep, void *b1, void *stream);
 
+/* The staged (GridOpt) outer-k transforms for any model shape (nw <= 32, nm <= 48, any window width), FP32:
+ *  - ephip_staged_project: stages 2/3 of RR->kR with the k-side projection, as ephip_gridopt_kR_project_mfma, for
+ *    nplanes <= 8 k1 planes in one launch. op1 (host array of nplanes device pointers) holds the planes' stage-1
+ *    sums (ephip_gridopt_stage1_planes with nb = 1, faces np x np, 3 <= np <= 8) and l0 / l1 (host arrays) their
+ *    lines (or line pieces; at most 64 k and max_line_units <= 128 units each), all with lb0 <= l. ngcol = the
+ *    operator's columns g = i + nw rest, a multiple of nw (nw nm nrp for the e-ph tensor); op1 rows are
+ *    d = i + nw (j + nw rest). kus, line_start, ucol, ph2, ph3: as for ephip_gridopt_kR_project_mfma
+ *    (ephip_gridopt_kR_tables, any nw). ukpos (int32 per unit): the unit's position in the surviving k. Writes
+ *    A[u lda + g] = sum_j g(k_u)[j, g] U_u[j], u counted from kus[k0]; units of k0 <= k < k1.
+ *  - ephip_staged_kq: ephip_gridopt_kq_rotate for those shapes (arguments and output as there, no pre-pass).
+ *    cols_hint, width_hint: expected kept q of one (unit, q1) slab and window bands per kept q; they size the
+ *    workgroups only. e1 (m1 rows of n1), e2 (m2 rows) and e3 (m3 rows of np rounded up to even): the q grid's
+ *    phases along each axis, complex64, from ephip_staged_phases.
+ *  - ephip_staged_phases: out[x ne + b] = e^{2 pi i (x / m) (pmin + b)} for x < m, b < n; zero for n <= b < ne. */
+int ephip_staged_phases(int32_t m, int32_t n, int32_t ne, int32_t pmin, void *out, void *stream);
+int ephip_staged_project(int32_t nw, int64_t ngcol, int32_t np, int32_t r2min, int32_t nplanes,
+                         const void *const *op1, const int32_t *l0, const int32_t *l1, int64_t k0, int64_t k1,
+                         int32_t lb0, const int32_t *line_start, int32_t max_line_units, const int32_t *kus,
+                         const int32_t *ukpos, const void *ucol, const void *ph2, const void *ph3, void *A,
+                         int64_t lda, void *stream);
+int ephip_staged_kq(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits, int32_t n1, int32_t np, int32_t p1min,
+                    int32_t p2min, int32_t p3min, const int32_t *rmap, const int32_t *qgrid, const void *e1,
+                    const void *e2, const void *e3, const void *A, int64_t lda, int64_t ldr, const int32_t *line_off, const int32_t *col_index, const int32_t *ikq,
+                    int64_t cs, const void *U, const int64_t *bmin, const int64_t *bmax, const void *uph,
+                    const double *omega, const int32_t *dense_strides, double cols_hint, double width_hint,
+                    float *g2, void *ep, void *stream);
+
 /* kR->kq Fourier over Rp fused with the k+q-window and phonon rotations and g2 (the
  * get_eph_kR_to_kq_batched! + eph_apply_rotations! + g2 sequence of src/wannier_to_bloch_batched.jl:
  * 245-273 and :442-455 in one kernel) for nw = 16, nm = 12, nbw <= 4, split-BF16: apk holds the
