@@ -125,6 +125,208 @@ __global__ void bte_accumulate_kernel(int nunits, int64_t cs, int nbw, int nm, c
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same sums with everything that does not depend on the (state, mode) pair taken out of the inner loop:
+//   tab_q: phonon frequency and, per temperature, occupation of every (mode, q), q fastest (lanes hold
+//          neighbouring q): omega[nu][q], then n (method 5: sqrt(n (n + 1))) [t][nu][q];
+//   tab_s: per temperature and state, the Fermi function (method 5: its energy derivative) [t][state].
+// What is left per (state pair, mode) is the two smeared deltas, shared by temperatures of one width, and a few
+// multiplications: 2 FP64 exponentials where the per-term form takes 10 per temperature. S_out is summed over the
+// wave before its atomic (where every (kept q, band) of a unit added to the same address).
+// ---------------------------------------------------------------------------------------------
+__global__ void bte_tables_kernel(int nq, int nm, const double *__restrict__ omega, int64_t nstates,
+                                  const double *__restrict__ e_state, int nT, const double *__restrict__ mus,
+                                  const double *__restrict__ Ts, int method, double *__restrict__ tab_q,
+                                  double *__restrict__ tab_s) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, nmq = (int64_t)nm * nq;
+    if (e < nmq) {
+        const int64_t nu = e / nq, q = e % nq;
+        const double w = omega[nm * q + nu];
+        tab_q[e] = w;
+        for (int t = 0; t < nT; t++) {
+            const double n = occ_boson(w, Ts[t]);
+            tab_q[(1 + t) * nmq + e] = method == 5 ? sqrt(n * (n + 1)) : n;
+        }
+    } else if (e < nmq + nT * nstates) {
+        const int64_t f = e - nmq, t = f / nstates, i = f % nstates;
+        const double x = e_state[i] - mus[t];
+        tab_s[f] = method == 5 ? occ_fd_deriv(x, Ts[t]) : occ_fd(x, Ts[t]);
+    }
+}
+
+// Factors of the increments that the modes of one (initial, final) state pair share, at one temperature.
+template <int METHOD>
+struct BtePair {
+    double a, b, c, d;
+    __device__ void set(double si, double sf, double ek, double ekq, double T) {
+        if constexpr (METHOD == 1) {
+            a = si;
+            b = sf;
+        } else if constexpr (METHOD == 2) {
+            const double gi = si * (1 - si), gf = sf * (1 - sf);
+            a = si;
+            b = sf;
+            c = gf / gi;
+            d = gi / gf;
+        } else if constexpr (METHOD == 3) {
+            c = (1 - sf) / (1 - si);
+            d = (1 - si) / (1 - sf);
+        } else if constexpr (METHOD == 4) {
+            c = sf / si;
+            d = si / sf;
+        } else if constexpr (METHOD == 5) {
+            c = sqrt(sf / si);
+            d = sqrt(si / sf);
+        } else {
+            c = occ_boson(ekq - ek, T) + sf;
+            d = occ_boson(ek - ekq, T) + si;
+        }
+    }
+    // n: the mode's occupation factor; so = d1 f1o + d2 f2o, si = d2 f1i + d1 f2i (vanishing deltas left out)
+    __device__ void add(double n, double d1, double d2, double pref, double &so, double &si) const {
+        double f1o, f2o, f1i, f2i;
+        if constexpr (METHOD == 1) {
+            f1o = n + b, f2o = n + 1 - b, f1i = n + a, f2i = n + 1 - a;
+        } else if constexpr (METHOD == 2) {
+            f1o = c * (n + 1 - a), f2o = c * (n + a), f1i = d * (n + 1 - b), f2i = d * (n + b);
+        } else if constexpr (METHOD == 3) {
+            f1o = c * n, f2o = c * (n + 1), f1i = d * n, f2i = d * (n + 1);
+        } else if constexpr (METHOD == 4) {
+            f1o = c * (n + 1), f2o = c * n, f1i = d * (n + 1), f2i = d * n;
+        } else if constexpr (METHOD == 5) {
+            f1o = f2o = n * c, f1i = f2i = n * d;
+        } else {
+            f1o = c, f2o = -c, f1i = d, f2i = -d;
+        }
+        so += ((d1 == 0.0 ? 0.0 : d1 * f1o) + (d2 == 0.0 ? 0.0 : d2 * f2o)) * pref;
+        si += ((d2 == 0.0 ? 0.0 : d2 * f1i) + (d1 == 0.0 ? 0.0 : d1 * f2i)) * pref;
+    }
+};
+
+// The kept (q, window band) pairs of 256 columns are listed in LDS, so that lanes hold pairs: taken column by column
+// the few second bands cost every wave that has one a whole pass (measured 1.33 against 0.80 ms, 3.07M rows of 12
+// modes at 3 temperatures; the per-term form took 7.65 ms). Bound by the FP64 exponentials.
+template <int METHOD, int NT>  // NT temperatures per pass
+__global__ __launch_bounds__(256) void bte_accumulate_tab_kernel(
+    int64_t cs, int nbw, int nm, int nq, const int *__restrict__ count, const int *__restrict__ col_index,
+    const int *__restrict__ ikq, const float *__restrict__ g2, const int64_t *__restrict__ unit_state_index,
+    const int64_t *__restrict__ state_offset, const int64_t *__restrict__ bmin, const int64_t *__restrict__ bmax,
+    const double *__restrict__ e_state, const double *__restrict__ tab_q, const double *__restrict__ tab_s, double wtq,
+    int nT, const double *__restrict__ Ts, const double *__restrict__ etas, int smearing, double w_cut,
+    int64_t nstates, const int64_t *__restrict__ rowptr, double *__restrict__ S_out, double *__restrict__ S_in,
+    uint32_t *__restrict__ row_code, int quad) {
+    __shared__ int ciq[256], cf0[256], wsum[4];
+    extern __shared__ uint16_t list[];  // [256 nbw] column | band << 8
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t c0 = (int64_t)blockIdx.x * 256;
+    const int u = blockIdx.y, cnt = count[u];
+    if (c0 >= cnt) return;  // uniform
+    const int64_t i = unit_state_index[u], row0 = (int64_t)u * cs + c0, orow0 = rowptr[u] + c0;
+    int nb = 0;
+    if (c0 + t < cnt) {
+        const int64_t kq = ikq[row0 + t];
+        nb = bmin[kq] > 0 ? min((int)(bmax[kq] - bmin[kq] + 1), nbw) : 0;
+        ciq[t] = col_index[row0 + t];
+        cf0[t] = (int)state_offset[kq];
+        row_code[orow0 + t] = (uint32_t)cf0[t] | ((uint32_t)nb << 27);
+        for (int m = nb; m < nbw; m++)
+            for (int x = 0; x < nT; x++) S_in[((orow0 + t) * nbw + m) * nT + x] = 0.0;
+    }
+    int pre = nb;  // inclusive prefix
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(pre, off, 64);
+        if (lane >= off) pre += o;
+    }
+    if (lane == 63) wsum[wave] = pre;
+    __syncthreads();
+    int npair = 0;
+    for (int w = 0; w < 4; w++) {
+        if (w == wave) pre += npair;
+        npair += wsum[w];
+    }
+    for (int m = 0; m < nb; m++) list[pre - nb + m] = (uint16_t)(t | (m << 8));
+    __syncthreads();
+    const double ek = e_state[i], pre2 = 2.0 * M_PI * wtq;
+    const int64_t nmq = (int64_t)nm * nq;
+    for (int t0 = 0; t0 < nT; t0 += NT) {
+        double tot[NT];
+        double eta[NT], ie[NT], nrm[NT];  // width, its inverse, prefactor of the delta
+#pragma unroll
+        for (int x = 0; x < NT; x++) {
+            tot[x] = 0.0;
+            eta[x] = etas[min(t0 + x, nT - 1)];
+            ie[x] = 1.0 / eta[x];
+            nrm[x] = smearing == 1 ? (1.0 / sqrt(M_PI)) / eta[x] : eta[x] / M_PI;
+        }
+        for (int e = t; e < npair; e += 256) {
+            const int col = list[e] & 255, m = list[e] >> 8, iq = ciq[col];
+            const int64_t f = cf0[col] + m;
+            const double ekq = e_state[f], x0 = ek - ekq;
+            double so[NT], si[NT];
+            BtePair<METHOD> pr[NT];
+#pragma unroll
+            for (int x = 0; x < NT; x++) {
+                const int tt = min(t0 + x, nT - 1);
+                so[x] = si[x] = 0.0;
+                pr[x].set(tab_s[tt * nstates + i], tab_s[tt * nstates + f], ek, ekq, Ts[tt]);
+            }
+            const float *gr = g2 + ((row0 + col) * nbw + m) * nm;
+            for (int nu0 = 0; nu0 < nm; nu0 += 4) {  // four modes' loads in flight together
+                double w[4], n[4][NT];
+                float g[4];
+                if (quad) {  // nm a multiple of 4 and g2 16-byte aligned
+                    const float4 v = *reinterpret_cast<const float4 *>(gr + nu0);
+                    g[0] = v.x, g[1] = v.y, g[2] = v.z, g[3] = v.w;
+                } else {
+#pragma unroll
+                    for (int y = 0; y < 4; y++) g[y] = gr[min(nu0 + y, nm - 1)];
+                }
+#pragma unroll
+                for (int y = 0; y < 4; y++) {
+                    const int64_t at = (int64_t)min(nu0 + y, nm - 1) * nq + iq;
+                    w[y] = tab_q[at];
+#pragma unroll
+                    for (int x = 0; x < NT; x++) n[y][x] = tab_q[(1 + min(t0 + x, nT - 1)) * nmq + at];
+                }
+#pragma unroll
+                for (int y = 0; y < 4; y++) {
+                    const bool in = nu0 + y < nm && !(w[y] < w_cut);  // else both deltas zero: nothing added
+                    const double pref = in ? pre2 * (double)g[y] : 0.0;
+                    double d1 = 0.0, d2 = 0.0;
+#pragma unroll
+                    for (int x = 0; x < NT; x++) {
+                        if (x == 0 || eta[x] != eta[x - 1]) {  // uniform: one width for all temperatures as a rule
+                            const double a = x0 + w[y], b = x0 - w[y];
+                            if (smearing == 1) {
+                                d1 = nrm[x] * exp(-(a * ie[x]) * (a * ie[x]));
+                                d2 = nrm[x] * exp(-(b * ie[x]) * (b * ie[x]));
+                            } else {
+                                d1 = nrm[x] / (a * a + eta[x] * eta[x]);
+                                d2 = nrm[x] / (b * b + eta[x] * eta[x]);
+                            }
+                            if (!in) d1 = d2 = 0.0;
+                        }
+                        pr[x].add(n[y][x], d1, d2, pref, so[x], si[x]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < NT; x++)
+                if (t0 + x < nT) {
+                    S_in[((orow0 + col) * nbw + m) * nT + t0 + x] = si[x];
+                    tot[x] += so[x];
+                }
+        }
+#pragma unroll
+        for (int x = 0; x < NT; x++)
+            if (t0 + x < nT) {
+                const double v = wave_sum(tot[x]);
+                if (lane == 0) atomicAdd(&S_out[i + nstates * (t0 + x)], v);
+            }
+    }
+}
+
 // bte_window_accumulate! with the reference's arguments (ext/ElectronPhononCUDAExt.jl:323-372, generic
 // src/boltzmann/boltzmann_calculator.jl:336-372): one thread per (m, n, j) of a q batch. i = imap_i[n]
 // (outer state, 1-based, 0 = outside the window), f = imap_f[m + ld_f (ikqs[j] - 1)] (inner state); per
@@ -335,6 +537,53 @@ extern "C" int ephip_bte_accumulate_units(int32_t nunits, int64_t cs, int32_t nb
                                                             unit_state_index, state_offset, bmin, bmax, e_state, omega,
                                                             wtq, nT, mus, Ts, etas, method, smearing, w_cut, nstates,
                                                             rowptr, S_out, S_in, row_code);
+    EPHIP_LAUNCHED();
+    return EPHIP_OK;
+}
+
+extern "C" int ephip_bte_tables(int32_t nq, int32_t nm, const double *omega, int64_t nstates, const double *e_state,
+                                int32_t nT, const double *mus, const double *Ts, int32_t method, double *tab_q,
+                                double *tab_s, void *stream) {
+    EPHIP_REQUIRE(nq >= 0 && nm >= 1 && nstates >= 0 && nT >= 1, "bte_tables: bad sizes");
+    EPHIP_REQUIRE(method >= 1 && method <= 6, "bte_tables: method %d outside 1..6", method);
+    const int64_t n = (int64_t)nm * nq + nT * nstates;
+    if (n == 0) return EPHIP_OK;
+    EPHIP_REQUIRE(n <= 0x7fffffffLL * 256, "bte_tables: too many entries");
+    EPHIP_REQUIRE(omega && e_state && mus && Ts && tab_q && tab_s, "bte_tables: null device pointer");
+    bte_tables_kernel<<<nbk(n), 256, 0, as_stream(stream)>>>(nq, nm, omega, nstates, e_state, nT, mus, Ts, method, tab_q,
+                                                            tab_s);
+    EPHIP_LAUNCHED();
+    return EPHIP_OK;
+}
+
+extern "C" int ephip_bte_accumulate_tables(int32_t nunits, int64_t cs, int32_t nbw, int32_t nm, int32_t nq,
+                                           const int32_t *count, const int32_t *col_index, const int32_t *ikq,
+                                           const float *g2, const int64_t *unit_state_index,
+                                           const int64_t *state_offset, const int64_t *bmin, const int64_t *bmax,
+                                           const double *e_state, const double *tab_q, const double *tab_s,
+                                           double wtq, int32_t nT, const double *Ts, const double *etas,
+                                           int32_t method, int32_t smearing, double w_cut, int64_t nstates,
+                                           const int64_t *rowptr, double *S_out, double *S_in, uint32_t *row_code,
+                                           void *stream) {
+    EPHIP_REQUIRE(nunits >= 0 && nunits <= 65535 && cs >= 0 && nbw >= 1 && nbw <= 31 && nm >= 1 && nT >= 1 && nq >= 0,
+                  "bte_accumulate_tables: bad sizes");
+    EPHIP_REQUIRE(nstates < (1LL << 27), "bte_accumulate_tables: %lld states exceed the row code range",
+                  (long long)nstates);
+    EPHIP_REQUIRE(method >= 1 && method <= 6 && (smearing == 1 || smearing == 2),
+                  "bte_accumulate_tables: bad method/smearing");
+    if (nunits == 0 || cs == 0) return EPHIP_OK;
+    EPHIP_REQUIRE(count && col_index && ikq && g2 && unit_state_index && state_offset && bmin && bmax && e_state &&
+                      tab_q && tab_s && Ts && etas && rowptr && S_out && S_in && row_code,
+                  "bte_accumulate_tables: null device pointer");
+    using K = decltype(&bte_accumulate_tab_kernel<1, 1>);
+#define BTE_ROW(m) {bte_accumulate_tab_kernel<m, 1>, bte_accumulate_tab_kernel<m, 2>, bte_accumulate_tab_kernel<m, 3>}
+    static const K kern[6][3] = {BTE_ROW(1), BTE_ROW(2), BTE_ROW(3), BTE_ROW(4), BTE_ROW(5), BTE_ROW(6)};
+#undef BTE_ROW
+    kern[method - 1][nT == 1 ? 0 : nT == 2 ? 1 : 2]<<<dim3(nbk(cs), (unsigned)nunits), 256,
+                                                      (size_t)256 * nbw * sizeof(uint16_t), as_stream(stream)>>>(
+        cs, nbw, nm, nq, count, col_index, ikq, g2, unit_state_index, state_offset, bmin, bmax, e_state, tab_q, tab_s,
+        wtq, nT, Ts, etas, smearing, w_cut, nstates, rowptr, S_out, S_in, row_code,
+        (nm & 3) == 0 && (reinterpret_cast<uintptr_t>(g2) & 15) == 0);
     EPHIP_LAUNCHED();
     return EPHIP_OK;
 }

@@ -54,6 +54,9 @@ SIGNATURES = {
     "ephip_bte_increments": [_i64, _i32, _i32, _vp, _vp, _vp],
     "ephip_bte_accumulate_units": [_i32, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _d,
                                    _i32, _vp, _vp, _vp, _i32, _i32, _d, _i64, _vp, _vp, _vp, _vp, _vp],
+    "ephip_bte_tables": [_i32, _i32, _vp, _i64, _vp, _i32, _vp, _vp, _i32, _vp, _vp, _vp],
+    "ephip_bte_accumulate_tables": [_i32, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                    _d, _i32, _vp, _vp, _i32, _i32, _d, _i64, _vp, _vp, _vp, _vp, _vp],
     "ephip_band_velocity": [_i32, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp],
     "ephip_el_velocity_direct_batched": [_i32, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp],
     "ephip_batched_gemm": [_i32, _i32, _i32, _i32, _i32, _i32, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp,

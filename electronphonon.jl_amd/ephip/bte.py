@@ -281,7 +281,13 @@ class BoltzmannCalculator:
         self.mus = torch.as_tensor(self.params.mulist, device=dev)
         self.Ts = torch.as_tensor(self.params.Tlist, device=dev)
         self.etas_d = torch.as_tensor(self.etas, device=dev)
-        self.wtq = 1.0 / st.ph.xq.shape[0]
+        self.nq = st.ph.xq.shape[0]
+        self.wtq = 1.0 / self.nq
+        # occupations of every phonon mode and state at every temperature (ephip_bte_tables)
+        self.tab_q = torch.empty((1 + nT) * st.nm * self.nq, dtype=torch.float64, device=dev)
+        self.tab_s = torch.empty(nT * self.bs.n, dtype=torch.float64, device=dev)
+        L.call("ephip_bte_tables", self.nq, st.nm, L.ptr(loop.omega), self.bs.n, L.ptr(self.bs.es), nT,
+               L.ptr(self.mus), L.ptr(self.Ts), self.method, L.ptr(self.tab_q), L.ptr(self.tab_s), L.stream_handle())
         return self
 
     def run(self, p):
@@ -299,11 +305,10 @@ class BoltzmannCalculator:
         S_in = torch.empty((max(nrows, 1), p.nbw, self.nT), dtype=torch.float64, device=usi.device)
         row_code = torch.empty(max(nrows, 1), dtype=torch.int32, device=usi.device)
         cs = p.col_index.stride(0)
-        L.call("ephip_bte_accumulate_units", nu, cs, p.nbw, st.nm, L.ptr(p.count), L.ptr(p.col_index),
+        L.call("ephip_bte_accumulate_tables", nu, cs, p.nbw, st.nm, self.nq, L.ptr(p.count), L.ptr(p.col_index),
                L.ptr(p.ikq), L.ptr(p.g2), L.ptr(usi), L.ptr(bs.state_offset), L.ptr(f.band_min),
-               L.ptr(f.band_max), L.ptr(bs.es), L.ptr(self.loop.omega), self.wtq, self.nT, L.ptr(self.mus),
-               L.ptr(self.Ts), L.ptr(self.etas_d), self.method, self.kind, self.omega_cutoff, bs.n,
-               L.ptr(rowptr), L.ptr(self.S_out), L.ptr(S_in), L.ptr(row_code), L.stream_handle())
+               L.ptr(f.band_max), L.ptr(bs.es), L.ptr(self.tab_q), L.ptr(self.tab_s), self.wtq, self.nT,
+               L.ptr(self.Ts), L.ptr(self.etas_d), self.method, self.kind, self.omega_cutoff, bs.n, L.ptr(rowptr), L.ptr(self.S_out), L.ptr(S_in), L.ptr(row_code), L.stream_handle())
         self.blocks.append(SinBlock(usi, rowptr, row_code, S_in[:nrows], nrows))
 
     def postprocess(self):

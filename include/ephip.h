@@ -472,6 +472,21 @@ int ephip_bte_accumulate_units(int32_t nunits, int64_t cs, int32_t nbw, int32_t 
                                int32_t smearing, double w_cut, int64_t nstates, const int64_t *rowptr, double *S_out,
                                double *S_in, uint32_t *row_code, void *stream);
 
+/* ephip_bte_accumulate_units with the occupations tabulated ahead (same outputs and arguments):
+ *  - ephip_bte_tables: tab_q, double (1 + nT) x nm x nq, q fastest: omega, then per temperature the phonon
+ *    occupation n (method 5: sqrt(n (n + 1))); tab_s, double nT x nstates: the Fermi function of e_state - mu
+ *    (method 5: its energy derivative). omega (nm x nq) as elsewhere, mode fastest.
+ *  - ephip_bte_accumulate_tables: the accumulation of one outer-k batch with those tables. */
+int ephip_bte_tables(int32_t nq, int32_t nm, const double *omega, int64_t nstates, const double *e_state, int32_t nT,
+                     const double *mus, const double *Ts, int32_t method, double *tab_q, double *tab_s, void *stream);
+int ephip_bte_accumulate_tables(int32_t nunits, int64_t cs, int32_t nbw, int32_t nm, int32_t nq, const int32_t *count,
+                                const int32_t *col_index, const int32_t *ikq, const float *g2,
+                                const int64_t *unit_state_index, const int64_t *state_offset, const int64_t *bmin,
+                                const int64_t *bmax, const double *e_state, const double *tab_q, const double *tab_s,
+                                double wtq, int32_t nT, const double *Ts, const double *etas, int32_t method,
+                                int32_t smearing, double w_cut, int64_t nstates, const int64_t *rowptr, double *S_out,
+                                double *S_in, uint32_t *row_code, void *stream);
+
 /* Band-diagonal velocities v[3*s + a] = Re(u^H dH_a u) of nstates states (k block state_k[s], band
  * state_band[s] of the nw x nw complex64 eigenvector blocks U); dH: complex128 operator columns of
  * ld_dh >= 3 nw^2 entries (direction slowest), column state_col[s]. Replaces the per-k
