@@ -49,6 +49,7 @@ SIGNATURES = {
     "ephip_silu_bwd": [_i64, _vp, _vp, _vp, _vp],
     "ephip_mse_grad": [_i64, _vp, _vp, C.c_float, _vp, _vp, _vp],
     "ephip_colsum": [_i32, _i32, _vp, _i64, _vp, _vp],
+    "ephip_mlp_train_step": [_i64, _vp, _i32, _vp, _i32, _i32] + 12 * [_vp] + [_i32, _vp, _vp, _vp],
     "ephip_adam_step": [_i64, _vp, _vp, _vp, _vp, C.c_float, C.c_float, C.c_float, C.c_float, _i32, _vp],
     "ephip_f32_to_bf16": [_i64, _vp, _vp, _vp],
     "ephip_bte_increments": [_i64, _i32, _i32, _vp, _vp, _vp],

@@ -130,6 +130,8 @@ class BandSurrogate:
         """Mean squared error over points and outputs; fills self.g. Returns (loss tensor (device), acts)."""
         torch = _torch()
         n = xk.shape[0]
+        if self._fused():
+            return self._loss_and_grad_fused(xk, target, acts, grads)
         a = self.forward(xk, acts)
         st = L.stream_handle()
         O, H = self.nout, self.hidden
@@ -158,6 +160,29 @@ class BandSurrogate:
         # layer 1
         self._wgrad(gw["gz"], a["f"], "W1", gw["part"])
         self._bgrad(gw["gz"], "b1", gw["part"], gw["ones"])
+        return gw["partial"], a, gw
+
+    def _fused(self) -> bool:
+        """Sizes of ephip_mlp_train_step: features and hidden multiples of 16 up to 128, outputs up to 64."""
+        return self.nf % 16 == 0 and self.nf <= 128 and self.hidden % 16 == 0 and self.hidden <= 128 and self.nout <= 64
+
+    def _loss_and_grad_fused(self, xk, target, acts, grads):
+        """loss_and_grad in three launches; ga and gz of the returned buffers hold dL/dz of the two hidden layers."""
+        torch = _torch()
+        n, O, H = xk.shape[0], self.nout, self.hidden
+        a = acts if acts is not None else self._alloc_acts(n)
+        nparts = max(1, min(256, (n + 31) // 32))   # workgroups of the weight gradients, at least 32 points each
+        gw = grads if grads is not None else dict(gy=torch.empty((n, O), dtype=torch.float32, device=self.dev),
+                                                  ga=torch.empty((n, H), dtype=torch.float32, device=self.dev),
+                                                  gz=torch.empty((n, H), dtype=torch.float32, device=self.dev),
+                                                  part=torch.empty(nparts * self.nparam, dtype=torch.float32,
+                                                                   device=self.dev),
+                                                  partial=torch.empty((n * O + 255) // 256, dtype=torch.float64,
+                                                                      device=self.dev))
+        L.call("ephip_mlp_train_step", n, L.ptr(xk), self.nf2, L.ptr(self.mvec), H, O, L.ptr(self.p), L.ptr(target),
+               L.ptr(a["f"]), L.ptr(a["z1"]), L.ptr(a["a1"]), L.ptr(a["z2"]), L.ptr(a["a2"]), L.ptr(a["y"]),
+               L.ptr(gw["gy"]), L.ptr(gw["ga"]), L.ptr(gw["gz"]), L.ptr(gw["partial"]), nparts, L.ptr(gw["part"]),
+               L.ptr(self.g), L.stream_handle())
         return gw["partial"], a, gw
 
     def targets(self, E):

@@ -431,6 +431,17 @@ int ephip_mse_grad(int64_t n, const float *y, const float *t, float scale, float
 /* out[c] = sum over rows of x[r*ldx + c]. */
 int ephip_colsum(int32_t rows, int32_t cols, const float *x, int64_t ldx, float *out, void *stream);
 
+/* One gradient of the mean squared error of the network on npts points: features, forward and data-backward pass,
+ * weight and bias gradients. params and grad: the flat vectors W1 (hidden x 2 nf2), b1, W2 (hidden x hidden), b2,
+ * W3 (nout x hidden), b3 (params 16-byte aligned). Stores f (npts x 2 nf2), z1, a1, z2, a2 (npts x hidden), y
+ * (npts x nout), gy = dL/dy, gz2, gz1 = dL/dz and the squared error's sums over 256 entries as ephip_mse_grad.
+ * part: workspace of nparts partial gradients (nparts x the parameter count). 2 nf2 and hidden multiples of 16 up to
+ * 128, nout a multiple of 16 up to 64. z, a and y are those of ephip_gemm_f32 and ephip_silu_fwd bit for bit. */
+int ephip_mlp_train_step(int64_t npts, const double *xk, int32_t nf2, const int32_t *mvec, int32_t hidden,
+                         int32_t nout, const float *params, const float *target, float *f, float *z1, float *a1,
+                         float *z2, float *a2, float *y, float *gy, float *gz2, float *gz1, double *partial,
+                         int32_t nparts, float *part, float *grad, void *stream);
+
 /* One Adam step (bias-corrected, step counts from 1) on n parameters. */
 int ephip_adam_step(int64_t n, float *p, const float *g, float *m, float *v, float lr, float beta1, float beta2,
                     float eps, int32_t step, void *stream);
