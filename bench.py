@@ -334,7 +334,7 @@ def main():
     results = {}
     # ---- plain outer-q path (reference CS2 shape: separate Fourier / rotate kernels, full K_surv per q)
     if args.path in ("plain", "both"):
-        loop = eph.OuterQLoop(st, nk_batch=args.kbatch, nq_tile=args.qtile, precision=L.PREC_FP32)
+        loop = eph.OuterQLoop(st, nk_batch=args.kbatch, nq_tile=args.qtile, precision=L.PREC_FP32, staged=False)
         ev = []
         loop.ft_timer = ev
         for s in range(args.warmup):

@@ -267,7 +267,9 @@ class OuterQLoop:
     k, k+q lookup, windowed rotations and g2. Buffers are allocated once."""
 
     def __init__(self, st: OuterQSetup, nk_batch: int = 8192, nq_tile: int = 16,
-                 precision: int = L.PREC_FP32, keep_ep: bool = False):
+                 precision: int = L.PREC_FP32, keep_ep: bool = False, staged: bool = True):
+        """``staged``: Rq->kq by per-axis partial sums over the grid (FP32, csrc/staged_q.hip) where the Re box fits;
+        False, and other boxes, run the phase sums over Re at every k."""
         torch = _torch()
         self.st = st
         self.nk_batch = int(nk_batch)
@@ -279,11 +281,13 @@ class OuterQLoop:
         self.nr_el = st.epmat.ndata // nd_q
         self.gq_work = torch.empty((self.nq_tile, st.epmat.ndata), dtype=torch.complex64, device=dev)
         self.eRpq = torch.empty((self.nq_tile, st.epmat.ndata), dtype=torch.complex64, device=dev)
-        self.gk = torch.empty((self.nk_batch, nd_q), dtype=torch.complex64, device=dev)
-        self.g2 = torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.float32, device=dev)
-        self.ep = (torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.complex64, device=dev)
-                   if keep_ep else None)
         self.xk_surv = st.el.xk.index_select(0, st.ksurv).contiguous()
+        self.staged = _StagedRQ.build(self) if staged else None
+        if self.staged is None:
+            self.gk = torch.empty((self.nk_batch, nd_q), dtype=torch.complex64, device=dev)
+            self.g2 = torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.float32, device=dev)
+            self.ep = (torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.complex64, device=dev)
+                       if keep_ep else None)
         self.xq_host = st.ph.xq.cpu().numpy()
         # optional list collecting (start event, end event, columns) around each Rq->kq Fourier launch;
         # the events are recorded on the current stream, which is the stream the kernels run on
@@ -291,6 +295,19 @@ class OuterQLoop:
 
     def run_qtile(self, iq0: int, nq: int, calculators=()):
         st = self.st
+        if self.staged is not None:
+            self.staged.run(self, iq0, nq)
+            nks = st.ksurv.shape[0]
+            for t in range(nq):
+                for c in calculators:
+                    c.begin_q(iq0 + t)
+                for s in range(0, nks, self.nk_batch):
+                    payload = self.staged.payload(self, iq0, t, s, min(nks, s + self.nk_batch))
+                    for c in calculators:
+                        c.run(payload)
+                for c in calculators:
+                    c.end_q(iq0 + t)
+            return
         xq = st.ph.xq[iq0:iq0 + nq]
         uph = st.ph.u[iq0:iq0 + nq]
         get_eph_RR_to_Rq_batched(st.epmat, st.nw, st.nm, xq, uph, self.precision, work=self.gq_work,
@@ -328,6 +345,83 @@ class OuterQLoop:
         iq_stop = nq if iq_stop is None else min(nq, iq_stop)
         for iq0 in range(iq_start, iq_stop, self.nq_tile):
             self.run_qtile(iq0, min(self.nq_tile, iq_stop - iq0), calculators)
+
+
+class _StagedRQ:
+    """Staged Rq->kq of a tile of q (csrc/staged_q.hip): RR->Rq with the tile's q side by side, stage 1 of each k1
+    plane and the k-side projection of every unit (k, in-window band) over the rows (i, j, nu, q), then the k+q window
+    rotation and g2 of every (k, q)."""
+
+    @classmethod
+    def build(cls, loop):
+        st = loop.st
+        ks = st.ksurv.cpu().numpy()
+        if st.nw > 32 or st.nm > 48 or len(ks) == 0:
+            return None
+        go = _GridOptKR.build(st, ks, loop.nq_tile * st.nw * st.nw * st.nm, general=True, small=True)
+        return None if go is None else cls(loop, ks, go)
+
+    def __init__(self, loop, ks, go):
+        import ctypes
+        torch = _torch()
+        st = loop.st
+        dev = st.el.xk.device
+        nw, nm = st.nw, st.nm
+        self.go = go
+        self.st = st
+        f = st.el.filt
+        nb = (f.band_max - f.band_min + 1).cpu().numpy()[ks].astype(np.int64)
+        self.k_unit_start = np.concatenate([[0], np.cumsum(nb)])
+        self.k_unit_start_dev = torch.from_numpy(self.k_unit_start.astype(np.int32)).to(dev)
+        self.unit_kpos = torch.from_numpy(np.repeat(np.arange(len(ks)), nb).astype(np.int32)).to(dev)
+        self.unit_state = torch.from_numpy(np.repeat(ks, nb).astype(np.int64)).to(dev)
+        first = f.band_min.cpu().numpy()[ks] - 1
+        band = np.arange(self.k_unit_start[-1]) - np.repeat(self.k_unit_start[:-1] - first, nb)
+        self.unit_band = torch.from_numpy(band.astype(np.int32)).to(dev)
+        self.max_units_per_k = int(nb.max())
+        self.xk_surv = loop.xk_surv
+        self.nk_batch = min(loop.nk_batch, len(ks))
+        starts = range(0, len(ks), self.nk_batch)
+        self.max_units = max(int(self.k_unit_start[min(s + self.nk_batch, len(ks))] - self.k_unit_start[s]) for s in starts)
+        nt = loop.nq_tile
+        self.nrp = nm * nt   # go.run's columns per i: (nu, q)
+        self.A = torch.empty((self.max_units, nw * nm * nt), dtype=torch.complex64, device=dev)
+        self.epmat_el = loop.eRpq.view(loop.nr_el, nt * nw * nw * nm)   # rows (i, j, nu, q) of each Re
+        nrp = st.epmat.nr
+        self.phases = torch.empty(((nt + 15) // 16) * 16 * ((nrp + 3) // 4 * 4), dtype=torch.complex64, device=dev)
+        shape = (nt, len(ks), nm, st.nbw, st.nbw)
+        self.g2 = torch.empty(shape, dtype=torch.float32, device=dev)
+        self.ep = torch.empty(shape, dtype=torch.complex64, device=dev) if loop.keep_ep else None
+        self.ikq = torch.empty((nt, len(ks)), dtype=torch.int64, device=dev)
+        self.omega = st.ph.omega.contiguous()
+        self.uph = st.ph.u.contiguous()
+        self.kgrid_c = (ctypes.c_int32 * 3)(*map(int, st.kgrid))
+
+    def run(self, loop, iq0, nq):
+        """g2, ep and ikq of the tile's q at every surviving k."""
+        import ctypes as C
+        st, go = self.st, self.go
+        nw, nm = st.nw, st.nm
+        nks = st.ksurv.shape[0]
+        stream = L.stream_handle()
+        xq, om = st.ph.xq[iq0:iq0 + nq], self.omega[iq0:iq0 + nq]
+        L.call("ephip_staged_rr_to_rq", nw * nw, nm, loop.nr_el, st.epmat.nr, L.ptr(st.epmat.op_r), st.epmat.op_r.stride(0),
+               L.ptr(st.epmat.irvec_dev()), nq, L.ptr(xq), L.ptr(self.uph[iq0:iq0 + nq]), L.ptr(self.phases),
+               L.ptr(loop.gq_work), loop.gq_work.stride(0), L.ptr(self.epmat_el), self.epmat_el.stride(0), stream)
+        go.nd = nq * nw * nw * nm
+        go.invalidate()
+        for s in range(0, nks, self.nk_batch):
+            n = min(self.nk_batch, nks - s)
+            u0, u1 = int(self.k_unit_start[s]), int(self.k_unit_start[s + n])
+            go.run(self, s, n, u0, u1, self.A, stream)
+            L.call("ephip_staged_rq_rotate", nw, nm, st.nbw, nq, s, n, L.ptr(st.ksurv), L.ptr(st.el.xk), L.ptr(xq),
+                   C.addressof(self.kgrid_c), L.ptr(self.k_unit_start_dev), L.ptr(self.A), self.A.stride(0),
+                   L.ptr(st.el.U), L.ptr(st.el.filt.band_min), L.ptr(st.el.filt.band_max), L.ptr(om), nks,
+                   L.ptr(self.ikq), L.ptr(self.g2), L.ptr(self.ep), stream)
+
+    def payload(self, loop, iq0, t, s, e):
+        return EPDataKWindowed(iq0 + t, self.st.ksurv[s:e], self.ikq[t, s:e], self.g2[t, s:e],
+                               None if self.ep is None else self.ep[t, s:e], self.st.nbw)
 
 
 class _RqObject(WannierObject):
@@ -899,20 +993,20 @@ class _GridOptKR:
     SMALL_BOX = 3
 
     @classmethod
-    def build(cls, st, ks, nd, mfma=True, general=False):
+    def build(cls, st, ks, nd, mfma=True, general=False, small=False):
         r = np.asarray(st.irvec_el_dev.cpu().numpy(), dtype=np.int64)
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         kg = np.asarray(st.kgrid, dtype=np.int64)
         if (len(ks) == 0 or n[0] > cls.N1_MAX or n[1] > cls.N23_MAX or n[2] > cls.N23_MAX
-                or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and n.max() <= cls.SMALL_BOX)):
+                or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)):
             return None
         return cls(st, ks, nd, r, lo, n, kg, mfma, general)
 
     def __init__(self, st, ks, nd, r, lo, n, kg, mfma, general=False):
         torch = _torch()
         dev = st.el.xk.device
-        self.nd = nd
+        self.nd = self.nd_max = nd   # rows in use, and what the plane buffers hold
         # stages 2/3 on the matrix cores for nw = 16 (op1 rows in natural order); otherwise the VALU form,
         # whose lane reduction wants op1 rows j-fastest
         self.mfma = bool(mfma) and st.nw == 16
@@ -978,7 +1072,7 @@ class _GridOptKR:
         g = self.plane_pos[plane] // self.PLANES
         members = self.planes[g * self.PLANES:(g + 1) * self.PLANES]
         if len(self.cache) < 2:
-            bufs = [torch.empty((self.np * self.np, self.nd), dtype=torch.complex64, device=epmat_el.device)
+            bufs = [torch.empty((self.np * self.np, self.nd_max), dtype=torch.complex64, device=epmat_el.device)
                     for _ in range(self.PLANES)]
         else:  # reuse the older group's buffers (stream order: its projections are already queued)
             bufs = self.cache.pop(0)[2]

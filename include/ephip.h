@@ -356,6 +356,25 @@ int ephip_staged_kq(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits, int32_t
                     const double *omega, const int32_t *dense_strides, double cols_hint, double width_hint,
                     float *g2, void *ep, void *stream);
 
+/* The outer-q loop by staged transforms, for a tile of nq q (FP32, nw <= 32, nm <= 48):
+ *  - ephip_staged_rr_to_rq: get_eph_RR_to_Rq! (src/wannier_to_bloch.jl:277-300) at the tile's q (xq, 3 per q) from the
+ *    "ph" layout tensor op (rows b + nbasis (nu + nm Re), nbasis = nw^2, one column per Rp, ldop), with the q side by
+ *    side: out[b + nbasis (nu' + nm q) + ldout Re]. work: nq columns of ldwork >= nbasis nm nre complex64; phases:
+ *    workspace of ceil(nq / 16) 16 nrp' complex64, nrp' = nrp rounded up to a multiple of 4. uph (nm, nm, nq).
+ *    Its rows (i, j, nu, q) then take ephip_gridopt_stage1_planes and ephip_staged_project (ngcol = nw nm nq).
+ *  - ephip_staged_rq_rotate: k+q window rotation and g2 (eph_apply_rotations_rqkq! after the k-side projection,
+ *    src/wannier_to_bloch_batched.jl:360-377 and :451-453) for the surviving k k0 <= k < k0 + nk (states ks) and the
+ *    tile's q: A (lda per unit, columns i + nw (nu + nm q)) from ephip_staged_project, kus as there; xk of every grid
+ *    state, ngrid (host) the k grid, omega (nm, nq). Row ldk q + k of ikq (int64), g2 and ep (complex64, may be NULL)
+ *    holds k+q's grid index and the window block of ephip_eph_rotate_rqkq_g2. */
+int ephip_staged_rr_to_rq(int64_t nbasis, int32_t nm, int32_t nre, int32_t nrp, const void *op, int64_t ldop,
+                          const int32_t *irvec, int32_t nq, const double *xq, const void *uph, void *phases, void *work,
+                          int64_t ldwork, void *out, int64_t ldout, void *stream);
+int ephip_staged_rq_rotate(int32_t nw, int32_t nm, int32_t nbw, int32_t nq, int64_t k0, int32_t nk, const int64_t *ks,
+                           const double *xk, const double *xq, const int32_t *ngrid, const int32_t *kus, const void *A,
+                           int64_t lda, const void *U, const int64_t *bmin, const int64_t *bmax, const double *omega,
+                           int64_t ldk, int64_t *ikq, float *g2, void *ep, void *stream);
+
 /* kR->kq Fourier over Rp fused with the k+q-window and phonon rotations and g2 (the
  * get_eph_kR_to_kq_batched! + eph_apply_rotations! + g2 sequence of src/wannier_to_bloch_batched.jl:
  * 245-273 and :442-455 in one kernel) for nw = 16, nm = 12, nbw <= 4, split-BF16: apk holds the

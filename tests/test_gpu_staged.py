@@ -93,3 +93,50 @@ def test_staged_entries_refuse_what_they_do_not_cover(backend):
         with pytest.raises(L.EphipError, match=msg):
             kq(**kw)
     kq(nunits=0)
+
+
+@pytest.mark.parametrize("nw,atoms,box,cut,kgrid,qgrid,window,tile,nk_batch", [
+    (1, 1, 3, None, (4, 5, 4), (4, 5, 4), 4.0, 3, 8),
+    (3, 1, 5, None, (5, 7, 3), (5, 7, 3), 1.5, 17, 1000),       # odd rows: no paired loads; two launches of q columns
+    (4, 1, 7, (None, -2, -1), (4, 6, 4), (2, 6, 4), 1.0, 16, 13),  # uneven box, several k batches
+    (7, 2, 5, None, (4, 4, 4), (4, 4, 4), 1.5, 5, 40),
+    (16, 4, 3, None, (4, 4, 4), (2, 2, 2), 1.5, 8, 8192),
+    (13, 6, 5, None, (4, 3, 4), (4, 3, 4), 2.5, 4, 20),          # 18 modes, wide window
+    (32, 1, 3, None, (3, 4, 2), (3, 4, 2), 1.0, 2, 5),
+])
+def test_staged_outer_q_against_direct(backend, nw, atoms, box, cut, kgrid, qgrid, window, tile, nk_batch):
+    import torch
+    from ephip import eph
+    m = M.make_model(nw=nw, natoms=atoms, box_hd=5, box_g=box, seed=700 + nw, g_dtype=np.complex64)
+    if cut is not None:
+        m = _cut(m, cut)
+    st = eph.setup_outer_q(m, kgrid, qgrid, (-window, window), backend)
+    nq = st.ph.xq.shape[0]
+    staged = eph.OuterQLoop(st, nk_batch=nk_batch, nq_tile=tile, keep_ep=True)
+    direct = eph.OuterQLoop(st, nk_batch=nk_batch, nq_tile=tile, keep_ep=True, staged=False)
+    assert staged.staged is not None and direct.staged is None
+
+    class Keep(eph.AbstractCalculator):
+        def __init__(self):
+            self.got = []
+
+        def run(self, p):
+            self.got.append((p.iq, p.ik.clone(), p.ikq.clone(), p.g2.clone(), p.ep.clone()))
+
+    a, b = Keep(), Keep()
+    for iq0, n in ((0, min(tile, nq)), (nq - 1, 1), (1, min(tile, nq - 1))):   # whole, single and partial tiles
+        staged.run_qtile(iq0, n, [a])
+        direct.run_qtile(iq0, n, [b])
+    assert len(a.got) == len(b.got)
+    num = den = 0.0
+    for x, y in zip(a.got, b.got):
+        assert x[0] == y[0] and torch.equal(x[1], y[1]) and torch.equal(x[2], y[2])
+        ok = st.ph.omega[x[0]] > 1e-4
+        assert torch.equal(x[3] == 0, y[3] == 0)
+        if not bool(ok.any()):   # q = 0 of one atom: acoustic modes only
+            continue
+        g, r = x[3].double()[:, ok], y[3].double()[:, ok]
+        num, den = max(num, float((g - r).abs().max())), max(den, float(r.max()))
+        e2 = x[4].abs().double().square()[:, ok] / (2 * st.ph.omega[x[0]][ok]).view(1, -1, 1, 1)
+        assert bool(((e2 - g).abs() <= 1e-5 * (g.abs() + 1e-30)).all())
+    assert den > 0 and num <= 1e-5 * den, num / den
