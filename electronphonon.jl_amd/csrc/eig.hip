@@ -262,17 +262,20 @@ __global__ __launch_bounds__(256) void heev_c32_kernel(int n, int64_t nb, const 
 //      (V is orthonormal to ~1e-6, two steps reach ~1e-23);
 //   2. M = Q^H H Q is unitarily similar to H and nearly diagonal (off-diagonal ~ FP32 residual);
 //   3. cyclic Jacobi sweeps on M in FP64, the n/2 disjoint rotations of a round-robin round applied
-//      in parallel (columns: lane = row; rows: lane = column), accumulated into Q. Convergence is
+//      in parallel (a lane per rotation and row or column), accumulated into Q. Convergence is
 //      quadratic from a nearly diagonal start, and exact or close eigenvalue pairs need no special
 //      handling (a degenerate pair gets a well-defined 45-degree rotation).
 // Eigenvalues are diag(M) sorted ascending, eigenvectors the matching columns of Q (rounded to FP32).
-// LDS per wave: H | Q | W | M (n columns of c64 each, column pitch ld = n | 1) + rotation table and
-// ranks. The odd pitch spreads the 16-byte column-strided accesses (lane = column) over the banks; with
-// ld = n = 16 every lane of such an access fell on the same banks.
+// LDS per wave: three matrices of n columns of c64 (column pitch ld = n | 1), which hold Q, S = Q^H Q and the
+// orthonormalised Q in turn, then Q, H Q and H or M, + rotation table and ranks. The odd pitch spreads the 16-byte
+// column-strided accesses (lane = column) over the banks; with ld = n = 16 every lane of such an access fell on the
+// same banks. The LDS sets how many matrices a CU works on, and they hide one another's latencies.
+// With the rotations' items spread over all lanes (they were n lanes working through the pairs) and three matrices for
+// four: 110592 matrices of n = 16 in 5.3 ms for 15.4, the same bits.
 // ---------------------------------------------------------------------------------------------
-constexpr int REFINE_EXTRA_DOUBLES = 176;
+constexpr int REFINE_EXTRA_DOUBLES = 128;
 __host__ __device__ constexpr int refine_ld(int n) { return n | 1; }
-__host__ __device__ constexpr int refine_lds_doubles(int n) { return 8 * n * refine_ld(n) + REFINE_EXTRA_DOUBLES; }
+__host__ __device__ constexpr int refine_lds_doubles(int n) { return 6 * n * refine_ld(n) + REFINE_EXTRA_DOUBLES; }
 
 __device__ __forceinline__ double rdl64(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
@@ -286,39 +289,57 @@ __device__ __forceinline__ c64 cmulc(c64 a, c64 b) {  // conj(a) * b
 }
 __device__ __forceinline__ c64 cadd(c64 a, c64 b) { return c64{a.re + b.re, a.im + b.im}; }
 
-struct JacobiRot {
+struct JacobiRot {  // G = diag(1, e^{-i phi}) [[cs, sn], [-sn, cs]] on (p, q); its upper row is real
+    double cs, sn;
+    c64 gqp, gqq;
     int p, q;
-    c64 gpp, gpq, gqp, gqq;  // G = diag(1, e^{-i phi}) [[cs, sn], [-sn, cs]] on (p, q)
 };
+static_assert(16 * sizeof(JacobiRot) + 32 * sizeof(int) <= REFINE_EXTRA_DOUBLES * sizeof(double));
 
-// n x n matrices in LDS with column pitch ld (element (r, j) at r + ld*j); lanes over entries.
-// out = alpha * A B + beta * C
-__device__ void lds_gemm_nn(int n, int ld, const c64 *A, const c64 *B, c64 *out, double alpha, double beta,
-                            const c64 *C, int lane) {
-    for (int e = lane; e < n * n; e += 64) {
-        const int r = e % n, j = e / n;
-        c64 s{0.0, 0.0};
-        for (int k = 0; k < n; k++) s = cadd(s, cmul(A[r + ld * k], B[k + ld * j]));
-        c64 v{alpha * s.re, alpha * s.im};
-        if (beta != 0.0) v = c64{v.re + beta * C[r + ld * j].re, v.im + beta * C[r + ld * j].im};
-        out[r + ld * j] = v;
-    }
-}
-
-// out = A^H B
-__device__ void lds_gemm_cn(int n, int ld, const c64 *A, const c64 *B, c64 *out, int lane) {
-    for (int e = lane; e < n * n; e += 64) {
-        const int i = e % n, j = e / n;
-        c64 s{0.0, 0.0};
-        for (int r = 0; r < n; r++) s = cadd(s, cmulc(A[r + ld * i], B[r + ld * j]));
-        out[i + ld * j] = s;
+// n x n matrices in LDS with column pitch ld (element (r, j) at r + ld*j); a lane forms 2 x 2 entries at a time, so an
+// operand read serves two of them. The sum over k of an entry runs in order.
+// out = alpha * A B + beta * C (op == 0) or A^H B (op == 1)
+template <int OP>
+__device__ __forceinline__ void lds_gemm(int n, int ld, const c64 *A, const c64 *B, c64 *out, double alpha, double beta,
+                                         const c64 *C, int lane) {
+    const int T = (n + 1) >> 1;
+    for (int e = lane; e < T * T; e += 64) {
+        const int tr = e % T, tj = e / T;
+        const int r0 = 2 * tr, r1 = min(r0 + 1, n - 1), j0 = 2 * tj, j1 = min(j0 + 1, n - 1);
+        c64 s00{0.0, 0.0}, s01{0.0, 0.0}, s10{0.0, 0.0}, s11{0.0, 0.0};
+        for (int k = 0; k < n; k++) {
+            const c64 a0 = OP ? A[k + ld * r0] : A[r0 + ld * k], a1 = OP ? A[k + ld * r1] : A[r1 + ld * k];
+            const c64 b0 = B[k + ld * j0], b1 = B[k + ld * j1];
+            if constexpr (OP) {
+                s00 = cadd(s00, cmulc(a0, b0));
+                s01 = cadd(s01, cmulc(a0, b1));
+                s10 = cadd(s10, cmulc(a1, b0));
+                s11 = cadd(s11, cmulc(a1, b1));
+            } else {
+                s00 = cadd(s00, cmul(a0, b0));
+                s01 = cadd(s01, cmul(a0, b1));
+                s10 = cadd(s10, cmul(a1, b0));
+                s11 = cadd(s11, cmul(a1, b1));
+            }
+        }
+        auto put = [&](int r, int j, c64 v) {  // the repeated row or column of an odd n writes the same value again
+            if constexpr (!OP) {
+                v = c64{alpha * v.re, alpha * v.im};
+                if (beta != 0.0) v = c64{v.re + beta * C[r + ld * j].re, v.im + beta * C[r + ld * j].im};
+            }
+            out[r + ld * j] = v;
+        };
+        put(r0, j0, s00);
+        put(r0, j1, s01);
+        put(r1, j0, s10);
+        put(r1, j1, s11);
     }
 }
 
 // Parallel cyclic Jacobi on the n x n Hermitian M (LDS, column pitch ldm, n <= 32): the n/2 disjoint
-// rotations of a round-robin round are applied in parallel (columns: lane = row; rows: lane = column) and
-// accumulated into the n columns of Q (qrows x n, column pitch ldq, qrows <= 64). Stops when the
-// strict upper triangle's Frobenius norm (the part the rotations remove; rounding leaves M Hermitian only
+// rotations of a round-robin round are applied in parallel, one lane per (rotation, row) of M and Q, then one per
+// (rotation, column) of M, and accumulated into the n columns of Q (qrows x n, column pitch ldq, qrows <= 64). Stops
+// when the strict upper triangle's Frobenius norm (the part the rotations remove; rounding leaves M Hermitian only
 // to a few ulps, and unitary rotations cannot remove that anti-Hermitian residue) is <= tol/sqrt(2) x the
 // Frobenius norm, or after 12 sweeps. A pivot below 1e-20 of its diagonal scale is left alone: rotating it
 // would only shrink it further, towards the subnormal range where its phase can no longer be normalised
@@ -345,15 +366,17 @@ __device__ void wave_jacobi(int n, c64 *M, int ldm, c64 *Q, int ldq, int qrows, 
                 if (lane == 0) {
                     a = N - 1;
                     c = rd;
-                } else {
-                    a = (rd + lane) % (N - 1);
-                    c = (rd - lane + (N - 1)) % (N - 1);
+                } else {  // (rd + lane) and (rd - lane) modulo N - 1
+                    a = rd + lane;
+                    c = rd - lane;
+                    if (a >= N - 1) a -= N - 1;
+                    if (c < 0) c += N - 1;
                 }
                 JacobiRot g;
                 g.p = min(a, c);
                 g.q = max(a, c);
-                g.gpp = c64{1.0, 0.0};
-                g.gpq = c64{0.0, 0.0};
+                g.cs = 1.0;
+                g.sn = 0.0;
                 g.gqp = c64{0.0, 0.0};
                 g.gqq = c64{1.0, 0.0};
                 if (g.q < n) {
@@ -365,8 +388,8 @@ __device__ void wave_jacobi(int n, c64 *M, int ldm, c64 *Q, int ldq, int qrows, 
                         const double tau = (M[g.q + ldm * g.q].re - M[g.p + ldm * g.p].re) / (2.0 * amp);
                         const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
                         const double cs = 1.0 / sqrt(1.0 + t * t), sn = t * cs;
-                        g.gpp = c64{cs, 0.0};
-                        g.gpq = c64{sn, 0.0};
+                        g.cs = cs;
+                        g.sn = sn;
                         g.gqp = c64{-sn * er, sn * ei};
                         g.gqq = c64{cs * er, -cs * ei};
                     }
@@ -376,31 +399,35 @@ __device__ void wave_jacobi(int n, c64 *M, int ldm, c64 *Q, int ldq, int qrows, 
                 rot[lane] = g;
             }
             wave_lds_sync();
-            if (lane < n || lane < qrows) {  // M <- M G, Q <- Q G (lane = row)
-                for (int k = 0; k < npairs; k++) {
-                    const JacobiRot g = rot[k];
-                    if (g.p == g.q) continue;
-                    if (lane < n) {
-                        const c64 mp = M[lane + ldm * g.p], mq = M[lane + ldm * g.q];
-                        M[lane + ldm * g.p] = cadd(cmul(mp, g.gpp), cmul(mq, g.gqp));
-                        M[lane + ldm * g.q] = cadd(cmul(mp, g.gpq), cmul(mq, g.gqq));
-                    }
-                    if (lane < qrows) {
-                        const c64 qp = Q[lane + ldq * g.p], qq = Q[lane + ldq * g.q];
-                        Q[lane + ldq * g.p] = cadd(cmul(qp, g.gpp), cmul(qq, g.gqp));
-                        Q[lane + ldq * g.q] = cadd(cmul(qp, g.gpq), cmul(qq, g.gqq));
-                    }
-                }
+            // M <- M G, Q <- Q G
+            for (int e = lane; e < npairs * n; e += 64) {
+                const int k = e / n, r = e - k * n;
+                const JacobiRot g = rot[k];
+                if (g.p == g.q) continue;
+                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
+                const c64 mp = M[r + ldm * g.p], mq = M[r + ldm * g.q];
+                M[r + ldm * g.p] = cadd(cmul(mp, gpp), cmul(mq, g.gqp));
+                M[r + ldm * g.q] = cadd(cmul(mp, gpq), cmul(mq, g.gqq));
+            }
+            for (int e = lane; e < npairs * qrows; e += 64) {
+                const int k = e / qrows, r = e - k * qrows;
+                const JacobiRot g = rot[k];
+                if (g.p == g.q) continue;
+                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
+                const c64 qp = Q[r + ldq * g.p], qq = Q[r + ldq * g.q];
+                Q[r + ldq * g.p] = cadd(cmul(qp, gpp), cmul(qq, g.gqp));
+                Q[r + ldq * g.q] = cadd(cmul(qp, gpq), cmul(qq, g.gqq));
             }
             wave_lds_sync();
-            if (lane < n) {  // M <- G^H M (lane = column)
-                for (int k = 0; k < npairs; k++) {
-                    const JacobiRot g = rot[k];
-                    if (g.p == g.q) continue;
-                    const c64 mp = M[g.p + ldm * lane], mq = M[g.q + ldm * lane];
-                    M[g.p + ldm * lane] = cadd(cmulc(g.gpp, mp), cmulc(g.gqp, mq));
-                    M[g.q + ldm * lane] = cadd(cmulc(g.gpq, mp), cmulc(g.gqq, mq));
-                }
+            // M <- G^H M
+            for (int e = lane; e < npairs * n; e += 64) {
+                const int k = e / n, c = e - k * n;
+                const JacobiRot g = rot[k];
+                if (g.p == g.q) continue;
+                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
+                const c64 mp = M[g.p + ldm * c], mq = M[g.q + ldm * c];
+                M[g.p + ldm * c] = cadd(cmulc(gpp, mp), cmulc(g.gqp, mq));
+                M[g.q + ldm * c] = cadd(cmulc(gpq, mp), cmulc(g.gqq, mq));
             }
             wave_lds_sync();
         }
@@ -415,35 +442,39 @@ __global__ __launch_bounds__(256) void heev_refine_kernel(int n, int64_t nb, con
     const int64_t b = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave;
     if (b >= nb) return;
     const int nn = n * n, ld = refine_ld(n), nl = n * ld;
-    c64 *Hs = reinterpret_cast<c64 *>(lds64 + (int64_t)wave * refine_lds_doubles(n));
-    c64 *Q = Hs + nl;
+    c64 *Q = reinterpret_cast<c64 *>(lds64 + (int64_t)wave * refine_lds_doubles(n));
     c64 *W = Q + nl;
     c64 *M = W + nl;
-    JacobiRot *rot = reinterpret_cast<JacobiRot *>(M + nl);  // 16 x 72 bytes
+    JacobiRot *rot = reinterpret_cast<JacobiRot *>(M + nl);  // 16 x 56 bytes
     int *rank_s = reinterpret_cast<int *>(rot + 16);           // n ints
+    for (int e = lane; e < nn; e += 64) {
+        const int i = e % n, j = e / n;
+        const c32 u = U[b * nn + e];
+        Q[i + ld * j] = c64{u.re, u.im};
+    }
+    wave_lds_sync();
+    // 1. two Loewdin steps: S = Q^H Q (in W), M = 3/2 Q - 1/2 Q S, which is the next Q
+    for (int it = 0; it < 2; it++) {
+        lds_gemm<1>(n, ld, Q, Q, W, 0.0, 0.0, nullptr, lane);
+        wave_lds_sync();
+        lds_gemm<0>(n, ld, Q, W, M, -0.5, 1.5, Q, lane);
+        wave_lds_sync();
+        c64 *x = Q;
+        Q = M;
+        M = x;
+    }
+    // 2. M = Q^H (H Q), H where M goes
     for (int e = lane; e < nn; e += 64) {
         const int i = e % n, j = e / n;
         c64 h = (i <= j) ? H[b * nn + i + (int64_t)n * j] : H[b * nn + j + (int64_t)n * i];
         if (i > j) h.im = -h.im;
         if (i == j) h.im = 0.0;
-        Hs[i + ld * j] = h;
-        const c32 u = U[b * nn + e];
-        Q[i + ld * j] = c64{u.re, u.im};
+        M[i + ld * j] = h;
     }
     wave_lds_sync();
-    // 1. two Loewdin steps: S = Q^H Q (in W), M = 3/2 Q - 1/2 Q S, Q <- M
-    for (int it = 0; it < 2; it++) {
-        lds_gemm_cn(n, ld, Q, Q, W, lane);
-        wave_lds_sync();
-        lds_gemm_nn(n, ld, Q, W, M, -0.5, 1.5, Q, lane);
-        wave_lds_sync();
-        for (int e = lane; e < nn; e += 64) Q[e % n + ld * (e / n)] = M[e % n + ld * (e / n)];
-        wave_lds_sync();
-    }
-    // 2. M = Q^H (H Q)
-    lds_gemm_nn(n, ld, Hs, Q, W, 1.0, 0.0, nullptr, lane);
+    lds_gemm<0>(n, ld, M, Q, W, 1.0, 0.0, nullptr, lane);
     wave_lds_sync();
-    lds_gemm_cn(n, ld, Q, W, M, lane);
+    lds_gemm<1>(n, ld, Q, W, M, 0.0, 0.0, nullptr, lane);
     wave_lds_sync();
     // 3. parallel cyclic Jacobi
     wave_jacobi(n, M, ld, Q, ld, n, rot, lane, tol);
@@ -567,6 +598,17 @@ static int waves_per_block(size_t lds_per_wave) {
     return w < 1 ? 1 : (w > 4 ? 4 : w);
 }
 
+// The same for the refinement, whose LDS decides how many matrices share a CU: of the workgroups of 1, 2 and 4 waves
+// that its 160 KiB hold, the larger ones where they hold as many waves.
+static int refine_waves_per_block(size_t lds_per_wave) {
+    int best = 1;
+    for (int w : {2, 4}) {
+        const size_t cu = 160 * 1024;
+        if (w * lds_per_wave <= 64 * 1024 && cu / (w * lds_per_wave) * w >= cu / (best * lds_per_wave) * best) best = w;
+    }
+    return best;
+}
+
 static int heev_launch_check(int n, int64_t nb) {
     EPHIP_REQUIRE(n >= 1 && n <= 32, "heev: n=%d outside 1..32 (one wavefront per matrix)", n);
     EPHIP_REQUIRE(nb >= 0, "heev: negative batch");
@@ -600,9 +642,9 @@ extern "C" int ephip_heev_refine(int32_t n, int64_t nb, const void *H64, void *U
     EPHIP_REQUIRE(H64 && U && E64, "heev_refine: null device pointer");
     EPHIP_REQUIRE(tol >= 0.0, "heev_refine: negative tolerance");
     (void)E32;
-    const int wpb = waves_per_block(sizeof(double) * refine_lds_doubles(n));
+    const int wpb = refine_waves_per_block(sizeof(double) * refine_lds_doubles(n));
     const size_t lds = wpb * sizeof(double) * refine_lds_doubles(n);
-    if (lds > 64 * 1024) {  // n = 32: one matrix's FP64 working set (67 KiB) in a one-wave block; gfx950 has
+    if (lds > 64 * 1024) {  // n = 32: one matrix's FP64 working set in a one-wave block; gfx950 has
                             // 160 KiB of LDS per workgroup
         EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(heev_refine_kernel),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
