@@ -1,4 +1,4 @@
-// Batched Hermitian eigensolve for small matrices (n <= 32), one wavefront per matrix.
+// Batched Hermitian eigensolve for small matrices (n <= 32), one wavefront or a part of one per matrix.
 //
 // Replaces the reference's eigen_batched / eigvals_batched (src/wannier_to_bloch_batched.jl:30-65,
 // CUDA method ext/ElectronPhononCUDAExt.jl:80-115): ascending eigenvalues, orthonormal eigenvectors,
@@ -26,7 +26,10 @@ namespace ephip {
 struct c32 {
     float re, im;
 };
-struct c64 {
+struct c64u {  // a caller's element, aligned to its parts
+    double re, im;
+};
+struct alignas(16) c64 {  // one in LDS, moved by 16-byte accesses
     double re, im;
 };
 
@@ -257,25 +260,23 @@ __global__ __launch_bounds__(256) void heev_c32_kernel(int n, int64_t nb, const 
 }
 
 // ---------------------------------------------------------------------------------------------
-// FP64 refinement, one wave per matrix, in the basis of the FP32 eigenvectors:
+// FP64 refinement, one, two or four matrices per wave, in the basis of the FP32 eigenvectors:
 //   1. Q = V orthonormalised in FP64 by two Loewdin steps Q <- Q (3/2 I - 1/2 Q^H Q)
 //      (V is orthonormal to ~1e-6, two steps reach ~1e-23);
 //   2. M = Q^H H Q is unitarily similar to H and nearly diagonal (off-diagonal ~ FP32 residual);
 //   3. cyclic Jacobi sweeps on M in FP64, the n/2 disjoint rotations of a round-robin round applied
-//      in parallel (a lane per rotation and row or column), accumulated into Q. Convergence is
-//      quadratic from a nearly diagonal start, and exact or close eigenvalue pairs need no special
-//      handling (a degenerate pair gets a well-defined 45-degree rotation).
+//      in parallel, accumulated into Q. Convergence is quadratic from a nearly diagonal start, and exact or
+//      close eigenvalue pairs need no special handling (a degenerate pair gets a well-defined 45-degree
+//      rotation).
 // Eigenvalues are diag(M) sorted ascending, eigenvectors the matching columns of Q (rounded to FP32).
-// LDS per wave: three matrices of n columns of c64 (column pitch ld = n | 1), which hold Q, S = Q^H Q and the
-// orthonormalised Q in turn, then Q, H Q and H or M, + rotation table and ranks. The odd pitch spreads the 16-byte
-// column-strided accesses (lane = column) over the banks; with ld = n = 16 every lane of such an access fell on the
-// same banks. The LDS sets how many matrices a CU works on, and they hide one another's latencies.
-// With the rotations' items spread over all lanes (they were n lanes working through the pairs) and three matrices for
-// four: 110592 matrices of n = 16 in 5.3 ms for 15.4, the same bits.
+// LDS per matrix: Q and M (n columns of c64, column pitch ld = n | 1); M holds Q^H Q and H before. The odd pitch
+// spreads the 16-byte column-strided accesses (lane = column) over the banks; with ld = n = 16 every lane of such an
+// access fell on the same banks. Its accesses bound the kernel, then the FP64 arithmetic; 16-byte alignment halves their
+// cycles (an 8-byte aligned element goes as two 8-byte accesses with a stride of 16).
+// 110592 matrices of n = 16: 2.9 ms; one lane a row working through the rotations of one matrix took 15.4.
 // ---------------------------------------------------------------------------------------------
-constexpr int REFINE_EXTRA_DOUBLES = 128;
 __host__ __device__ constexpr int refine_ld(int n) { return n | 1; }
-__host__ __device__ constexpr int refine_lds_doubles(int n) { return 6 * n * refine_ld(n) + REFINE_EXTRA_DOUBLES; }
+__host__ __device__ constexpr int refine_lds_doubles(int n) { return 4 * n * refine_ld(n); }
 
 __device__ __forceinline__ double rdl64(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
@@ -283,218 +284,271 @@ __device__ __forceinline__ double rdl64(double v, int l) {
     return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ c64 cmul(c64 a, c64 b) { return c64{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
+// Products with the contraction written out: the vectors' phases come from rounding, so every form of these kernels
+// rounds alike.
+__device__ __forceinline__ c64 cmul(c64 a, c64 b) {
+    return c64{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.re, b.im, a.im * b.re)};
+}
+__device__ __forceinline__ c64 cmul_swapped(c64 a, c64 b) {  // a * b as cmul(b, a) rounds it
+    return c64{__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im)};
+}
 __device__ __forceinline__ c64 cmulc(c64 a, c64 b) {  // conj(a) * b
-    return c64{a.re * b.re + a.im * b.im, a.re * b.im - a.im * b.re};
+    return c64{__builtin_fma(a.re, b.re, a.im * b.im), __builtin_fma(a.re, b.im, -(a.im * b.re))};
 }
 __device__ __forceinline__ c64 cadd(c64 a, c64 b) { return c64{a.re + b.re, a.im + b.im}; }
 
-struct JacobiRot {  // G = diag(1, e^{-i phi}) [[cs, sn], [-sn, cs]] on (p, q); its upper row is real
-    double cs, sn;
-    c64 gqp, gqq;
-    int p, q;
+// e / n for e < 2048, n <= 32 by a multiplication: an integer division by a run-time n costs twenty instructions
+struct SmallDiv {
+    int n;
+    unsigned magic;
+    __device__ explicit SmallDiv(int n_) : n(n_), magic(65536u / n_ + 1u) {}
+    __device__ int div(int e) const { return (int)(((unsigned)e * magic) >> 16); }
+    __device__ int mod(int e) const { return e - div(e) * n; }
 };
-static_assert(16 * sizeof(JacobiRot) + 32 * sizeof(int) <= REFINE_EXTRA_DOUBLES * sizeof(double));
 
-// n x n matrices in LDS with column pitch ld (element (r, j) at r + ld*j); a lane forms 2 x 2 entries at a time, so an
-// operand read serves two of them. The sum over k of an entry runs in order.
-// out = alpha * A B + beta * C (op == 0) or A^H B (op == 1)
-template <int OP>
+// n x n matrices in LDS with column pitch ld (element (r, j) at r + ld*j), W lanes a matrix (l = lane of W). A lane
+// forms tiles of 2 x 2 entries, so an operand read serves two of them, and keeps them in registers: out may be A or B.
+// The sum over k of an entry runs in order. NT * W >= the ceil(n/2)^2 tiles.
+// out = alpha * A B + beta * C (OP == 0) or A^H B (OP == 1); C is read before out is written
+template <int OP, int NT, int W>
 __device__ __forceinline__ void lds_gemm(int n, int ld, const c64 *A, const c64 *B, c64 *out, double alpha, double beta,
-                                         const c64 *C, int lane) {
+                                         const c64 *C, int l) {
     const int T = (n + 1) >> 1;
-    for (int e = lane; e < T * T; e += 64) {
-        const int tr = e % T, tj = e / T;
-        const int r0 = 2 * tr, r1 = min(r0 + 1, n - 1), j0 = 2 * tj, j1 = min(j0 + 1, n - 1);
-        c64 s00{0.0, 0.0}, s01{0.0, 0.0}, s10{0.0, 0.0}, s11{0.0, 0.0};
-        for (int k = 0; k < n; k++) {
-            const c64 a0 = OP ? A[k + ld * r0] : A[r0 + ld * k], a1 = OP ? A[k + ld * r1] : A[r1 + ld * k];
-            const c64 b0 = B[k + ld * j0], b1 = B[k + ld * j1];
-            if constexpr (OP) {
-                s00 = cadd(s00, cmulc(a0, b0));
-                s01 = cadd(s01, cmulc(a0, b1));
-                s10 = cadd(s10, cmulc(a1, b0));
-                s11 = cadd(s11, cmulc(a1, b1));
-            } else {
-                s00 = cadd(s00, cmul(a0, b0));
-                s01 = cadd(s01, cmul(a0, b1));
-                s10 = cadd(s10, cmul(a1, b0));
-                s11 = cadd(s11, cmul(a1, b1));
-            }
-        }
-        auto put = [&](int r, int j, c64 v) {  // the repeated row or column of an odd n writes the same value again
-            if constexpr (!OP) {
-                v = c64{alpha * v.re, alpha * v.im};
-                if (beta != 0.0) v = c64{v.re + beta * C[r + ld * j].re, v.im + beta * C[r + ld * j].im};
-            }
-            out[r + ld * j] = v;
-        };
-        put(r0, j0, s00);
-        put(r0, j1, s01);
-        put(r1, j0, s10);
-        put(r1, j1, s11);
+    const SmallDiv byT(T);
+    c64 acc[NT][2][2];
+    int r[NT][2], j[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int e = min(l + t * W, T * T - 1);  // the lanes left over repeat the last tile
+        const int tj = byT.div(e), tr = e - T * tj;
+        r[t][0] = 2 * tr;
+        r[t][1] = min(2 * tr + 1, n - 1);  // an odd n's repeated row or column writes the same value again
+        j[t][0] = 2 * tj;
+        j[t][1] = min(2 * tj + 1, n - 1);
+#pragma unroll
+        for (int x = 0; x < 4; x++) acc[t][x >> 1][x & 1] = c64{0.0, 0.0};
     }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+        for (int k = 0; k < n; k++) {
+            c64 a[2], b[2];
+#pragma unroll
+            for (int x = 0; x < 2; x++) {
+                a[x] = OP ? A[k + ld * r[t][x]] : A[r[t][x] + ld * k];
+                b[x] = B[k + ld * j[t][x]];
+            }
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+                acc[t][x >> 1][x & 1] =
+                    cadd(acc[t][x >> 1][x & 1], OP ? cmulc(a[x >> 1], b[x & 1]) : cmul_swapped(a[x >> 1], b[x & 1]));
+        }
+    if constexpr (OP == 0) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                c64 &v = acc[t][x >> 1][x & 1];
+                v = c64{alpha * v.re, alpha * v.im};
+                if (beta != 0.0) {
+                    const c64 c = C[r[t][x >> 1] + ld * j[t][x & 1]];
+                    v = c64{v.re + beta * c.re, v.im + beta * c.im};
+                }
+            }
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) out[r[t][x >> 1] + ld * j[t][x & 1]] = acc[t][x >> 1][x & 1];
+    wave_lds_sync();
 }
 
 // Parallel cyclic Jacobi on the n x n Hermitian M (LDS, column pitch ldm, n <= 32): the n/2 disjoint
-// rotations of a round-robin round are applied in parallel, one lane per (rotation, row) of M and Q, then one per
-// (rotation, column) of M, and accumulated into the n columns of Q (qrows x n, column pitch ldq, qrows <= 64). Stops
+// rotations of a round-robin round are applied in parallel and accumulated into the n columns of Q (qrows x n, column
+// pitch ldq, qrows <= 64). A wave works on G matrices, 64 / G lanes each (active: this lane's group has one). Each
+// rotation has its own lanes: all of them form it from M, which costs no more than one lane's forming it and needs no
+// table in LDS, then they share its rows of M and Q, then its columns of M. Stops
 // when the strict upper triangle's Frobenius norm (the part the rotations remove; rounding leaves M Hermitian only
 // to a few ulps, and unitary rotations cannot remove that anti-Hermitian residue) is <= tol/sqrt(2) x the
 // Frobenius norm, or after 12 sweeps. A pivot below 1e-20 of its diagonal scale is left alone: rotating it
 // would only shrink it further, towards the subnormal range where its phase can no longer be normalised
-// and the rotation stops being unitary. rot: 16 entries of LDS.
-__device__ void wave_jacobi(int n, c64 *M, int ldm, c64 *Q, int ldq, int qrows, JacobiRot *rot, int lane,
-                            double tol) {
+// and the rotation stops being unitary. The norms are summed in the order of one matrix a wave for any G.
+template <int G>
+__device__ void wave_jacobi(int n, c64 *M, int ldm, c64 *Q, int ldq, int qrows, int lane, double tol, bool active) {
+    constexpr int W = 64 / G, CH = 4;
+    const int l = lane & (W - 1);
     const int nn = n * n;
     const int N = n + (n & 1);
     const int npairs = N / 2;
+    const int L = W / npairs;  // lanes of a rotation
+    const int pair = l / L, sub = l - pair * L;
+    const SmallDiv byn(n);
     for (int sweep = 0; sweep < 12; sweep++) {
-        double off = 0.0, tot = 0.0;
-        for (int e = lane; e < nn; e += 64) {
-            const c64 me = M[e % n + ldm * (e / n)];
-            const double a2 = me.re * me.re + me.im * me.im;
-            tot += a2;
-            if (e % n < e / n) off += 2.0 * a2;
+        double off, tot;
+        {
+            double offs[G], tots[G];
+#pragma unroll
+            for (int v = 0; v < G; v++) {
+                offs[v] = tots[v] = 0.0;
+                for (int e = l + W * v; e < nn; e += 64) {
+                    const int c = byn.div(e), r = e - n * c;
+                    const c64 me = M[r + ldm * c];
+                    const double a2 = me.re * me.re + me.im * me.im;
+                    tots[v] += a2;
+                    if (r < c) offs[v] += 2.0 * a2;
+                }
+            }
+#pragma unroll
+            for (int h = G / 2; h >= 1; h >>= 1)
+#pragma unroll
+                for (int v = 0; v < h; v++) {
+                    offs[v] += offs[v + h];
+                    tots[v] += tots[v + h];
+                }
+            off = offs[0];
+            tot = tots[0];
         }
-        off = wave_sum(off);
-        tot = wave_sum(tot);
-        if (off <= tol * tol * tot) break;
+#pragma unroll
+        for (int x = W / 2; x >= 1; x >>= 1) {
+            off += __shfl_xor(off, x, 64);
+            tot += __shfl_xor(tot, x, 64);
+        }
+        if (off <= tol * tol * tot) active = false;
+        if (!__any(active)) break;
         for (int rd = 0; rd < N - 1; rd++) {
-            if (lane < npairs) {
-                int a, c;
-                if (lane == 0) {
-                    a = N - 1;
-                    c = rd;
-                } else {  // (rd + lane) and (rd - lane) modulo N - 1
-                    a = rd + lane;
-                    c = rd - lane;
-                    if (a >= N - 1) a -= N - 1;
-                    if (c < 0) c += N - 1;
+            int a, c;
+            if (pair == 0) {
+                a = N - 1;
+                c = rd;
+            } else {  // (rd + pair) and (rd - pair) modulo N - 1
+                a = rd + pair;
+                c = rd - pair;
+                if (a >= N - 1) a -= N - 1;
+                if (c < 0) c += N - 1;
+            }
+            const int p = min(a, c), q = max(a, c);
+            const bool rotates = active && pair < npairs && q < n;  // q == n: the dummy partner of an odd n
+            // G = diag(1, e^{-i phi}) [[cs, sn], [-sn, cs]] on (p, q); its upper row is real
+            c64 gpp{1.0, 0.0}, gpq{0.0, 0.0}, gqp{0.0, 0.0}, gqq{1.0, 0.0};
+            if (rotates) {
+                const c64 mpq = M[p + ldm * q];
+                const double mpp = M[p + ldm * p].re, mqq = M[q + ldm * q].re;
+                const double amp = hypot(mpq.re, mpq.im);
+                const double scale = fabs(mpp) + fabs(mqq);
+                if (amp > 1e-20 * scale && amp > 1e-280) {
+                    const double er = mpq.re / amp, ei = mpq.im / amp;
+                    const double tau = (mqq - mpp) / (2.0 * amp);
+                    const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+                    const double cs = 1.0 / sqrt(1.0 + t * t), sn = t * cs;
+                    gpp.re = cs;
+                    gpq.re = sn;
+                    gqp = c64{-sn * er, sn * ei};
+                    gqq = c64{cs * er, -cs * ei};
                 }
-                JacobiRot g;
-                g.p = min(a, c);
-                g.q = max(a, c);
-                g.cs = 1.0;
-                g.sn = 0.0;
-                g.gqp = c64{0.0, 0.0};
-                g.gqq = c64{1.0, 0.0};
-                if (g.q < n) {
-                    const c64 mpq = M[g.p + ldm * g.q];
-                    const double amp = hypot(mpq.re, mpq.im);
-                    const double scale = fabs(M[g.p + ldm * g.p].re) + fabs(M[g.q + ldm * g.q].re);
-                    if (amp > 1e-20 * scale && amp > 1e-280) {
-                        const double er = mpq.re / amp, ei = mpq.im / amp;
-                        const double tau = (M[g.q + ldm * g.q].re - M[g.p + ldm * g.p].re) / (2.0 * amp);
-                        const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-                        const double cs = 1.0 / sqrt(1.0 + t * t), sn = t * cs;
-                        g.cs = cs;
-                        g.sn = sn;
-                        g.gqp = c64{-sn * er, sn * ei};
-                        g.gqq = c64{cs * er, -cs * ei};
+            }
+            wave_lds_sync();
+            if (rotates) {  // M <- M G, Q <- Q G, CH rows at once
+                const int rows = n + qrows;
+                for (int i = sub; i < rows; i += CH * L) {
+                    c64 *xp[CH], *xq[CH], vp[CH], vq[CH];
+#pragma unroll
+                    for (int u = 0; u < CH; u++) {
+                        const int r = i + u * L < rows ? i + u * L : i;  // past the end: the first one's values again
+                        c64 *X = r < n ? M + r : Q + (r - n);
+                        const int ldx = r < n ? ldm : ldq;
+                        xp[u] = X + ldx * p;
+                        xq[u] = X + ldx * q;
+                        vp[u] = *xp[u];
+                        vq[u] = *xq[u];
                     }
-                } else {
-                    g.q = g.p;  // dummy partner of an odd n: identity on a single index
+#pragma unroll
+                    for (int u = 0; u < CH; u++) {
+                        *xp[u] = cadd(cmul(vp[u], gpp), cmul(vq[u], gqp));
+                        *xq[u] = cadd(cmul(vp[u], gpq), cmul(vq[u], gqq));
+                    }
                 }
-                rot[lane] = g;
             }
             wave_lds_sync();
-            // M <- M G, Q <- Q G
-            for (int e = lane; e < npairs * n; e += 64) {
-                const int k = e / n, r = e - k * n;
-                const JacobiRot g = rot[k];
-                if (g.p == g.q) continue;
-                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
-                const c64 mp = M[r + ldm * g.p], mq = M[r + ldm * g.q];
-                M[r + ldm * g.p] = cadd(cmul(mp, gpp), cmul(mq, g.gqp));
-                M[r + ldm * g.q] = cadd(cmul(mp, gpq), cmul(mq, g.gqq));
-            }
-            for (int e = lane; e < npairs * qrows; e += 64) {
-                const int k = e / qrows, r = e - k * qrows;
-                const JacobiRot g = rot[k];
-                if (g.p == g.q) continue;
-                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
-                const c64 qp = Q[r + ldq * g.p], qq = Q[r + ldq * g.q];
-                Q[r + ldq * g.p] = cadd(cmul(qp, gpp), cmul(qq, g.gqp));
-                Q[r + ldq * g.q] = cadd(cmul(qp, gpq), cmul(qq, g.gqq));
-            }
-            wave_lds_sync();
-            // M <- G^H M
-            for (int e = lane; e < npairs * n; e += 64) {
-                const int k = e / n, c = e - k * n;
-                const JacobiRot g = rot[k];
-                if (g.p == g.q) continue;
-                const c64 gpp{g.cs, 0.0}, gpq{g.sn, 0.0};
-                const c64 mp = M[g.p + ldm * c], mq = M[g.q + ldm * c];
-                M[g.p + ldm * c] = cadd(cmulc(gpp, mp), cmulc(g.gqp, mq));
-                M[g.q + ldm * c] = cadd(cmulc(gpq, mp), cmulc(g.gqq, mq));
+            if (rotates) {  // M <- G^H M
+                for (int i = sub; i < n; i += CH * L) {
+                    c64 *xp[CH], *xq[CH], vp[CH], vq[CH];
+#pragma unroll
+                    for (int u = 0; u < CH; u++) {
+                        const int col = i + u * L < n ? i + u * L : i;
+                        xp[u] = M + p + ldm * col;
+                        xq[u] = M + q + ldm * col;
+                        vp[u] = *xp[u];
+                        vq[u] = *xq[u];
+                    }
+#pragma unroll
+                    for (int u = 0; u < CH; u++) {
+                        *xp[u] = cadd(cmulc(gpp, vp[u]), cmulc(gqp, vq[u]));
+                        *xq[u] = cadd(cmulc(gpq, vp[u]), cmulc(gqq, vq[u]));
+                    }
+                }
             }
             wave_lds_sync();
         }
     }
 }
 
-__global__ __launch_bounds__(256) void heev_refine_kernel(int n, int64_t nb, const c64 *__restrict__ H,
+template <int G, int NT>
+__global__ __launch_bounds__(256) void heev_refine_kernel(int n, int64_t nb, const c64u *__restrict__ H,
                                                           c32 *__restrict__ U, double *__restrict__ E64,
                                                           double tol) {
     extern __shared__ double lds64[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t b = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave;
-    if (b >= nb) return;
+    constexpr int W = 64 / G;
+    const int lane = threadIdx.x & 63, l = lane & (W - 1);
+    const int64_t slot = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / W;
     const int nn = n * n, ld = refine_ld(n), nl = n * ld;
-    c64 *Q = reinterpret_cast<c64 *>(lds64 + (int64_t)wave * refine_lds_doubles(n));
-    c64 *W = Q + nl;
-    c64 *M = W + nl;
-    JacobiRot *rot = reinterpret_cast<JacobiRot *>(M + nl);  // 16 x 56 bytes
-    int *rank_s = reinterpret_cast<int *>(rot + 16);           // n ints
-    for (int e = lane; e < nn; e += 64) {
-        const int i = e % n, j = e / n;
+    const bool active = slot < nb;
+    if (!__any(active)) return;
+    const int64_t b = active ? slot : nb - 1;  // lanes without a matrix compute along on the last one, and write nothing
+    const SmallDiv byn(n);
+    c64 *Q = reinterpret_cast<c64 *>(lds64) + (threadIdx.x / W) * 2 * nl;
+    c64 *M = Q + nl;
+    for (int e = l; e < nn; e += W) {
+        const int j = byn.div(e), i = e - n * j;
         const c32 u = U[b * nn + e];
         Q[i + ld * j] = c64{u.re, u.im};
     }
     wave_lds_sync();
-    // 1. two Loewdin steps: S = Q^H Q (in W), M = 3/2 Q - 1/2 Q S, which is the next Q
+    // 1. two Loewdin steps: M = Q^H Q, Q = 3/2 Q - 1/2 Q M
     for (int it = 0; it < 2; it++) {
-        lds_gemm<1>(n, ld, Q, Q, W, 0.0, 0.0, nullptr, lane);
-        wave_lds_sync();
-        lds_gemm<0>(n, ld, Q, W, M, -0.5, 1.5, Q, lane);
-        wave_lds_sync();
-        c64 *x = Q;
-        Q = M;
-        M = x;
+        lds_gemm<1, NT, W>(n, ld, Q, Q, M, 0.0, 0.0, nullptr, l);
+        lds_gemm<0, NT, W>(n, ld, Q, M, Q, -0.5, 1.5, Q, l);
     }
     // 2. M = Q^H (H Q), H where M goes
-    for (int e = lane; e < nn; e += 64) {
-        const int i = e % n, j = e / n;
-        c64 h = (i <= j) ? H[b * nn + i + (int64_t)n * j] : H[b * nn + j + (int64_t)n * i];
+    for (int e = l; e < nn; e += W) {
+        const int j = byn.div(e), i = e - n * j;
+        const c64u hu = (i <= j) ? H[b * nn + i + (int64_t)n * j] : H[b * nn + j + (int64_t)n * i];
+        c64 h{hu.re, hu.im};
         if (i > j) h.im = -h.im;
         if (i == j) h.im = 0.0;
         M[i + ld * j] = h;
     }
     wave_lds_sync();
-    lds_gemm<0>(n, ld, M, Q, W, 1.0, 0.0, nullptr, lane);
-    wave_lds_sync();
-    lds_gemm<1>(n, ld, Q, W, M, 0.0, 0.0, nullptr, lane);
-    wave_lds_sync();
+    lds_gemm<0, NT, W>(n, ld, M, Q, M, 1.0, 0.0, nullptr, l);
+    lds_gemm<1, NT, W>(n, ld, Q, M, M, 0.0, 0.0, nullptr, l);
     // 3. parallel cyclic Jacobi
-    wave_jacobi(n, M, ld, Q, ld, n, rot, lane, tol);
-    // 4. ascending order
-    double d = 0.0;
-    if (lane < n) d = M[lane + ld * lane].re;
-    int rank = 0;
-    for (int k = 0; k < n; k++) {
-        const double dk = rdl64(d, k);
-        rank += (dk < d || (dk == d && k < lane)) ? 1 : 0;
-    }
-    if (lane < n) {
+    wave_jacobi<G>(n, M, ld, Q, ld, n, lane, tol, active);
+    if (!active) return;
+    // 4. ascending order; the rank of a column goes beside its eigenvalue
+    if (l < n) {
+        const double d = M[l + ld * l].re;
+        int rank = 0;
+        for (int k = 0; k < n; k++) {
+            const double dk = M[k + ld * k].re;
+            rank += (dk < d || (dk == d && k < l)) ? 1 : 0;
+        }
         E64[b * n + rank] = d;
-        rank_s[lane] = rank;
+        M[l + ld * l].im = rank;
     }
     wave_lds_sync();
-    for (int e = lane; e < nn; e += 64) {
-        const int r = e % n, j = e / n;
-        const c64 q = Q[r + ld * j];
-        U[b * nn + r + (int64_t)n * rank_s[j]] = c32{static_cast<float>(q.re), static_cast<float>(q.im)};
+    for (int e = l; e < nn; e += W) {
+        const int j = byn.div(e), r = e - n * j;
+        const c64 v = Q[r + ld * j];
+        U[b * nn + r + (int64_t)n * (int)M[j + ld * j].im] = c32{static_cast<float>(v.re), static_cast<float>(v.im)};
     }
 }
 
@@ -508,16 +562,16 @@ __global__ __launch_bounds__(256) void heev_refine_kernel(int n, int64_t nb, con
 // the columns in ascending order of M's eigenvalues. The gauge inside each group is then fixed by H and P
 // alone (up to one phase per column), whatever gauge the solver returned. Matrices without a pair closer
 // than the cutoff are not touched. LDS (one wave per workgroup): U_g | W = P U_g | M (n*n c64 each),
-// rotation table, ranks.
+// ranks.
 // ---------------------------------------------------------------------------------------------
-__host__ __device__ constexpr int gauge_lds_bytes(int n) { return 3 * n * n * 16 + 16 * (int)sizeof(JacobiRot) + 4 * n; }
+__host__ __device__ constexpr int gauge_lds_bytes(int n) { return 3 * n * n * 16 + 4 * n; }
 
 __device__ __forceinline__ c64 degeneracy_perturbation(int r, int c) {  // P[r, c], 0-based row r, column c
     return c64{0.25644832 + 0.005 * (double)(r + c + 2), 0.0125 * (double)(r - c)};
 }
 
 __device__ void gauge_fix_group(int n, int a, int m, c32 *__restrict__ Ub, c64 *Ug, c64 *W, c64 *M,
-                                JacobiRot *rot, int *rank_s, int lane) {
+                                int *rank_s, int lane) {
     for (int t = lane; t < n * m; t += 64) {
         const c32 u = Ub[t % n + n * (a + t / n)];
         Ug[t] = c64{u.re, u.im};
@@ -526,7 +580,7 @@ __device__ void gauge_fix_group(int n, int a, int m, c32 *__restrict__ Ub, c64 *
     for (int t = lane; t < n * m; t += 64) {  // W = P U_g
         const int r = t % n, c = t / n;
         c64 acc{0.0, 0.0};
-        for (int k = 0; k < n; k++) acc = cadd(acc, cmul(degeneracy_perturbation(r, k), Ug[k + n * c]));
+        for (int k = 0; k < n; k++) acc = cadd(acc, cmul_swapped(degeneracy_perturbation(r, k), Ug[k + n * c]));
         W[t] = acc;
     }
     wave_lds_sync();
@@ -540,7 +594,7 @@ __device__ void gauge_fix_group(int n, int a, int m, c32 *__restrict__ Ub, c64 *
         M[j + m * i] = c64{acc.re, -acc.im};
     }
     wave_lds_sync();
-    wave_jacobi(m, M, m, Ug, n, n, rot, lane, 1e-15);
+    wave_jacobi<1>(m, M, m, Ug, n, n, lane, 1e-15, true);
     const double d = lane < m ? M[lane + m * lane].re : 0.0;
     int rank = 0;
     for (int k = 0; k < m; k++) {
@@ -568,8 +622,7 @@ __global__ __launch_bounds__(64) void degenerate_gauge_kernel(int n, int64_t nb,
     c64 *Ug = reinterpret_cast<c64 *>(lds64);
     c64 *W = Ug + n * n;
     c64 *M = W + n * n;
-    JacobiRot *rot = reinterpret_cast<JacobiRot *>(M + n * n);
-    int *rank_s = reinterpret_cast<int *>(rot + 16);
+    int *rank_s = reinterpret_cast<int *>(M + n * n);
     c32 *Ub = U + b * n * n;
     double first = rdl64(e, 0);
     int a = 0;
@@ -582,7 +635,7 @@ __global__ __launch_bounds__(64) void degenerate_gauge_kernel(int n, int64_t nb,
             last = i + 1;
         else
             continue;
-        if (last > a) gauge_fix_group(n, a, last - a + 1, Ub, Ug, W, M, rot, rank_s, lane);
+        if (last > a) gauge_fix_group(n, a, last - a + 1, Ub, Ug, W, M, rank_s, lane);
         first = next;
         a = i + 1;
     }
@@ -609,6 +662,14 @@ static int refine_waves_per_block(size_t lds_per_wave) {
     return best;
 }
 
+template <int G, int NT>
+static void refine_launch(int n, int64_t nb, const void *H64, void *U, double *E64, double tol, void *stream) {
+    const size_t lds_wave = G * sizeof(double) * refine_lds_doubles(n);
+    const int wpb = refine_waves_per_block(lds_wave);
+    heev_refine_kernel<G, NT><<<(unsigned)((nb + G * wpb - 1) / (G * wpb)), 64 * wpb, wpb * lds_wave, as_stream(stream)>>>(
+        n, nb, static_cast<const c64u *>(H64), static_cast<c32 *>(U), E64, tol);
+}
+
 static int heev_launch_check(int n, int64_t nb) {
     EPHIP_REQUIRE(n >= 1 && n <= 32, "heev: n=%d outside 1..32 (one wavefront per matrix)", n);
     EPHIP_REQUIRE(nb >= 0, "heev: negative batch");
@@ -627,7 +688,7 @@ extern "C" int ephip_heev_c32(int32_t n, int64_t nb, const void *H, int32_t h_is
     const unsigned grid = (unsigned)((nb + wpb - 1) / wpb);
     hipStream_t s = as_stream(stream);
     if (h_is_c64)
-        heev_c32_kernel<c64><<<grid, 64 * wpb, lds, s>>>(n, nb, static_cast<const c64 *>(H), static_cast<c32 *>(U), E, info);
+        heev_c32_kernel<c64u><<<grid, 64 * wpb, lds, s>>>(n, nb, static_cast<const c64u *>(H), static_cast<c32 *>(U), E, info);
     else
         heev_c32_kernel<c32><<<grid, 64 * wpb, lds, s>>>(n, nb, static_cast<const c32 *>(H), static_cast<c32 *>(U), E, info);
     EPHIP_LAUNCHED();
@@ -642,15 +703,20 @@ extern "C" int ephip_heev_refine(int32_t n, int64_t nb, const void *H64, void *U
     EPHIP_REQUIRE(H64 && U && E64, "heev_refine: null device pointer");
     EPHIP_REQUIRE(tol >= 0.0, "heev_refine: negative tolerance");
     (void)E32;
-    const int wpb = refine_waves_per_block(sizeof(double) * refine_lds_doubles(n));
-    const size_t lds = wpb * sizeof(double) * refine_lds_doubles(n);
-    if (lds > 64 * 1024) {  // n = 32: one matrix's FP64 working set in a one-wave block; gfx950 has
-                            // 160 KiB of LDS per workgroup
-        EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(heev_refine_kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    }
-    heev_refine_kernel<<<(unsigned)((nb + wpb - 1) / wpb), 64 * wpb, lds, as_stream(stream)>>>(
-        n, nb, static_cast<const c64 *>(H64), static_cast<c32 *>(U), E64, tol > 0.0 ? tol : 1e-15);
+    const double t = tol > 0.0 ? tol : 1e-15;
+    // Matrices a wave. Two share the forming of the rotations, which every lane of a wave waits for: 27000 of n = 16 in
+    // 744 us for 1137, 13824 of n = 12 in 271 for 463. While one a wave leaves SIMDs idle (a matrix each, 256 CUs), it
+    // is the quicker: 500 of n = 16 in 58 us for 72. Four up to n = 8, where they still fill the lanes, win from the
+    // smallest batch on: 500 of n = 8 in 29 us for 30, 30000 in 139 for 292 (two) and 595 (one). Above n = 16 the LDS
+    // holds too few matrices to pair them.
+    if (n > 16)
+        refine_launch<1, 4>(n, nb, H64, U, E64, t, stream);
+    else if (n <= 8)
+        refine_launch<4, 1>(n, nb, H64, U, E64, t, stream);
+    else if (nb > 1024)
+        refine_launch<2, 2>(n, nb, H64, U, E64, t, stream);
+    else
+        refine_launch<1, 1>(n, nb, H64, U, E64, t, stream);
     EPHIP_LAUNCHED();
     return EPHIP_OK;
 }
