@@ -13,10 +13,12 @@
 // used here were checked on gfx950: f32 16x16x4 and bf16 16x16x32 return C[4(l/16)+r][l%16] in
 // lane l, register r; f64 16x16x4 returns C[4r+l/16][l%16].
 //
-// Tiles: 256 threads = 4 waves in a 2 x 2 arrangement; a workgroup owns TM = 64 complex rows and
-// TN columns; K advances KC = 16 complex R per LDS stage. FP32 and FP64 use the 16x16x4 MFMA
+// Tiles (ft64_kernel has its own): 256 threads = 4 waves in a 2 x 2 arrangement; a workgroup owns
+// TM = 64 complex rows and TN columns; K advances KC = 16 complex R per LDS stage. FP32 and FP64 use the 16x16x4 MFMA
 // (lane l holds A[l%16][l/16], B[l/16][l%16]); the split-BF16 form uses
 // 16x16x32 bf16 MFMAs with hi/lo operand splitting and three products per real product.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace ephip {
@@ -131,17 +133,17 @@ struct FtBatch {
     const int *ncol = nullptr;
 };
 
-template <class T, int TN>
-__global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, const cplx<T> *__restrict__ op,
+template <int TN>
+__global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, const cplx<float> *__restrict__ op,
                                                       int64_t ldop, const int *__restrict__ irvec, int nk,
-                                                      const double *__restrict__ xk, cplx<T> *__restrict__ out,
+                                                      const double *__restrict__ xk, cplx<float> *__restrict__ out,
                                                       int64_t ldout, FtBatch bt) {
-    using acc_t = typename std::conditional<sizeof(T) == 4, f32x4, f64x4>::type;
+    using T = float;
+    using acc_t = f32x4;
     constexpr int NCB = TN / 32;  // 16-column blocks per wave
     __shared__ cplx<T> As[FT_KC][FT_TM + FT_APAD];
     __shared__ T Bs[FT_KC][2][TN + FT_BPAD];
-    constexpr bool kSep = sizeof(T) == 4;  // separable phases for FP32 (FP64 keeps direct sincos)
-    __shared__ float2 tab[kSep ? FT_TAB_MAX : 1][kSep ? TN : 1];
+    __shared__ float2 tab[FT_TAB_MAX][TN];
     __shared__ int red[24];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -156,15 +158,11 @@ __global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, con
         out += u * bt.out_stride;
         if (bt.col_index) bt.col_index += u * bt.col_stride;
     }
-    bool use_tab = false;
-    FtAxes ax{};
-    if constexpr (kSep) {
-        ax = ft_axes(irvec, nr, red);
-        use_tab = ax.total <= FT_TAB_MAX;
-        if (use_tab) {
-            ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
-            __syncthreads();  // a column's rows are written by 256 / TN waves and read by each of them
-        }
+    const FtAxes ax = ft_axes(irvec, nr, red);
+    const bool use_tab = ax.total <= FT_TAB_MAX;
+    if (use_tab) {
+        ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+        __syncthreads();  // a column's rows are written by 256 / TN waves and read by each of them
     }
 
     // The phase column this thread generates is fixed for the whole kernel; its R rows are uniform
@@ -219,11 +217,6 @@ __global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, con
             }
         }
         __syncthreads();
-        // The f32 MFMA returns row 4(l/16)+r of the 16x16 block in lane l, register r; the f64 MFMA
-        // returns row 4r + l/16. Feeding the f64 A operand with rows permuted by
-        // i -> 4(i%4) + i/4 makes both land in the same (lane, register) slots.
-        const int il = lane & 15;
-        const int irow = (sizeof(T) == 8) ? (4 * (il & 3) + (il >> 2)) : il;
 #pragma unroll
         for (int ks = 0; ks < FT_KC / 2; ks++) {
             const int kk = lane >> 4;
@@ -232,7 +225,7 @@ __global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, con
             T a[4], b[NCB];
 #pragma unroll
             for (int rb = 0; rb < 4; rb++) {
-                const int rr = wm * 64 + 16 * rb + irow;
+                const int rr = wm * 64 + 16 * rb + (lane & 15);
                 const cplx<T> v = As[rl][rr >> 1];
                 a[rb] = (rr & 1) == 0 ? (cc == 0 ? v.re : -v.im) : (cc == 0 ? v.im : v.re);
             }
@@ -258,6 +251,197 @@ __global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, con
                 if (d + 1 < ndata) out[d + 1 + ldout * j] = cplx<T>{acc[rb][cb][2], acc[rb][cb][3]};
             }
         }
+}
+
+// FP64 form. WR x WC waves of a workgroup own 8 RB WR complex rows and 16 CB WC columns, 16 RB real rows and 16 CB columns
+// each; an entry's sum runs over R in order, 2 R an MFMA, whatever the tile. Two LDS stages of KC complex R: the next
+// one is filled while the MFMAs of this one run, by FT64_FILL waves that do nothing else: the sincos keeps its constants
+// in the registers that hold the others' sums (one role for all waves spilled, or left room for a quarter of the tile).
+// Bound by the FP64 units, which the MFMAs and the phases share. 256 rows x 729 R x 32768 columns: 0.95 ms (51 TFLOP/s)
+// for 1.25 before, when each 64 rows formed the phases anew; without any phases 0.88, without filling 0.75.
+// 64 rows x 125 R x 505 columns: 9.6 us for 45, in 64 workgroups and 4 stages for 8 and 8.
+constexpr int FT64_FILL = 4;
+__host__ __device__ constexpr int ft64_apitch(int tm) { return tm + 8; }    // complex: the next R half a bank row on
+__host__ __device__ constexpr int ft64_bpitch(int tn) { return tn + 16; }   // doubles, likewise re and im
+__host__ __device__ constexpr size_t ft64_stage_doubles(int kc, int tm, int tn) {
+    return (size_t)kc * 2 * (ft64_apitch(tm) + ft64_bpitch(tn));
+}
+
+template <int RB, int CB, int KC, int AE>
+__global__ __launch_bounds__(1024) void ft64_kernel(int64_t ndata, int nr, const cplx<double> *__restrict__ op,
+                                                    int64_t ldop, const int *__restrict__ irvec, int nk,
+                                                    const double *__restrict__ xk, cplx<double> *__restrict__ out,
+                                                    int64_t ldout, int WR, int WC) {
+    extern __shared__ double ft64_lds[];
+    const int TM = 8 * RB * WR, TN = 16 * CB * WC;  // TN is a power of two, at most 64
+    const int PA = ft64_apitch(TM), PB = ft64_bpitch(TN);
+    const size_t stage = ft64_stage_doubles(KC, TM, TN);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t d0 = (int64_t)blockIdx.y * TM;
+    const int j0 = blockIdx.x * TN;
+    constexpr int NW = FT64_FILL;
+
+    // operand: items of 64 rows of one R, phases: items of 64 (R, column) pairs; a thread's column is fixed
+    const int nitem = KC * ((TM + 63) / 64), npitem = KC * TN / 64;
+    const int pj = lane & (TN - 1), psub = lane / TN, pper = 64 / TN;
+    const bool pvalid = j0 + pj < nk;
+    double x0 = 0, x1 = 0, x2 = 0;
+    cplx<double> areg[AE];
+    auto load_a = [&](int r0) {
+#pragma unroll
+        for (int i = 0; i < AE; i++) {
+            const int it = wave + NW * i, r = r0 + it % KC, dl = it / KC * 64 + lane;
+            areg[i] = (it < nitem && dl < TM && d0 + dl < ndata && r < nr) ? op[d0 + dl + ldop * r]
+                                                                            : cplx<double>{0, 0};
+        }
+    };
+    auto stash_a = [&](double *st) {
+        cplx<double> *A = reinterpret_cast<cplx<double> *>(st);
+#pragma unroll
+        for (int i = 0; i < AE; i++) {
+            const int it = wave + NW * i, dl = it / KC * 64 + lane;
+            if (it < nitem && dl < TM) A[it % KC * PA + dl] = areg[i];
+        }
+    };
+    auto phases = [&](int r0, double *st) {
+        double *B = st + 2 * KC * PA;
+        for (int it = wave; it < npitem; it += NW) {
+            const int rl = it * pper + psub, r = r0 + rl;
+            double c = 0, s = 0;
+            if (pvalid && r < nr) {
+                const double t = irvec[3 * r] * x0 + irvec[3 * r + 1] * x1 + irvec[3 * r + 2] * x2;
+                cis2pi(t, c, s);
+            }
+            B[2 * rl * PB + pj] = c;
+            B[(2 * rl + 1) * PB + pj] = s;
+        }
+    };
+    if (wave < NW) {
+        if (pvalid) {
+            x0 = xk[3 * (int64_t)(j0 + pj)];
+            x1 = xk[3 * (int64_t)(j0 + pj) + 1];
+            x2 = xk[3 * (int64_t)(j0 + pj) + 2];
+        }
+        load_a(0);
+        phases(0, ft64_lds);
+        stash_a(ft64_lds);
+        for (int r0 = KC, b = 1; r0 < nr; r0 += KC, b ^= 1) {
+            __syncthreads();
+            load_a(r0);
+            phases(r0, ft64_lds + b * stage);
+            stash_a(ft64_lds + b * stage);
+        }
+        __syncthreads();  // as many as the other waves meet, one a stage
+        return;
+    }
+    const int cw = wave - NW, wm = cw % WR, wn = cw / WR;
+
+    f64x4 acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < CB; j++) acc[i][j] = f64x4{0, 0, 0, 0};
+
+    // The MFMA returns row 4r + l/16 in lane l, register r; rows fed permuted by i -> 4(i%4) + i/4 come back with a
+    // complex number's parts in adjacent registers. Lane l holds k = l/16: R rl = 2 ks + k/2, the phase's part k%2.
+    const int il = lane & 15, kk = lane >> 4, cc = kk & 1;
+    const int irow = 4 * (il & 3) + (il >> 2);
+    const int part = cc ^ (irow & 1);                       // part of the operand: re * re - im * im, re * im + im * re
+    const unsigned flip = (cc && !(irow & 1)) ? 0x80000000u : 0u;
+    const int aoff = 2 * ((kk >> 1) * PA + (wm * 16 * RB + irow) / 2) + part;
+    const int boff = 2 * KC * PA + (2 * (kk >> 1) + cc) * PB + wn * 16 * CB + il;
+    for (int r0 = 0, b = 0; r0 < nr; r0 += KC, b ^= 1) {
+        __syncthreads();  // this stage is filled, and the other one read
+        const double *cur = ft64_lds + b * stage;
+#pragma unroll
+        for (int ks = 0; ks < KC / 2; ks++) {
+            double av[RB], bv[CB];
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+                const double v = cur[aoff + 4 * ks * PA + 16 * rb];
+                av[rb] = __hiloint2double(__double2hiint(v) ^ flip, __double2loint(v));
+            }
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) bv[cb] = cur[boff + 4 * ks * PB + 16 * cb];
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++)
+                    acc[rb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[rb], bv[cb], acc[rb][cb], 0, 0, 0);
+        }
+    }
+
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++) {
+            const int64_t d = d0 + wm * 8 * RB + 8 * rb + 2 * kk;
+            const int64_t j = j0 + wn * 16 * CB + 16 * cb + il;
+            if (j < nk) {
+                if (d < ndata) out[d + ldout * j] = cplx<double>{acc[rb][cb][0], acc[rb][cb][1]};
+                if (d + 1 < ndata) out[d + 1 + ldout * j] = cplx<double>{acc[rb][cb][2], acc[rb][cb][3]};
+            }
+        }
+}
+
+template <int RB, int CB, int KC, int AE>
+static int launch_ft64(int WR, int WC, int64_t ndata, int nr, const cplx<double> *op, int64_t ldop, const int *irvec,
+                       int nk, const double *xk, cplx<double> *out, int64_t ldout, hipStream_t s) {
+    const int TM = 8 * RB * WR, TN = 16 * CB * WC;
+    const size_t lds = 2 * sizeof(double) * ft64_stage_doubles(KC, TM, TN);
+    const int64_t gy = (ndata + TM - 1) / TM;
+    EPHIP_REQUIRE(FT64_FILL + WR * WC <= 16 && TN <= 64 && KC * ((TM + 63) / 64) <= AE * FT64_FILL && lds <= 160 * 1024,
+                  "fourier_c64: no workgroup of %d x %d waves", WR, WC);
+    if (lds > 64 * 1024)
+        EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ft64_kernel<RB, CB, KC, AE>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const dim3 g((unsigned)((nk + TN - 1) / TN), (unsigned)gy);
+    ft64_kernel<RB, CB, KC, AE><<<g, 64 * (FT64_FILL + WR * WC), lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out,
+                                                                           ldout, WR, WC);
+    return EPHIP_OK;
+}
+
+// The tile: the cheapest by an estimate in cycles of one SIMD, from three wave tiles (32 x 32 with stages of 8 R where
+// the MFMAs bound it, 16 x 16 with 16 and 8 x 16 with 32 where few columns or rows leave SIMDs idle or the latency of a
+// stage counts) and two widths. A workgroup's waves (4 that fill and up to 12) and its LDS say how many share a CU,
+// the grid how often the chip is filled; a stage costs its MFMAs (70 cycles each) beside its phases (800 cycles a wave
+// of 64; both use the FP64 units, so they overlap in part) and 750 to 1500 cycles of latency. Of the tiles measured on
+// 28 shapes (1 to 1024 rows, 27 to 729 R, 27 to 110592 columns) it names the quickest or one within 3% of it.
+struct Ft64Tile {
+    int form, wr, wc;
+    double cost;
+};
+
+static Ft64Tile ft64_tile(int64_t ndata, int nr, int nk) {
+    static const int forms[3][3] = {{4, 2, 8}, {2, 1, 16}, {1, 1, 32}};  // RB, CB, KC
+    static const int splits[3][2] = {{1, 8}, {2, 6}, {1, 4}};            // column waves, most row waves
+    Ft64Tile best{-1, 0, 0, 0.0};
+    for (int f = 0; f < 3; f++)
+        for (auto &sp : splits) {
+            const int rows = 8 * forms[f][0], kc = forms[f][2], wc = sp[0];
+            const int64_t n = (ndata + rows - 1) / rows, tiles = (n + sp[1] - 1) / sp[1];
+            const int wr = (int)((n + tiles - 1) / tiles), waves = wr * wc;
+            const int tm = rows * wr, tn = 16 * forms[f][1] * wc;
+            if ((ndata + tm - 1) / tm > 65535) continue;
+            const int64_t lds = 2 * 8 * (int64_t)ft64_stage_doubles(kc, tm, tn);
+            const int64_t most = std::max<int64_t>(1, std::min<int64_t>(16 / (4 + waves), 160 * 1024 / lds));
+            const int64_t wgs = ((int64_t)nk + tn - 1) / tn * ((ndata + tm - 1) / tm);
+            const int64_t share = std::min(most, (wgs + 255) / 256), rounds = (wgs + 256 * share - 1) / (256 * share);
+            const double mfma = (double)((waves * share + 3) / 4) * forms[f][0] * forms[f][1] * (kc / 2) * 70.0;
+            const double phase = (double)share * kc * tn / 256 * 800.0;
+            const double stage = std::max(mfma + 0.6 * phase, phase + 750.0) + 750.0;
+            const double cost = (double)rounds * (((nr + kc - 1) / kc) * stage + 4000.0);
+            if (best.form < 0 || cost < best.cost) best = Ft64Tile{f, wr, wc, cost};
+        }
+    return best;
+}
+
+static int ft64_run(int64_t ndata, int nr, const cplx<double> *op, int64_t ldop, const int *irvec, int nk,
+                    const double *xk, cplx<double> *out, int64_t ldout, hipStream_t s) {
+    const Ft64Tile t = ft64_tile(ndata, nr, nk);
+    if (t.form == 0) return launch_ft64<4, 2, 8, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
+    if (t.form == 1) return launch_ft64<2, 1, 16, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
+    return launch_ft64<1, 1, 32, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
 }
 
 // Double-buffered form of ft_mfma_kernel: two LDS stages; the next stage's operand loads are issued
@@ -347,7 +531,10 @@ __global__ __launch_bounds__(256) void ft_mfma_db_kernel(int64_t ndata, int nr, 
     __syncthreads();
 
     const int il = lane & 15;
-    const int irow = (sizeof(T) == 8) ? (4 * (il & 3) + (il >> 2)) : il;  // see ft_mfma_kernel
+    // The f32 MFMA returns row 4(l/16)+r of the 16x16 block in lane l, register r; the f64 MFMA
+    // returns row 4r + l/16. Feeding the f64 A operand with rows permuted by
+    // i -> 4(i%4) + i/4 makes both land in the same (lane, register) slots.
+    const int irow = (sizeof(T) == 8) ? (4 * (il & 3) + (il >> 2)) : il;
     const int nchunks = (nr + KC - 1) / KC;
     for (int ch = 0; ch < nchunks; ch++) {
         const int buf = ch & 1;
@@ -393,7 +580,7 @@ __global__ __launch_bounds__(256) void ft_mfma_db_kernel(int64_t ndata, int nr, 
 }
 
 // Kernel variant per contraction kind, set by the tuner (ephip_ft_set_variant). Kinds:
-// 0 = FP32 wide (nk > 64), 1 = FP32 narrow (nk <= 64), 2 = FP64. Variants: 0 = single-buffered,
+// 0 = FP32 wide (nk > 64), 1 = FP32 narrow (nk <= 64), 2 = FP64. Variants: 0 = single-buffered (FP64: ft64_kernel),
 // 1 = double-buffered KC 16, 2 = double-buffered KC 8.
 static int g_ft_variant[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 
@@ -404,8 +591,8 @@ static void launch_ft(int variant, dim3 g, hipStream_t s, int64_t ndata, int nr,
         ft_mfma_db_kernel<T, TN, 16><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
     else if (variant == 2)
         ft_mfma_db_kernel<T, TN, 8><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
-    else
-        ft_mfma_kernel<T, TN><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
+    else if constexpr (sizeof(T) == 4)
+        ft_mfma_kernel<TN><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1810,9 +1997,15 @@ extern "C" int ephip_fourier_c64(int64_t ndata, int32_t nr, const void *op, int6
     if (ndata == 0 || nk == 0) return EPHIP_OK;
     hipStream_t s = as_stream(stream);
     if (nr == 0) return zero_out<double>(ndata, nk, out, ldout, s);
-    dim3 g((nk + 63) / 64, (unsigned)((ndata + FT_TM - 1) / FT_TM));
-    launch_ft<double, 64>(g_ft_variant[2], g, s, ndata, nr, static_cast<const cplx<double> *>(op), ldop, irvec, nk,
-                          xk, static_cast<cplx<double> *>(out), ldout, FtBatch{});
+    auto o = static_cast<const cplx<double> *>(op);
+    auto c = static_cast<cplx<double> *>(out);
+    if (g_ft_variant[2] == 0) {
+        st = ft64_run(ndata, nr, o, ldop, irvec, nk, xk, c, ldout, s);
+        if (st) return st;
+    } else {
+        dim3 g((nk + 63) / 64, (unsigned)((ndata + FT_TM - 1) / FT_TM));
+        launch_ft<double, 64>(g_ft_variant[2], g, s, ndata, nr, o, ldop, irvec, nk, xk, c, ldout, FtBatch{});
+    }
     EPHIP_LAUNCHED();
     return EPHIP_OK;
 }
