@@ -1,4 +1,4 @@
-"""Several matrices a wave in the FP64 refinement: one, two or four by n and the batch."""
+"""Several matrices a wave in the FP32 eigensolve (by n) and the FP64 refinement (by n and the batch)."""
 import numpy as np
 import pytest
 
@@ -45,3 +45,23 @@ def test_refine_partial_waves(backend, n, nb):
         assert np.abs(E[b] - w).max() < 1e-13 * max(np.abs(w).max(), 1.0)
         V = U[b].T.astype(np.complex128)
         assert np.abs(h[b] @ V - V * E[b]).max() < 1e-6 * max(np.abs(w).max(), 1.0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 16, 17, 32])
+def test_heev_mixed_matrices_in_a_wave(backend, n):
+    """Matrices that take different ways through the QL iteration side by side in a wave (dense, decoupled, diagonal,
+    zero, and scaled so that squares leave the range in which hypot and the quotients need no scaling): each gives the
+    bits that it gives alone."""
+    import torch
+    from ephip import core
+    h = _batch(n, 45, 70 + n)
+    h[2::9] *= 2.0 ** -70
+    h[4::9] *= 2.0 ** 55
+    h[6::9] = 0
+    h[7::9] = np.eye(n) * np.arange(n)
+    hc = torch.from_numpy(np.ascontiguousarray(np.transpose(h, (0, 2, 1)).astype(np.complex64))).cuda()
+    E, U = core.eigen_batched(hc)
+    assert torch.equal(E, core.eigvals_batched(hc))
+    for b in range(45):
+        Eb, Ub = core.eigen_batched(hc[b:b + 1].contiguous())
+        assert torch.equal(Eb[0], E[b]) and torch.equal(Ub[0], U[b])
