@@ -73,6 +73,7 @@ SIGNATURES = {
     "ephip_eph_window_scatter": [_i32, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _i32, _i32, _i32,
                                  _i64, _i64, _i64, _vp, _vp],
     "ephip_bte_spmv": [_i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+    "ephip_bte_step": [_i64, _vp, _vp, _vp, C.c_double, _vp, _vp, C.c_double, _vp, _vp, _vp, _vp],
     "ephip_mlp_bf16_prune": [_i64, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, C.c_float, C.c_float,
                              C.c_float, _vp, _vp, _vp],
     "ephip_ft_pack_operand": [_i64, _i32, _vp, _i64, _i32, _i64, _vp, _vp],

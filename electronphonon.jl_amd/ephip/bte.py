@@ -471,6 +471,18 @@ def occupation_to_conductivity(df, bs: BandStates, params: ElectronTransportPara
     return (df.T @ bs.vs) * (bs.weight * params.spin_degeneracy / params.volume)
 
 
+def _bte_step(y, inv_tau, rhs, mixing: float, df, bs: BandStates, params: ElectronTransportParams, old=None):
+    """df <- mixing (y / inv_tau + rhs) + (1 - mixing) df (y None: unchanged); returns 10 float64: the conductivity of
+    df and, with ``old`` (an earlier return), the norm of its change relative to its own."""
+    torch = _torch()
+    vs = bs.vs.contiguous()
+    buf = torch.empty(9 * 256 + 10, dtype=torch.float64, device=df.device)
+    out = buf[9 * 256:]
+    L.call("ephip_bte_step", df.shape[0], L.ptr(y), L.ptr(inv_tau), L.ptr(rhs), mixing, L.ptr(df), L.ptr(vs),
+           float(bs.weight * params.spin_degeneracy / params.volume), L.ptr(old), L.ptr(buf), L.ptr(out), L.stream_handle())
+    return out
+
+
 @dataclasses.dataclass
 class BTEResult:
     sigma_serta: np.ndarray   # (nT, 3, 3)
@@ -489,31 +501,31 @@ def solve_electron_bte(calc: BoltzmannCalculator, max_iter: int = 100, rtol: flo
     bs, params = calc.bs, calc.params
     if bs.vs is None:
         raise ValueError("velocities are not set: call compute_velocities first")
+    if bs.vs.dtype != torch.float64 or tuple(bs.vs.shape) != (bs.n, 3):
+        raise ValueError(f"velocities {tuple(bs.vs.shape)} {bs.vs.dtype}, expected ({bs.n}, 3) float64")
     nT = len(params.Tlist)
     out_s = np.zeros((nT, 3, 3))
     out = np.zeros((nT, 3, 3))
     niters, conv, hist = [], [], []
     for iT in range(nT):
         mu, T = float(params.mulist[iT]), float(params.Tlist[iT])
-        inv_tau = calc.S_out[iT]
+        inv_tau = calc.S_out[iT].contiguous()
         rhs = (_dfermi(bs.es - mu, T) / inv_tau).unsqueeze(1) * bs.vs
-        s_serta = occupation_to_conductivity(rhs, bs, params)
         df = rhs.clone()
+        obs = _bte_step(None, None, None, 1.0, df, bs, params)
         tmp = torch.empty_like(df)
-        obs = s_serta
-        h = [s_serta.cpu().numpy()]
+        h = [obs[:9].view(3, 3).cpu().numpy()]
         it, ok = 0, False
         for it in range(1, max_iter + 1):
             calc.spmv(iT, df, tmp)
-            new = tmp / inv_tau.unsqueeze(1) + rhs
-            df = new * mixing + df * (1.0 - mixing)
-            obs_old, obs = obs, occupation_to_conductivity(df, bs, params)
-            h.append(obs.cpu().numpy())
-            if float(torch.linalg.norm(obs - obs_old) / torch.linalg.norm(obs)) < rtol:
+            obs = _bte_step(tmp, inv_tau, rhs, mixing, df, bs, params, old=obs)
+            host = obs.cpu().numpy()
+            h.append(host[:9].reshape(3, 3))
+            if host[9] < rtol:
                 ok = True
                 break
-        out_s[iT] = s_serta.cpu().numpy()
-        out[iT] = obs.cpu().numpy()
+        out_s[iT] = h[0]
+        out[iT] = h[-1]
         niters.append(it)
         conv.append(ok)
         hist.append(h)

@@ -619,6 +619,13 @@ int ephip_bte_spmv(int32_t nunits, int32_t nbw, int32_t nT, int32_t iT, const in
                    const uint32_t *row_code, const int64_t *unit_state_index, const double *S_in, const double *x,
                    double *y, void *stream);
 
+/* The rest of an iteration of that solve: df[3*i + a] <- mixing (y[3*i + a] / inv_tau[i] + rhs[3*i + a])
+ * + (1 - mixing) df[3*i + a] for n states (y null: df is left as it is), then out[3*a + b] = scale * sum_i
+ * df[3*i + a] vs[3*i + b] (occupation_to_conductivity, src/boltzmann/electron_lbte.jl:43-50) and out[9] =
+ * |out - old| / |out| over the nine (0 if old is null). work: 9 * 256 doubles; out: 10 doubles, not old. */
+int ephip_bte_step(int64_t n, const double *y, const double *inv_tau, const double *rhs, double mixing, double *df,
+                   const double *vs, double scale, const double *old, double *work, double *out, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
