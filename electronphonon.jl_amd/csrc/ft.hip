@@ -13,7 +13,7 @@
 // used here were checked on gfx950: f32 16x16x4 and bf16 16x16x32 return C[4(l/16)+r][l%16] in
 // lane l, register r; f64 16x16x4 returns C[4r+l/16][l%16].
 //
-// Tiles (ft64_kernel has its own): 256 threads = 4 waves in a 2 x 2 arrangement; a workgroup owns
+// Tiles (ft64_kernel and ft32_kernel have their own): 256 threads = 4 waves in a 2 x 2 arrangement; a workgroup owns
 // TM = 64 complex rows and TN columns; K advances KC = 16 complex R per LDS stage. FP32 and FP64 use the 16x16x4 MFMA
 // (lane l holds A[l%16][l/16], B[l/16][l%16]); the split-BF16 form uses
 // 16x16x32 bf16 MFMAs with hi/lo operand splitting and three products per real product.
@@ -133,134 +133,14 @@ struct FtBatch {
     const int *ncol = nullptr;
 };
 
-template <int TN>
-__global__ __launch_bounds__(256) void ft_mfma_kernel(int64_t ndata, int nr, const cplx<float> *__restrict__ op,
-                                                      int64_t ldop, const int *__restrict__ irvec, int nk,
-                                                      const double *__restrict__ xk, cplx<float> *__restrict__ out,
-                                                      int64_t ldout, FtBatch bt) {
-    using T = float;
-    using acc_t = f32x4;
-    constexpr int NCB = TN / 32;  // 16-column blocks per wave
-    __shared__ cplx<T> As[FT_KC][FT_TM + FT_APAD];
-    __shared__ T Bs[FT_KC][2][TN + FT_BPAD];
-    __shared__ float2 tab[FT_TAB_MAX][TN];
-    __shared__ int red[24];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int64_t d0 = (int64_t)blockIdx.y * FT_TM;
-    const int64_t j0 = (int64_t)blockIdx.x * TN;
-    {
-        const int u = blockIdx.z;
-        if (bt.ncol) nk = bt.ncol[u];
-        if (j0 >= nk) return;  // uniform for the block: nothing of this unit in this column tile
-        op += u * bt.op_stride;
-        out += u * bt.out_stride;
-        if (bt.col_index) bt.col_index += u * bt.col_stride;
-    }
-    const FtAxes ax = ft_axes(irvec, nr, red);
-    const bool use_tab = ax.total <= FT_TAB_MAX;
-    if (use_tab) {
-        ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
-        __syncthreads();  // a column's rows are written by 256 / TN waves and read by each of them
-    }
-
-    // The phase column this thread generates is fixed for the whole kernel; its R rows are uniform
-    // per wavefront (TN is a multiple of 64).
-    const int pj = tid % TN;
-    const int prl0 = __builtin_amdgcn_readfirstlane(tid / TN);
-    constexpr int PSTEP = 256 / TN;
-    double x0 = 0, x1 = 0, x2 = 0;
-    const bool pvalid = (j0 + pj) < nk;
-    if (pvalid) {
-        const int64_t pt = bt.col_index ? bt.col_index[j0 + pj] : j0 + pj;
-        x0 = xk[3 * pt];
-        x1 = xk[3 * pt + 1];
-        x2 = xk[3 * pt + 2];
-    }
-
-    acc_t acc[4][NCB];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < NCB; j++) acc[i][j] = acc_t{0, 0, 0, 0};
-
-    for (int r0 = 0; r0 < nr; r0 += FT_KC) {
-        // op tile: FT_TM x FT_KC complex, coalesced along d
-        for (int e = tid; e < FT_TM * FT_KC; e += 256) {
-            const int dl = e % FT_TM, rl = e / FT_TM;
-            const int64_t d = d0 + dl;
-            const int r = r0 + rl;
-            cplx<T> v{0, 0};
-            if (d < ndata && r < nr) v = op[d + ldop * r];
-            As[rl][dl] = v;
-        }
-        // phase tile: FT_KC x TN
-        if (use_tab) {
-            for (int rl = prl0; rl < FT_KC; rl += PSTEP) {
-                const int r = r0 + rl;
-                float c = 0.f, s = 0.f;
-                if (r < nr) ft_table_phase(&tab[0][0], TN, ax, irvec + 3 * r, pj, c, s);
-                Bs[rl][0][pj] = c;
-                Bs[rl][1][pj] = s;
-            }
-        } else {
-            for (int rl = prl0; rl < FT_KC; rl += PSTEP) {
-                const int r = r0 + rl;
-                T c = 0, s = 0;
-                if (pvalid && r < nr) {
-                    const double t = irvec[3 * r] * x0 + irvec[3 * r + 1] * x1 + irvec[3 * r + 2] * x2;
-                    cis2pi(t, c, s);
-                }
-                Bs[rl][0][pj] = c;
-                Bs[rl][1][pj] = s;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < FT_KC / 2; ks++) {
-            const int kk = lane >> 4;
-            const int rl = 2 * ks + (kk >> 1);
-            const int cc = kk & 1;
-            T a[4], b[NCB];
-#pragma unroll
-            for (int rb = 0; rb < 4; rb++) {
-                const int rr = wm * 64 + 16 * rb + (lane & 15);
-                const cplx<T> v = As[rl][rr >> 1];
-                a[rb] = (rr & 1) == 0 ? (cc == 0 ? v.re : -v.im) : (cc == 0 ? v.im : v.re);
-            }
-#pragma unroll
-            for (int cb = 0; cb < NCB; cb++) b[cb] = Bs[rl][cc][wn * (TN / 2) + 16 * cb + (lane & 15)];
-#pragma unroll
-            for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-                for (int cb = 0; cb < NCB; cb++) acc[rb][cb] = mfma16x16x4<T>(a[rb], b[cb], acc[rb][cb]);
-        }
-        __syncthreads();
-    }
-
-    const int q = lane >> 4;
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-        for (int cb = 0; cb < NCB; cb++) {
-            const int64_t d = d0 + (wm * 64 + 16 * rb) / 2 + 2 * q;
-            const int64_t j = j0 + wn * (TN / 2) + 16 * cb + (lane & 15);
-            if (j < nk) {
-                if (d < ndata) out[d + ldout * j] = cplx<T>{acc[rb][cb][0], acc[rb][cb][1]};
-                if (d + 1 < ndata) out[d + 1 + ldout * j] = cplx<T>{acc[rb][cb][2], acc[rb][cb][3]};
-            }
-        }
-}
-
 // FP64 form. WR x WC waves of a workgroup own 8 RB WR complex rows and 16 CB WC columns, 16 RB real rows and 16 CB columns
 // each; an entry's sum runs over R in order, 2 R an MFMA, whatever the tile. Two LDS stages of KC complex R: the next
-// one is filled while the MFMAs of this one run, by FT64_FILL waves that do nothing else: the sincos keeps its constants
+// one is filled while the MFMAs of this one run, by FT_FILL waves that do nothing else: the sincos keeps its constants
 // in the registers that hold the others' sums (one role for all waves spilled, or left room for a quarter of the tile).
 // Bound by the FP64 units, which the MFMAs and the phases share. 256 rows x 729 R x 32768 columns: 0.95 ms (51 TFLOP/s)
 // for 1.25 before, when each 64 rows formed the phases anew; without any phases 0.88, without filling 0.75.
 // 64 rows x 125 R x 505 columns: 9.6 us for 45, in 64 workgroups and 4 stages for 8 and 8.
-constexpr int FT64_FILL = 4;
+constexpr int FT_FILL = 4;
 __host__ __device__ constexpr int ft64_apitch(int tm) { return tm + 8; }    // complex: the next R half a bank row on
 __host__ __device__ constexpr int ft64_bpitch(int tn) { return tn + 16; }   // doubles, likewise re and im
 __host__ __device__ constexpr size_t ft64_stage_doubles(int kc, int tm, int tn) {
@@ -279,7 +159,7 @@ __global__ __launch_bounds__(1024) void ft64_kernel(int64_t ndata, int nr, const
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t d0 = (int64_t)blockIdx.y * TM;
     const int j0 = blockIdx.x * TN;
-    constexpr int NW = FT64_FILL;
+    constexpr int NW = FT_FILL;
 
     // operand: items of 64 rows of one R, phases: items of 64 (R, column) pairs; a thread's column is fixed
     const int nitem = KC * ((TM + 63) / 64), npitem = KC * TN / 64;
@@ -390,13 +270,13 @@ static int launch_ft64(int WR, int WC, int64_t ndata, int nr, const cplx<double>
     const int TM = 8 * RB * WR, TN = 16 * CB * WC;
     const size_t lds = 2 * sizeof(double) * ft64_stage_doubles(KC, TM, TN);
     const int64_t gy = (ndata + TM - 1) / TM;
-    EPHIP_REQUIRE(FT64_FILL + WR * WC <= 16 && TN <= 64 && KC * ((TM + 63) / 64) <= AE * FT64_FILL && lds <= 160 * 1024,
+    EPHIP_REQUIRE(FT_FILL + WR * WC <= 16 && TN <= 64 && KC * ((TM + 63) / 64) <= AE * FT_FILL && lds <= 160 * 1024,
                   "fourier_c64: no workgroup of %d x %d waves", WR, WC);
     if (lds > 64 * 1024)
         EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ft64_kernel<RB, CB, KC, AE>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const dim3 g((unsigned)((nk + TN - 1) / TN), (unsigned)gy);
-    ft64_kernel<RB, CB, KC, AE><<<g, 64 * (FT64_FILL + WR * WC), lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out,
+    ft64_kernel<RB, CB, KC, AE><<<g, 64 * (FT_FILL + WR * WC), lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out,
                                                                            ldout, WR, WC);
     return EPHIP_OK;
 }
@@ -444,7 +324,167 @@ static int ft64_run(int64_t ndata, int nr, const cplx<double> *op, int64_t ldop,
     return launch_ft64<1, 1, 32, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
 }
 
-// Double-buffered form of ft_mfma_kernel: two LDS stages; the next stage's operand loads are issued
+// FP32 form. As ft64_kernel: FT_FILL waves fill two LDS stages of KC complex R, WR x WC waves multiply. A wave owns
+// 16 RB complex rows and 32 columns on 32x32x2 MFMAs, one R each: a sum runs over R in order, the real part's term
+// first, as on the 16x16x4 ones. All waves tabulate the per-axis phases first. Bound by the filling between the MFMAs
+// and the table: 128 units of 48 rows x 125 R x 2158 of 4096 columns in 174 us (60 TFLOP/s) for 391 with one role for
+// all waves, rows padded to 64 and the column tiles fastest in the grid (290 with that order alone); 107 TFLOP/s at
+// 729 R.
+using f32x16 = __attribute__((__vector_size__(16 * sizeof(float)))) float;
+
+template <int RB, int TN, int KC>
+__global__ __launch_bounds__(1024) void ft32_kernel(int64_t ndata, int nr, const cplx<float> *__restrict__ op,
+                                                    int64_t ldop, const int *__restrict__ irvec, int nk,
+                                                    const double *__restrict__ xk, cplx<float> *__restrict__ out,
+                                                    int64_t ldout, FtBatch bt, unsigned nunits, int WR) {
+    extern __shared__ float ft32_lds[];
+    constexpr int NF = FT_FILL, NPI = KC * TN / (64 * NF), AE = 3 * KC / NF, PB = TN + 32;
+    __shared__ float2 tab[FT_TAB_MAX][TN];
+    __shared__ int red[96];
+    const int TM = 16 * RB * WR, PA = TM + 4;
+    const int stage = KC * 2 * (PA + PB);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Units first: the chip hands workgroups to its shader engines in turn, and a tail of column tiles without work in
+    // every unit would leave the same engines idle (half of the columns kept: twice the time).
+    const unsigned tile = blockIdx.x / nunits, rtiles = (unsigned)((ndata + TM - 1) / TM);
+    const int64_t d0 = (int64_t)(tile % rtiles) * TM;
+    const int j0 = (int)(tile / rtiles) * TN;
+    {
+        const int u = blockIdx.x % nunits;
+        if (bt.ncol) nk = bt.ncol[u];
+        if (j0 >= nk) return;  // uniform for the block: nothing of this unit in this column tile
+        op += u * bt.op_stride;
+        out += u * bt.out_stride;
+        if (bt.col_index) bt.col_index += u * bt.col_stride;
+    }
+    const FtAxes ax = ft_axes(irvec, nr, red);
+    const bool use_tab = ax.total <= FT_TAB_MAX;
+    if (use_tab) ft_fill_table<TN>(tab, ax, xk, bt.col_index, j0, nk);
+    __syncthreads();  // the table is filled
+
+    if (wave < NF) {
+        const int nchunk = (TM + 63) / 64, nitem = KC * nchunk;
+        const int pj = lane & (TN - 1);
+        static_assert(TN % 64 == 0, "a phase item is 64 columns of one R");
+        cplx<float> areg[AE];
+        auto fill = [&](int r0, float *st) {
+#pragma unroll
+            for (int i = 0; i < AE; i++) {
+                const int it = wave + NF * i, r = r0 + it % KC, dl = it / KC * 64 + lane;
+                areg[i] = (it < nitem && dl < TM && d0 + dl < ndata && r < nr) ? op[d0 + dl + ldop * r]
+                                                                                : cplx<float>{0, 0};
+            }
+            float *B = st + 2 * KC * PA;
+#pragma unroll
+            for (int i = 0; i < NPI; i++) {
+                const int it = wave + NF * i, rl = it % KC, r = r0 + rl, j = it / KC * 64 + pj % 64;
+                float c = 0.f, s = 0.f;
+                if (r < nr) {
+                    if (use_tab) {
+                        ft_table_phase(&tab[0][0], TN, ax, irvec + 3 * r, j, c, s);
+                    } else if (j0 + j < nk) {
+                        const int64_t pt = bt.col_index ? bt.col_index[j0 + j] : j0 + j;
+                        const double t = irvec[3 * r] * xk[3 * pt] + irvec[3 * r + 1] * xk[3 * pt + 1] +
+                                         irvec[3 * r + 2] * xk[3 * pt + 2];
+                        cis2pi(t, c, s);
+                    }
+                }
+                B[2 * rl * PB + j] = c;
+                B[(2 * rl + 1) * PB + j] = s;
+            }
+            cplx<float> *A = reinterpret_cast<cplx<float> *>(st);
+#pragma unroll
+            for (int i = 0; i < AE; i++) {
+                const int it = wave + NF * i, dl = it / KC * 64 + lane;
+                if (it < nitem && dl < TM) A[it % KC * PA + dl] = areg[i];
+            }
+        };
+        fill(0, ft32_lds);
+        for (int r0 = KC, b = 1; r0 < nr; r0 += KC, b ^= 1) {
+            __syncthreads();
+            fill(r0, ft32_lds + b * stage);
+        }
+        __syncthreads();  // as many as the other waves meet, one a stage
+        return;
+    }
+    const int cw = wave - NF, wm = cw % WR, wn = cw / WR;
+    f32x16 acc[RB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < 16; j++) acc[i][j] = 0.f;
+    // lane l: row l%32 of the block (complex row, part), column l%32, k = l/32: the phase's part
+    const int il = lane & 31, h = lane >> 5;
+    const int part = h ^ (il & 1);
+    const unsigned flip = (h && !(il & 1)) ? 0x80000000u : 0u;
+    const int aoff = 2 * (wm * 16 * RB + (il >> 1)) + part;
+    const int boff = 2 * KC * PA + h * PB + wn * 32 + il;
+    for (int r0 = 0, b = 0; r0 < nr; r0 += KC, b ^= 1) {
+        __syncthreads();  // this stage is filled, and the other one read
+        const float *cur = ft32_lds + b * stage;
+        float av[2][RB], bv[2];  // the next R's operands are on their way
+        auto load = [&](int rl, int p) {
+            bv[p] = cur[boff + 2 * rl * PB];
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) av[p][rb] = cur[aoff + 2 * rl * PA + 32 * rb];
+        };
+        load(0, 0);
+#pragma unroll
+        for (int rl = 0; rl < KC; rl++) {
+            if (rl + 1 < KC) load(rl + 1, (rl + 1) & 1);
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++)
+                acc[rb] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                    __uint_as_float(__float_as_uint(av[rl & 1][rb]) ^ flip), bv[rl & 1], acc[rb], 0, 0, 0);
+        }
+    }
+    const int64_t j = j0 + wn * 32 + il;
+    if (j >= nk) return;
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int q = 0; q < 8; q++) {  // registers 2q, 2q + 1: row 8 (q / 2) + 4 h + 2 (q % 2) of the block
+            const int64_t d = d0 + wm * 16 * RB + 16 * rb + 4 * (q >> 1) + 2 * h + (q & 1);
+            if (d < ndata) out[d + ldout * j] = cplx<float>{acc[rb][2 * q], acc[rb][2 * q + 1]};
+        }
+}
+
+template <int RB, int TN, int KC>
+static int launch_ft32(int WR, int nunits, int64_t ndata, int nr, const cplx<float> *op, int64_t ldop, const int *irvec,
+                       int nk, const double *xk, cplx<float> *out, int64_t ldout, const FtBatch &bt, hipStream_t s) {
+    const int TM = 16 * RB * WR, waves = FT_FILL + WR * TN / 32;
+    const size_t lds = 2 * sizeof(float) * KC * 2 * (TM + 4 + TN + 32);
+    EPHIP_REQUIRE(waves <= 16 && TM <= 192, "fourier_c32: no workgroup of %d row waves", WR);
+    if (lds + sizeof(float2) * FT_TAB_MAX * TN + 384 > 64 * 1024)
+        EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ft32_kernel<RB, TN, KC>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int64_t wgs = (int64_t)((nk + TN - 1) / TN) * ((ndata + TM - 1) / TM) * nunits;
+    EPHIP_REQUIRE(wgs <= 0x7fffffffLL, "fourier_c32: %lld workgroups", (long long)wgs);
+    ft32_kernel<RB, TN, KC><<<(unsigned)wgs, 64 * waves, lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt,
+                                                                   (unsigned)nunits, WR);
+    return EPHIP_OK;
+}
+
+// The tile: rows of a wave that leave the least padding (16, 32, 48), two row waves beyond 48 rows and 128 columns up to
+// there; smaller ones while the workgroups are fewer than the CUs, where the latency of a stage counts. 192 rows x 125 R
+// x 600 columns x 32 units: 58 us with 96 x 64 tiles, 56 with 64 x 64, 63 with 48 x 128; 12 rows x 125 R x 819 x 128
+// units: 54 with 16 x 64, 66 with 32 x 128; 48 rows x 125 R x 4096 columns: 18 with 16 x 64, 22 with 32 x 64.
+static int ft32_run(int nunits, int64_t ndata, int nr, const cplx<float> *op, int64_t ldop, const int *irvec, int nk,
+                    const double *xk, cplx<float> *out, int64_t ldout, const FtBatch &bt, hipStream_t s) {
+    auto wgs = [&](int tm, int tn) { return (ndata + tm - 1) / tm * ((nk + tn - 1) / tn) * nunits; };
+    auto padded = [&](int tm) { return (ndata + tm - 1) / tm * tm; };
+    if (ndata > 16 && ndata <= 32 && wgs(32, 128) >= 256)
+        return launch_ft32<2, 128, 8>(1, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);
+    if (ndata > 32 && ndata <= 48 && wgs(48, 128) >= 256)
+        return launch_ft32<3, 128, 8>(1, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);
+    if (ndata > 48 && padded(96) <= padded(64) && wgs(96, 64) >= 256)
+        return launch_ft32<3, 64, 8>(2, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);
+    if (ndata > 48 && wgs(64, 64) >= 128)
+        return launch_ft32<2, 64, 8>(2, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);
+    return launch_ft32<1, 64, 8>(1, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);
+}
+
+// Two LDS stages with every wave in both roles; the next stage's operand loads are issued
 // before the current stage's MFMAs and its phase entries are generated one per K step between them,
 // so global latency and the sincos work overlap the matrix cores; one barrier per stage. KC (complex R
 // per stage) is a tuning parameter.
@@ -580,8 +620,8 @@ __global__ __launch_bounds__(256) void ft_mfma_db_kernel(int64_t ndata, int nr, 
 }
 
 // Kernel variant per contraction kind, set by the tuner (ephip_ft_set_variant). Kinds:
-// 0 = FP32 wide (nk > 64), 1 = FP32 narrow (nk <= 64), 2 = FP64. Variants: 0 = single-buffered (FP64: ft64_kernel),
-// 1 = double-buffered KC 16, 2 = double-buffered KC 8.
+// 0 = FP32 wide (nk > 64), 1 = FP32 narrow (nk <= 64), 2 = FP64. Variants: 0 = filling and multiplying waves
+// (ft32_kernel, ft64_kernel), 1 = ft_mfma_db_kernel with KC 16, 2 = with KC 8.
 static int g_ft_variant[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 
 template <class T, int TN>
@@ -589,10 +629,8 @@ static void launch_ft(int variant, dim3 g, hipStream_t s, int64_t ndata, int nr,
                       const int *irvec, int nk, const double *xk, cplx<T> *out, int64_t ldout, FtBatch bt) {
     if (variant == 1)
         ft_mfma_db_kernel<T, TN, 16><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
-    else if (variant == 2)
+    else
         ft_mfma_db_kernel<T, TN, 8><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
-    else if constexpr (sizeof(T) == 4)
-        ft_mfma_kernel<TN><<<g, 256, 0, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1969,7 +2007,10 @@ extern "C" int ephip_fourier_c32(int64_t ndata, int32_t nr, const void *op, int6
     const unsigned gy = (unsigned)((ndata + FT_TM - 1) / FT_TM);
     auto o = static_cast<const cplx<float> *>(op);
     auto c = static_cast<cplx<float> *>(out);
-    if (precision == EPHIP_PREC_FP32) {
+    if (precision == EPHIP_PREC_FP32 && g_ft_variant[nk <= 64] == 0) {
+        st = ft32_run(1, ndata, nr, o, ldop, irvec, nk, xk, c, ldout, FtBatch{}, s);
+        if (st) return st;
+    } else if (precision == EPHIP_PREC_FP32) {
         if (nk <= 64) {
             dim3 g((nk + 63) / 64, gy);
             launch_ft<float, 64>(g_ft_variant[1], g, s, ndata, nr, o, ldop, irvec, nk, xk, c, ldout, FtBatch{});
@@ -2047,7 +2088,10 @@ extern "C" int ephip_fourier_batched_c32(int64_t ndata, int32_t nr, const void *
     auto c = static_cast<cplx<float> *>(out);
     const bool small = nk_max <= 64;
     dim3 g(small ? (nk_max + 63) / 64 : (nk_max + 127) / 128, gy, nunits);
-    if (precision == EPHIP_PREC_FP32) {
+    if (precision == EPHIP_PREC_FP32 && g_ft_variant[small] == 0) {
+        st = ft32_run(nunits, ndata, nr, o, ldop, irvec, nk_max, xk, c, ldout, bt, s);
+        if (st) return st;
+    } else if (precision == EPHIP_PREC_FP32) {
         if (small)
             launch_ft<float, 64>(g_ft_variant[1], g, s, ndata, nr, o, ldop, irvec, nk_max, xk, c, ldout, bt);
         else

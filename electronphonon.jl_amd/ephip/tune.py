@@ -26,7 +26,7 @@ KQ_FOLD_VARIANT_NAMES = {0: "folded stage-2/3 sums on symmetric boxes", 1: "gene
 KQ_STAGE1_VARIANTS = (0, 1)
 KQ_STAGE1_VARIANT_NAMES = {0: "stage 1 per (unit, q1) workgroup", 1: "stage-1 pre-pass into a workspace"}
 VARIANTS = (0, 1, 2)
-VARIANT_NAMES = {0: "single-buffered KC16", 1: "double-buffered KC16", 2: "double-buffered KC8"}
+VARIANT_NAMES = {0: "filling and multiplying waves", 1: "double-buffered KC16", 2: "double-buffered KC8"}
 PACKED_VARIANTS = (0, 1, 2, 3, 4, 5, 6, 7)
 PACKED_VARIANT_NAMES = {0: "128x128", 1: "128x128 + operand prefetch", 2: "192x64", 3: "192x64 XCD-grouped",
                         4: "192x64 XCD-grouped, mid-sequence LDS writes", 5: "as 4, pipelined", 6: "as 3, pipelined",

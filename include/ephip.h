@@ -394,8 +394,8 @@ int ephip_eph_kq_rotate_packed_bf16x3(int32_t nw, int32_t nm, int32_t nbw, int32
                                       void *stream);
 
 /* Kernel variant of the Fourier contractions, chosen by the tuner (ephip/tune.py) from timings on the
- * live shapes. kind: 0 = FP32 with nk > 64, 1 = FP32 with nk <= 64, 2 = FP64; variant: 0 = single-
- * buffered LDS stages of 16 R, 1 = double-buffered stages of 16 R, 2 = double-buffered stages of 8 R.
+ * live shapes. kind: 0 = FP32 with nk > 64, 1 = FP32 with nk <= 64, 2 = FP64; variant: 0 = some waves
+ * fill LDS stages while the others multiply, 1 = every wave does both with stages of 16 R, 2 = of 8 R.
  * kind 3 = pre-packed split-BF16 with ndata >= 128 (except 192-row operands, always 192 x 64);
  * variant: 0 = 128 x 128 tiles, 1 = 128 x 128 with the next stage's operand prefetched into registers,
  * 2 = 192 x 64 tiles (ndata a multiple of 192), 3 = 192 x 64 tiles in XCD-grouped workgroup order (the
