@@ -207,10 +207,11 @@ struct BtePair {
 
 // The kept (q, window band) pairs of 256 columns are listed in LDS, so that lanes hold pairs: taken column by column
 // the few second bands cost every wave that has one a whole pass (measured 1.33 against 0.80 ms, 3.07M rows of 12
-// modes at 3 temperatures; the per-term form took 7.65 ms). Bound by the FP64 exponentials.
+// modes at 3 temperatures, and 0.38 since the units come first in the grid; the per-term form took 7.65 ms). Bound by the
+// FP64 exponentials.
 template <int METHOD, int NT>  // NT temperatures per pass
 __global__ __launch_bounds__(256) void bte_accumulate_tab_kernel(
-    int64_t cs, int nbw, int nm, int nq, const int *__restrict__ count, const int *__restrict__ col_index,
+    int nunits, int64_t cs, int nbw, int nm, int nq, const int *__restrict__ count, const int *__restrict__ col_index,
     const int *__restrict__ ikq, const float *__restrict__ g2, const int64_t *__restrict__ unit_state_index,
     const int64_t *__restrict__ state_offset, const int64_t *__restrict__ bmin, const int64_t *__restrict__ bmax,
     const double *__restrict__ e_state, const double *__restrict__ tab_q, const double *__restrict__ tab_s, double wtq,
@@ -220,8 +221,9 @@ __global__ __launch_bounds__(256) void bte_accumulate_tab_kernel(
     __shared__ int ciq[256], cf0[256], wsum[4];
     extern __shared__ uint16_t list[];  // [256 nbw] column | band << 8
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int64_t c0 = (int64_t)blockIdx.x * 256;
-    const int u = blockIdx.y, cnt = count[u];
+    // units first: with the columns first, the empty workgroups at the end of every unit all fell to the same XCDs
+    const int64_t c0 = (int64_t)(blockIdx.x / nunits) * 256;
+    const int u = (int)(blockIdx.x % nunits), cnt = count[u];
     if (c0 >= cnt) return;  // uniform
     const int64_t i = unit_state_index[u], row0 = (int64_t)u * cs + c0, orow0 = rowptr[u] + c0;
     int nb = 0;
@@ -633,14 +635,16 @@ extern "C" int ephip_bte_accumulate_tables(int32_t nunits, int64_t cs, int32_t n
     EPHIP_REQUIRE(count && col_index && ikq && g2 && unit_state_index && state_offset && bmin && bmax && e_state &&
                       tab_q && tab_s && Ts && etas && rowptr && S_out && S_in && row_code,
                   "bte_accumulate_tables: null device pointer");
+    const int64_t wgs = (cs + 255) / 256 * nunits;
+    EPHIP_REQUIRE(wgs <= 0x7fffffffLL, "bte_accumulate_tables: %lld workgroups", (long long)wgs);
     using K = decltype(&bte_accumulate_tab_kernel<1, 1>);
 #define BTE_ROW(m) {bte_accumulate_tab_kernel<m, 1>, bte_accumulate_tab_kernel<m, 2>, bte_accumulate_tab_kernel<m, 3>}
     static const K kern[6][3] = {BTE_ROW(1), BTE_ROW(2), BTE_ROW(3), BTE_ROW(4), BTE_ROW(5), BTE_ROW(6)};
 #undef BTE_ROW
-    kern[method - 1][nT == 1 ? 0 : nT == 2 ? 1 : 2]<<<dim3(nbk(cs), (unsigned)nunits), 256,
+    kern[method - 1][nT == 1 ? 0 : nT == 2 ? 1 : 2]<<<(unsigned)wgs, 256,
                                                       (size_t)256 * nbw * sizeof(uint16_t), as_stream(stream)>>>(
-        cs, nbw, nm, nq, count, col_index, ikq, g2, unit_state_index, state_offset, bmin, bmax, e_state, tab_q, tab_s,
-        wtq, nT, Ts, etas, smearing, w_cut, nstates, rowptr, S_out, S_in, row_code,
+        nunits, cs, nbw, nm, nq, count, col_index, ikq, g2, unit_state_index, state_offset, bmin, bmax, e_state, tab_q,
+        tab_s, wtq, nT, Ts, etas, smearing, w_cut, nstates, rowptr, S_out, S_in, row_code,
         (nm & 3) == 0 && (reinterpret_cast<uintptr_t>(g2) & 15) == 0);
     EPHIP_LAUNCHED();
     return EPHIP_OK;
