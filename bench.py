@@ -55,7 +55,7 @@ def _staged(v) -> bool:
 
 
 KERNEL_NAMES = {
-    ("RR->kR", "gridopt"): "gridopt_stage1_kernel + gridopt_kR_project_mfma_kernel: staged (GridOpt) RR->kR over "
+    ("RR->kR", "gridopt"): "gridopt_stage1_kernel + lane_project_kernel: staged (GridOpt) RR->kR over "
                            "Re, stages 2/3 with the k-side window projection on FP32 MFMAs",
     ("kR->kq", "gridopt"): "gridopt_kq_rotate_kernel: staged (GridOpt) kR->kq over the q grid with the k+q/phonon "
                            "rotations and g2, FP32 VALU",

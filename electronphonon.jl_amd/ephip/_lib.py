@@ -93,6 +93,9 @@ SIGNATURES = {
                                 _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "ephip_staged_project": [_i32, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _i32, _vp, _i32, _vp, _vp, _vp,
                              _vp, _vp, _vp, _i64, _vp],
+    "ephip_lane_tables": [_i32, _i32, _i32, _vp, _i64, _i64, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                          _vp, _vp, _vp],
+    "ephip_lane_project": [_i32, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "ephip_staged_rr_to_rq": [_i64, _i32, _i32, _i32, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp],
     "ephip_staged_rq_rotate": [_i32, _i32, _i32, _i32, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
                                _i64, _vp, _vp, _vp, _vp],

@@ -978,7 +978,8 @@ class OuterKLoop:
 
 
 class _GridOptKR:
-    """Staged RR->kR over Re (ephip_gridopt_stage1_planes + ephip_gridopt_kR_project[_mfma]), the device
+    """Staged RR->kR over Re (ephip_gridopt_stage1_planes + ephip_lane_project where the box is symmetric along axes
+    2 and 3 and nw <= 16, else ephip_gridopt_kR_project[_mfma] or ephip_staged_project), the device
     GridOpt of src/wannier/GridOpt.jl: Re embedded in its bounding box, the surviving k (grid order,
     third index fastest) grouped into k1 planes and (k1, k2) lines. Stage 1 runs for a group of PLANES
     consecutive planes at once (one pass over the operand for all of them); the two most recent groups
@@ -1017,6 +1018,11 @@ class _GridOptKR:
         self.n1, self.n2, self.n3 = (int(x) for x in n)
         self.np = max(self.n2, self.n3, 3)
         self.rmin = [int(x) for x in lo]
+        # one lane per (operator column, j) where the box is symmetric along axes 2 and 3: j padded to 4, 8 or 16 lanes
+        self.jl = 0
+        if (st.nw <= 16 and (self.mfma or self.general) and self.np in (3, 5, 7)
+                and self.rmin[1] == self.rmin[2] == -(self.np // 2)):
+            self.jl = 4 if st.nw <= 4 else 8 if st.nw <= 8 else 16
         rmap = -np.ones((self.n3, self.n2, self.n1), np.int32)
         rmap[r[:, 2] - lo[2], r[:, 1] - lo[1], r[:, 0] - lo[0]] = np.arange(len(r), dtype=np.int32)
         self.rmap = torch.from_numpy(rmap.ravel()).to(dev)
@@ -1049,6 +1055,12 @@ class _GridOptKR:
     def use_general(self):
         """Take the general form (ephip_staged_project) in place of the VALU projection."""
         self.general, self._nb = True, 1
+        if self.np in (3, 5, 7) and self.rmin[1] == self.rmin[2] == -(self.np // 2):
+            self.jl = 8
+
+    def lanes(self) -> bool:
+        """The lane-private projection applies (ephip_lane_project)."""
+        return self.jl > 0 and (self.general or self.folded())
 
     def folded(self) -> bool:
         """The MFMA projection kernel's folded stage-2 sums apply: the Re box spans -h .. h along axis 2
@@ -1094,18 +1106,37 @@ class _GridOptKR:
             self.ph2 = torch.empty((loop.nk_batch, self.np), dtype=torch.complex64, device=dev)  # lines <= k
         return self.ucol, self.ph2, self.ph3
 
-    def _run_general(self, loop, i0, n, u0, u1, A, stream, l_first, l_last):
-        """Stage 1 and one projection launch per group of PLANES planes. Planes are kept between batches that
-        advance through the k list; a batch that starts before the last one's end recomputes what it needs."""
+    def _lane_tables(self, loop, dev):
+        """Per-batch tables of the lane-private form (four units of padding), allocated once."""
+        torch = _torch()
+        if getattr(self, "lane_ucol", None) is None:
+            self.lane_ucol = torch.empty((loop.max_units + 4, self.jl), dtype=torch.complex64, device=dev)
+            self.lane_c3 = torch.empty((loop.max_units + 4, 8), dtype=torch.float32, device=dev)
+            self.lane_c2 = torch.empty((loop.nk_batch, 8), dtype=torch.float32, device=dev)  # lines <= k
+            self.lane_ustart = torch.empty(loop.nk_batch + 1, dtype=torch.int32, device=dev)
+        return self.lane_ustart, self.lane_c2, self.lane_c3, self.lane_ucol
+
+    def _run_groups(self, loop, i0, n, u0, u1, A, stream, l_first, l_last):
+        """Stage 1 and one projection launch per group of PLANES planes. The general form keeps planes between batches
+        that advance through the k list; a batch that starts before the last one's end recomputes what it needs."""
         import ctypes as C
         st = loop.st
-        if i0 < self.next_k:
-            self.invalidate()
-        self.next_k = i0 + n
-        ucol, ph2, ph3 = self._tables(loop, A.device)
-        L.call("ephip_gridopt_kR_tables", st.nw, self.np, self.rmin[1], self.rmin[2], L.ptr(loop.xk_surv), i0,
-               i0 + n, l_first, l_last, L.ptr(self.line_start), u1 - u0, L.ptr(loop.unit_state[u0:u1]),
-               L.ptr(loop.unit_band[u0:u1]), L.ptr(st.el.U), L.ptr(ucol), L.ptr(ph2), L.ptr(ph3), stream)
+        if self.general:
+            if i0 < self.next_k:
+                self.invalidate()
+            self.next_k = i0 + n
+        lanes = self.lanes()
+        if lanes:
+            ustart, c2, c3, lucol = self._lane_tables(loop, A.device)
+            L.call("ephip_lane_tables", st.nw, self.jl, self.np, L.ptr(loop.xk_surv), i0, i0 + n, l_first, l_last,
+                   L.ptr(self.line_start), u1 - u0, L.ptr(loop.k_unit_start_dev), L.ptr(loop.unit_kpos),
+                   L.ptr(loop.unit_state[u0:u1]), L.ptr(loop.unit_band[u0:u1]), L.ptr(st.el.U), L.ptr(ustart),
+                   L.ptr(c2), L.ptr(c3), L.ptr(lucol), stream)
+        else:
+            ucol, ph2, ph3 = self._tables(loop, A.device)
+            L.call("ephip_gridopt_kR_tables", st.nw, self.np, self.rmin[1], self.rmin[2], L.ptr(loop.xk_surv), i0,
+                   i0 + n, l_first, l_last, L.ptr(self.line_start), u1 - u0, L.ptr(loop.unit_state[u0:u1]),
+                   L.ptr(loop.unit_band[u0:u1]), L.ptr(st.el.U), L.ptr(ucol), L.ptr(ph2), L.ptr(ph3), stream)
         planes = self.line_plane[l_first:l_last]
         cut = np.concatenate([[0], np.flatnonzero(np.diff(planes)) + 1, [len(planes)]])
         lines = [(int(planes[a]), l_first + int(a), l_first + int(b)) for a, b in zip(cut[:-1], cut[1:])]
@@ -1116,16 +1147,21 @@ class _GridOptKR:
             m = len(part)
             op1 = (C.c_void_p * m)(*[L.ptr(self._plane_buffer(p, loop.epmat_el, stream)) for p, _, _ in part])
             la, lz = (C.c_int32 * m)(*[x[1] for x in part]), (C.c_int32 * m)(*[x[2] for x in part])
-            L.call("ephip_staged_project", st.nw, self.nd // st.nw, self.np, self.rmin[1], m, C.addressof(op1),
-                   C.addressof(la), C.addressof(lz), i0, i0 + n, l_first, L.ptr(self.line_start),
-                   self.max_line_units, L.ptr(loop.k_unit_start_dev), L.ptr(loop.unit_kpos), L.ptr(ucol), L.ptr(ph2),
-                   L.ptr(ph3), L.ptr(A), A.stride(0), stream)
+            if lanes:
+                L.call("ephip_lane_project", st.nw, self.jl, self.nd // st.nw, self.np, m, C.addressof(op1),
+                       C.addressof(la), C.addressof(lz), l_first, L.ptr(ustart), L.ptr(c2), L.ptr(c3), L.ptr(lucol),
+                       L.ptr(A), A.stride(0), stream)
+            else:
+                L.call("ephip_staged_project", st.nw, self.nd // st.nw, self.np, self.rmin[1], m, C.addressof(op1),
+                       C.addressof(la), C.addressof(lz), i0, i0 + n, l_first, L.ptr(self.line_start),
+                       self.max_line_units, L.ptr(loop.k_unit_start_dev), L.ptr(loop.unit_kpos), L.ptr(ucol),
+                       L.ptr(ph2), L.ptr(ph3), L.ptr(A), A.stride(0), stream)
 
     def run(self, loop, i0, n, u0, u1, A, stream):
         st = loop.st
         l_first, l_last = int(self.line_of_k[i0]), int(self.line_of_k[i0 + n - 1]) + 1
-        if self.general:
-            return self._run_general(loop, i0, n, u0, u1, A, stream, l_first, l_last)
+        if self.general or self.lanes():
+            return self._run_groups(loop, i0, n, u0, u1, A, stream, l_first, l_last)
         if self.mfma:
             ucol, ph2, ph3 = self._tables(loop, A.device)
             L.call("ephip_gridopt_kR_tables", st.nw, self.np, self.rmin[1], self.rmin[2], L.ptr(loop.xk_surv), i0,

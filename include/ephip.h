@@ -356,6 +356,23 @@ int ephip_staged_kq(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits, int32_t
                     const double *omega, const int32_t *dense_strides, double cols_hint, double width_hint,
                     float *g2, void *ep, void *stream);
 
+/* Stages 2/3 of RR->kR with the k-side projection for nw <= 16 and boxes that span -h .. h along axes 2 and 3
+ * (np = 2h + 1 = 3, 5 or 7), one lane per (operator column, j), FP32:
+ *  - ephip_lane_tables: tables of the surviving k k0 <= k < k1, their lines l0 <= l < l1 and their nunits units.
+ *    ustart (l1 - l0 + 1): first unit of each line, counted from kus[k0], and the end. c2 (8 per line), c3 (8 per
+ *    unit): 1, cos(2 pi x j), j = 1 .. h, sin(2 pi x j), x the line's coordinate along axis 2 and the unit's along
+ *    axis 3. ucol (jl per unit, jl = 4, 8 or 16 >= nw): the U column, zero past nw. c3 and ucol hold four units more
+ *    than nunits (read, never used).
+ *  - ephip_lane_project: A of the lines l0[p] <= l < l1[p] of nplanes <= 8 k1 planes; op1, ngcol, A and lda as for
+ *    ephip_staged_project, lb0 the first line of the tables. */
+int ephip_lane_tables(int32_t nw, int32_t jl, int32_t np, const double *xk, int64_t k0, int64_t k1, int32_t l0,
+                      int32_t l1, const int32_t *line_start, int32_t nunits, const int32_t *kus, const int32_t *ukpos,
+                      const int64_t *ustate, const int32_t *uband, const void *U, int32_t *ustart, float *c2,
+                      float *c3, void *ucol, void *stream);
+int ephip_lane_project(int32_t nw, int32_t jl, int64_t ngcol, int32_t np, int32_t nplanes, const void *const *op1,
+                       const int32_t *l0, const int32_t *l1, int32_t lb0, const int32_t *ustart, const float *c2,
+                       const float *c3, const void *ucol, void *A, int64_t lda, void *stream);
+
 /* The outer-q loop by staged transforms, for a tile of nq q (FP32, nw <= 32, nm <= 48):
  *  - ephip_staged_rr_to_rq: get_eph_RR_to_Rq! (src/wannier_to_bloch.jl:277-300) at the tile's q (xq, 3 per q) from the
  *    "ph" layout tensor op (rows b + nbasis (nu + nm Re), nbasis = nw^2, one column per Rp, ldop), with the q side by
