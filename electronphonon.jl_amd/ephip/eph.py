@@ -608,6 +608,10 @@ class OuterKLoop:
         self.staged_q = _GridOptKQ.build(st, general=True) if (staged and self.gridopt_q is None) else None
         if self.gridopt is not None and not self.gridopt.mfma and nw != 16 and staged and self.gridopt.box > 3:
             self.gridopt.use_general()
+        # the lane-private projection adds in another order than the MFMA tiles: boxes of 27 R and callers without the
+        # general staged kernels keep the digits that FP64 rates are held to (_GridOptKR.SMALL_BOX)
+        if self.gridopt is not None and not self.gridopt.general and (not staged or self.gridopt.box <= 3):
+            self.gridopt.jl = 0
         self.rr = self.gridopt if self.gridopt is not None else self.staged_k
         self.kq = self.gridopt_q if self.gridopt_q is not None else self.staged_q
         # split-BF16: the contractions that are not staged run on pre-packed operands. The "el" tensor is
@@ -1020,7 +1024,7 @@ class _GridOptKR:
         self.rmin = [int(x) for x in lo]
         # one lane per (operator column, j) where the box is symmetric along axes 2 and 3: j padded to 4, 8 or 16 lanes
         self.jl = 0
-        if (st.nw <= 16 and (self.mfma or self.general) and self.np in (3, 5, 7)
+        if (st.nw <= 16 and (self.mfma or self.general) and self.np in (3, 5, 7) and nd // st.nw < 1 << 25
                 and self.rmin[1] == self.rmin[2] == -(self.np // 2)):
             self.jl = 4 if st.nw <= 4 else 8 if st.nw <= 8 else 16
         rmap = -np.ones((self.n3, self.n2, self.n1), np.int32)
@@ -1055,7 +1059,7 @@ class _GridOptKR:
     def use_general(self):
         """Take the general form (ephip_staged_project) in place of the VALU projection."""
         self.general, self._nb = True, 1
-        if self.np in (3, 5, 7) and self.rmin[1] == self.rmin[2] == -(self.np // 2):
+        if self.np in (3, 5, 7) and self.nd // 8 < 1 << 25 and self.rmin[1] == self.rmin[2] == -(self.np // 2):
             self.jl = 8
 
     def lanes(self) -> bool:

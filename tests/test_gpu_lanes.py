@@ -64,3 +64,16 @@ def test_lane_project(nw, rest, np_, lines, lda_pad):
         # in both parts; phases and their products rounded once each
         tol = 2 * (2 * np_ + 8 + nw) * 2.0 ** -24 * size
         assert (abs(got[u, :ng] - ref) <= tol).all(), (u, abs(got[u, :ng] - ref).max(), tol.min())
+
+
+@pytest.mark.parametrize("box,staged,lanes", [(3, True, False), (5, True, True), (5, False, False)])
+def test_lane_rule_keeps_the_digits_of_fp64_consumers(backend, box, staged, lanes):
+    """27-R boxes and loops without the general staged kernels feed FP64 rates: same projection kernel as ever."""
+    from ephip import _lib as L
+    from ephip import eph
+    from ephip import model as M
+    m = M.make_model(nw=16, natoms=1, box_hd=3, box_g=box, seed=5, g_dtype=np.complex64)
+    st = eph.setup_outer_q(m, (3, 3, 3), (3, 3, 3), (-0.3, 0.3), backend)
+    assert 1 <= st.nbw <= 4
+    loop = eph.OuterKLoop(st, nk_batch=8, staged=staged, precision=L.PREC_FP32)
+    assert loop.rr.mfma and loop.rr.lanes() is lanes
