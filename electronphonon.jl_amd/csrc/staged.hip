@@ -5,7 +5,7 @@
 //   * RR->kR with the k-side projection: 16 operator columns per workgroup, four j per wave on FP32 MFMAs, one
 //     launch for all k1 planes of a batch;
 //   * kR->kq with the rotations and g2: one thread per pair of (kept q, window band) slots of one q line.
-#include "common.hpp"
+#include "lanes.hpp"
 
 namespace ephip {
 
@@ -631,6 +631,214 @@ __global__ __launch_bounds__(512) void staged_kq_kernel(SqArgs a) {
     }
 }
 
+// The same in the lane-private form of lanes.hpp (nw <= 16, nm <= 16, boxes that span -h .. h): a lane is one
+// (mode, i), a wave 64 / JL modes. Stage 1 ends in the lane's registers; stage 2 forms four q2 lines at a time and
+// stage 3 four entries (kept q, window band) of a line, both as 4x4x1 MFMAs; the product with U and the sum over i run
+// on the VALU and leave t in LDS for the phonon rotation. The tables of the slab are laid down once; U columns and
+// stage-3 rows are staged for at most LQ_ENT entries of the four lines, in equal parts.
+// ms, staged_kq_kernel -> this: 16 orbitals, 12 modes, 5^3 boxes, 5 window bands, q 8^3, 10505 units 8.7 -> 5.0 (5.9 with
+// parts of 64 and the row of u_ph read as it was used; 5.5 at four waves a SIMD, which spill); 12 orbitals, 9 modes,
+// q 18 x 15 x 12, 1260 units 1.09 -> 0.82. Whole passes: 12, 12, 5^3, q 16^3, 3 bands 12.3 -> 4.5; 10, 15, q 20^3
+// 5.6 -> 2.7; 12, 12, 7^3, q 12^3 3.56 -> 3.25. Waves wait for the staging and its barriers 55% of their time; VALU
+// 45% busy, MFMAs 9%.
+constexpr int LQ_ENT = 96, LQ_TP = 18, LQ_SLAB = 4096;  // LQ_SLAB: words of the tables of a slab
+
+__host__ inline size_t lq_lds_bytes(const SqArgs &a, int jl) {
+    return sizeof(float) * LP_STEPS * (size_t)(a.m2 + a.m3 + LQ_ENT + 4) +
+           sizeof(float2) * (size_t)(LQ_ENT + 4) * (jl + LQ_TP) + sizeof(int) * ((4 + (size_t)a.nbw) * a.m2 * a.m3 + a.m2 + 2);
+}
+
+template <int N, int JL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N == 7 ? 2 : N == 5 ? 3 : 4))) void lane_kq_kernel(
+    SqArgs a) {
+    constexpr int NE = (N + 1) & ~1, H = N / 2, CL = 64 / JL;
+    extern __shared__ float4 sq_lds[];
+    const int nw = a.nw, nm = a.nm, m2 = a.m2, m3 = a.m3, slab = m2 * m3;
+    float2 *tq = reinterpret_cast<float2 *>(sq_lds);         // [LQ_ENT + 4][LQ_TP]
+    float2 *us = tq + (LQ_ENT + 4) * LQ_TP;                  // [LQ_ENT + 4][JL]: conj U_kq
+    float *c2t = reinterpret_cast<float *>(us + (LQ_ENT + 4) * JL), *c3t = c2t + LP_STEPS * m2;
+    float *c3e = c3t + LP_STEPS * m3;                        // [LQ_ENT + 4]: stage-3 row of an entry
+    int *skq = reinterpret_cast<int *>(c3e + LP_STEPS * (LQ_ENT + 4));  // k+q state of a kept q
+    int *siq = skq + slab, *smeta = siq + slab;              // q; window bands | first band << 8 | q3 << 16
+    int *eoff = smeta + slab;                                // [slab + 1] first entry of a kept q
+    int *slo = eoff + slab + 1;                              // [m2 + 1] first kept q of a line
+    int *ent = slo + m2 + 1;                                 // [slab nbw] entry -> kept q | band << 16
+    const int t = threadIdx.x, bd = blockDim.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // runs of (unit, q1) pairs go to one XCD, as in staged_kq_kernel
+    const int64_t T = (int64_t)gridDim.x * gridDim.y, L = blockIdx.x + (int64_t)gridDim.x * blockIdx.y;
+    const int64_t xc = L & 7, base = T >> 3, rem = T & 7, id = xc * base + (xc < rem ? xc : rem) + (L >> 3);
+    const int u = (int)(id / gridDim.x), q1 = (int)(id - (int64_t)u * gridDim.x);
+    const int *lo_u = a.line_off + (int64_t)u * (a.m1 * m2 + 1) + q1 * m2;
+    const int sb = lo_u[0], n = lo_u[m2] - sb;
+    if (n <= 0) return;  // uniform; n <= slab
+    const int64_t row0 = (int64_t)u * a.cs + sb;
+    for (int kk = t; kk < n; kk += bd) {
+        const int kq = a.ikq[row0 + kk], iq = a.col_index[row0 + kk];
+        const int b0 = (int)a.bmin[kq], b1 = (int)a.bmax[kq];
+        skq[kk] = kq;
+        siq[kk] = iq;
+        smeta[kk] = (b0 > 0 ? min(b1 - b0 + 1, a.nbw) | ((b0 - 1) << 8) : 0) | ((iq % m3) << 16);
+    }
+    for (int l = t; l <= m2; l += bd) slo[l] = lo_u[l] - sb;
+    for (int e = t; e < LP_STEPS * (m2 + m3); e += bd) {  // (1, cos, sin) of the q2 and q3
+        const int f = e / LP_STEPS, s = e % LP_STEPS;
+        const float2 *ph = f < m2 ? a.e2 + f * NE : a.e3 + (f - m2) * NE;
+        c2t[e] = s == 0 ? 1.f : s <= H ? ph[H + s].x : s <= 2 * H ? ph[s].y : 0.f;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int run = 0;
+        for (int k0 = 0; k0 < n; k0 += 64) {
+            const int v = k0 + lane < n ? smeta[k0 + lane] & 0xff : 0;
+            int p = v;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int o = __shfl_up(p, off, 64);
+                if (lane >= off) p += o;
+            }
+            if (k0 + lane < n) eoff[k0 + lane] = run + p - v;
+            for (int m = 0; m < v; m++) ent[run + p - v + m] = (k0 + lane) | (m << 16);
+            run += __builtin_amdgcn_readlane(p, 63);
+        }
+        if (lane == 0) eoff[n] = run;
+    }
+    const int j = lane / CL, nu = wave * CL + lane % CL;
+    const bool ok = j < nw && nu < nm;
+    const int r0 = ok ? j + nw * nu : 0;
+    const cplx<float> *au = a.A + (int64_t)u * a.lda;
+    const float2 *e1 = a.e1 + q1 * a.n1;
+    float xr[N][N], xi[N][N];
+#pragma unroll
+    for (int c = 0; c < N; c++) {
+        float br[N], bi[N];
+#pragma unroll
+        for (int b = 0; b < N; b++) br[b] = bi[b] = 0.f;
+#pragma unroll
+        for (int x = 0; x < N; x++)
+#pragma unroll
+            for (int b = 0; b < N; b++) {  // absent R: column 0 loaded, zero used
+                const int ir = a.rmap[b + 8 * (x + N * c)];  // uniform; the N entries are contiguous
+                const cplx<float> v = au[(int64_t)a.ldr * max(ir, 0) + r0];
+                const float kr = ir >= 0 ? v.re : 0.f, ki = ir >= 0 ? v.im : 0.f;
+                st_cmac(br[b], bi[b], e1[x].x, e1[x].y, kr, ki);
+            }
+#pragma unroll
+        for (int b = 0; b < N; b++) {
+            br[b] = ok ? br[b] : 0.f;
+            bi[b] = ok ? bi[b] : 0.f;
+        }
+        lp_fold<N>(xr[c], xi[c], br, bi);
+        __builtin_amdgcn_sched_barrier(0);  // one c's loads in flight: all of them would spill
+    }
+    __syncthreads();  // eoff, ent
+    const int row = lane & 3, step = (lane >> 2) & (LP_STEPS - 1);
+    float2 *tl = tq + (lane >> 4) * LQ_TP + wave * CL + (lane & (CL - 1));
+    for (int l = 0; l < m2; l += 4) {
+        const int ka = __builtin_amdgcn_readfirstlane(slo[l]), kz = __builtin_amdgcn_readfirstlane(slo[min(l + 4, m2)]);
+        if (ka == kz) continue;  // uniform
+        const int ea = __builtin_amdgcn_readfirstlane(eoff[ka]), ez = __builtin_amdgcn_readfirstlane(eoff[kz]);
+        const float mc2 = c2t[LP_STEPS * min(l + row, m2 - 1) + step];
+        f32x4 tr[N], ti[N];  // stage 2 of four lines, before the fold over c
+#pragma unroll
+        for (int c = 0; c < N; c++) lp_apply<N>(tr[c], ti[c], mc2, xr[c], xi[c]);
+        // the entries of the four lines in equal parts of at most LQ_ENT
+        const int parts = (ez - ea + LQ_ENT - 1) / LQ_ENT, part = (ez - ea + parts - 1) / parts;
+        for (int cb = ea; cb < ez; cb += part) {
+            const int ce = min(cb + part, ez);
+            __syncthreads();  // the last entries' tables no longer read
+            for (int e0 = t; e0 < (ce - cb) * JL; e0 += 4 * bd) {  // four loads in flight
+                cplx<float> v[4];
+#pragma unroll
+                for (int y = 0; y < 4; y++) {
+                    const int e = min(e0 + y * bd, (ce - cb) * JL - 1), s = ent[cb + e / JL], kk = s & 0xffff, jj = min(e % JL, nw - 1);
+                    v[y] = a.U[(int64_t)nw * nw * skq[kk] + jj + nw * (((smeta[kk] >> 8) & 0xff) + (s >> 16))];
+                }
+#pragma unroll
+                for (int y = 0; y < 4; y++) {
+                    const int e = e0 + y * bd;
+                    if (e < (ce - cb) * JL) us[e] = e % JL < nw ? make_float2(v[y].re, -v[y].im) : make_float2(0.f, 0.f);
+                }
+            }
+            for (int e = t; e < (ce - cb) * LP_STEPS; e += bd)
+                c3e[e] = c3t[LP_STEPS * (smeta[ent[cb + e / LP_STEPS] & 0xffff] >> 16) + e % LP_STEPS];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (l + r >= m2) break;
+                const int es = max(cb, __builtin_amdgcn_readfirstlane(eoff[slo[l + r]]));
+                const int ee = min(ce, __builtin_amdgcn_readfirstlane(eoff[slo[l + r + 1]]));
+                if (es >= ee) continue;
+                float br[N], bi[N], zr[N], zi[N];
+#pragma unroll
+                for (int c = 0; c < N; c++) {
+                    br[c] = tr[c][r];
+                    bi[c] = ti[c][r];
+                }
+                lp_fold<N>(zr, zi, br, bi);
+                float m = c3e[(es - cb + row) * LP_STEPS + step];
+                float2 w = us[(es - cb + row) * JL + j];
+                for (int e = es - cb; e < ee - cb; e += 4) {
+                    const float mm = m;
+                    const float2 ww = w;
+                    const int nx = min(e + 4, LQ_ENT);  // rows past the line are formed and written, then written over
+                    m = c3e[(nx + row) * LP_STEPS + step];
+                    w = us[(nx + row) * JL + j];
+                    f32x4 gr, gi;
+                    lp_apply<N>(gr, gi, mm, zr, zi);
+                    float vr[4], vi[4];
+                    lp_times<0>(vr[0], vi[0], ww.x, ww.y, gr[0], gi[0]);
+                    lp_times<1>(vr[1], vi[1], ww.x, ww.y, gr[1], gi[1]);
+                    lp_times<2>(vr[2], vi[2], ww.x, ww.y, gr[2], gi[2]);
+                    lp_times<3>(vr[3], vi[3], ww.x, ww.y, gr[3], gi[3]);
+                    tl[e * LQ_TP] = make_float2(lp_reduce<JL>(vr), lp_reduce<JL>(vi));
+                }
+            }
+            __syncthreads();  // t of the entries
+            for (int e = t; e < (ce - cb) * nm; e += bd) {
+                const int x = sq_div(e, a.mg_nm), n2 = e - x * nm, s = ent[cb + x], kk = s & 0xffff;
+                const int64_t col = (int64_t)nm * siq[kk] + n2;
+                const float2 *uv = reinterpret_cast<const float2 *>(a.uph) + col * nm;
+                const float w2 = 2.f * static_cast<float>(a.omega[col]);
+                const float2 *tv = tq + x * LQ_TP;
+                float er = 0.f, ei = 0.f;
+                for (int y0 = 0; y0 < nm; y0 += 12) {  // the row of u_ph, its loads in flight together
+                    float4 p[6];
+#pragma unroll
+                    for (int y = 0; y < 6; y++) {
+                        const int k = y0 + 2 * y;
+                        if (k >= nm) break;
+                        if (nm & 1) {  // t of the mode past the last is zero
+                            const float2 f = uv[k], g = uv[min(k + 1, nm - 1)];
+                            p[y] = make_float4(f.x, f.y, g.x, g.y);
+                        } else {
+                            p[y] = *reinterpret_cast<const float4 *>(uv + k);
+                        }
+                    }
+#pragma unroll
+                    for (int y = 0; y < 6; y++) {
+                        const int k = y0 + 2 * y;
+                        if (k >= nm) break;
+                        const float4 q = *reinterpret_cast<const float4 *>(tv + k);
+                        st_cmac(er, ei, q.x, q.y, p[y].x, p[y].y);
+                        st_cmac(er, ei, q.z, q.w, p[y].z, p[y].w);
+                    }
+                }
+                const int64_t oi = ((row0 + kk) * a.nbw + (s >> 16)) * nm + n2;
+                a.g2[oi] = (er * er + ei * ei) / w2;
+                if (a.ep) a.ep[oi] = make_float2(er, ei);
+            }
+        }
+        for (int m = 0; m < a.nbw; m++)  // zeros past the k+q window
+            for (int e = t; e < (kz - ka) * nm; e += bd) {
+                const int x = sq_div(e, a.mg_nm), n2 = e - x * nm;
+                if (m < (smeta[ka + x] & 0xff)) continue;
+                const int64_t oi = ((row0 + ka + x) * a.nbw + m) * nm + n2;
+                a.g2[oi] = 0.f;
+                if (a.ep) a.ep[oi] = make_float2(0.f, 0.f);
+            }
+    }
+}
+
 // e^{2 pi i (x / m) (pmin + b)} for x < m, b < n (zero for n <= b < ne)
 __global__ void staged_phases_kernel(int m, int n, int ne, int pmin, float2 *__restrict__ out) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -767,6 +975,14 @@ static int staged_kq_launch_form(SqArgs a, int nunits, double entries, hipStream
     return EPHIP_OK;
 }
 
+template <int N>
+static int lane_kq_launch(SqArgs a, int nunits, hipStream_t st) {
+    a.mg_nm = sq_magic(a.nm);
+    lane_kq_kernel<N, 16><<<dim3((unsigned)a.m1, (unsigned)nunits), 64 * ((a.nm + 3) / 4), lq_lds_bytes(a, 16), st>>>(a);
+    EPHIP_LAUNCHED();
+    return EPHIP_OK;
+}
+
 // Form by the mean window width w (bands per kept q): two kept q per thread while most windows hold one band
 // (a band's g is then formed for itself), else one kept q with up to 2 or 4 of its bands, which share g.
 template <int N, bool SYM>
@@ -813,6 +1029,15 @@ extern "C" int ephip_staged_kq(int32_t nw, int32_t nm, int32_t nbw, int32_t nuni
     a.uph = static_cast<const cplx<float> *>(uph), a.omega = omega, a.g2 = g2, a.ep = static_cast<float2 *>(ep);
     const bool sym = (np & 1) && n1 == np && p1min == -(np / 2) && p2min == -(np / 2) && p3min == -(np / 2);
     hipStream_t st = as_stream(stream);
+    // One lane per (mode, i): from 9 modes on, where a workgroup has three waves or four. With one or two the tables of a
+    // slab, read in turn, take too long: whole passes of 9 orbitals, 3 modes 0.52 -> 0.83 ms, 10, 6 (7^3 boxes) 1.33 ->
+    // 1.35; and at 8 lanes per mode 8, 6 84 -> 91 us. Slabs whose tables pass LQ_SLAB words (16 KB) would leave two
+    // workgroups a CU.
+    if (sym && nw > 8 && nw <= 16 && nm > 8 && nm <= 16 && (4 + nbw) * a.m2 * a.m3 <= LQ_SLAB) {
+        if (np == 3) return lane_kq_launch<3>(a, nunits, st);
+        if (np == 5) return lane_kq_launch<5>(a, nunits, st);
+        return lane_kq_launch<7>(a, nunits, st);
+    }
     if (sym) {
         if (np == 3) return staged_kq_launch<3, true>(a, nunits, cols_hint, width_hint, st);
         if (np == 5) return staged_kq_launch<5, true>(a, nunits, cols_hint, width_hint, st);
