@@ -981,6 +981,11 @@ class OuterKLoop:
             self.run_kbatch(i0, min(self.nk_batch, k_stop - i0), calculators)
 
 
+def _repeats(r) -> bool:
+    """The list names an R more than once. The direct sums add both; a box's index map holds one column per R."""
+    return len(np.unique(r, axis=0)) < len(r)
+
+
 class _GridOptKR:
     """Staged RR->kR over Re (ephip_gridopt_stage1_planes + ephip_lane_project where the box is symmetric along axes
     2 and 3 and nw <= 16, else ephip_gridopt_kR_project[_mfma] or ephip_staged_project), the device
@@ -1003,6 +1008,8 @@ class _GridOptKR:
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         kg = np.asarray(st.kgrid, dtype=np.int64)
+        if _repeats(r):
+            return None
         if (len(ks) == 0 or n[0] > cls.N1_MAX or n[1] > cls.N23_MAX or n[2] > cls.N23_MAX
                 or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)):
             return None
@@ -1206,7 +1213,7 @@ class _GridOptKQ:
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         m = np.asarray(st.qgrid, dtype=np.int64)
-        if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535:
+        if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535 or _repeats(r):
             return None
         if general and (st.nw > 32 or st.nm > 48 or n.max() <= _GridOptKR.SMALL_BOX):
             return None
