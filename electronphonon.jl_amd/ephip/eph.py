@@ -1055,8 +1055,8 @@ class _GridOptKR:
         cum = np.concatenate([[0], np.cumsum(nb_k)])
         self.max_line_units = int((cum[starts[1:]] - cum[starts[:-1]]).max())  # units of the fullest line
         x1 = st.el.xk.index_select(0, st.ksurv).cpu().numpy()[:, 0]
-        # planes with surviving k in order, their k1 coordinates, and the stage-1 group of each
-        first_line = np.flatnonzero(np.concatenate([[True], np.diff(self.line_plane) != 0]))
+        # planes with surviving k in order of their first one, their k1 coordinates, and the stage-1 group of each
+        first_line = np.sort(np.unique(self.line_plane, return_index=True)[1])
         self.planes = [int(p) for p in self.line_plane[first_line]]
         self.plane_x1 = {p: float(x1[starts[l]]) for p, l in zip(self.planes, first_line)}
         self.plane_pos = {p: i for i, p in enumerate(self.planes)}
@@ -1153,9 +1153,10 @@ class _GridOptKR:
         lines = [(int(planes[a]), l_first + int(a), l_first + int(b)) for a, b in zip(cut[:-1], cut[1:])]
         while lines:
             g = self.plane_pos[lines[0][0]] // self.PLANES
-            part = [x for x in lines if self.plane_pos[x[0]] // self.PLANES == g]
-            lines = lines[len(part):]
-            m = len(part)
+            m = 1   # runs of lines of one group, at most a launch's planes; k in another order come back to a plane
+            while m < min(len(lines), self.PLANES) and self.plane_pos[lines[m][0]] // self.PLANES == g:
+                m += 1
+            part, lines = lines[:m], lines[m:]
             op1 = (C.c_void_p * m)(*[L.ptr(self._plane_buffer(p, loop.epmat_el, stream)) for p, _, _ in part])
             la, lz = (C.c_int32 * m)(*[x[1] for x in part]), (C.c_int32 * m)(*[x[2] for x in part])
             if lanes:

@@ -59,3 +59,47 @@ def test_repeated_R_takes_the_direct_sums(nw, general):
     assert _kr(_setup(nw, re=twice), general=general) is None
     assert eph._GridOptKQ.build(_setup(nw, re=r), general=general) is not None
     assert eph._GridOptKQ.build(_setup(nw, re=r, rp=twice), general=general) is None
+
+
+@pytest.mark.parametrize("nw,general", [(9, True), (16, False)])
+@pytest.mark.parametrize("order", ["grid", "shuffled", "two_passes"])
+def test_projection_covers_every_line_in_any_order_of_k(monkeypatch, nw, general, order):
+    """Each line of the surviving k goes to one launch, from its own plane's sums, whatever the order of the k."""
+    import ctypes as C
+    st = _setup(nw, 3, (19, 2, 3))
+    ks = np.arange(19 * 6)
+    if order == "shuffled":
+        np.random.default_rng(1).shuffle(ks)
+    elif order == "two_passes":
+        ks = np.concatenate([ks[::2], ks[1::2]])
+    st.ksurv = torch.from_numpy(ks)
+    go = _kr(st, general=general)
+    assert go.lanes()
+    nk, nb = len(ks), st.nbw
+    k_units = torch.arange(nk + 1, dtype=torch.int32) * nb
+    loop = types.SimpleNamespace(st=st, xk_surv=st.el.xk[st.ksurv], k_unit_start_dev=k_units,
+                                 unit_kpos=torch.zeros(nk * nb, dtype=torch.int32),
+                                 unit_state=torch.zeros(nk * nb, dtype=torch.int64),
+                                 unit_band=torch.zeros(nk * nb, dtype=torch.int32), max_units=nk * nb, nk_batch=nk,
+                                 epmat_el=torch.zeros((len(st.irvec_el_dev), go.nd), dtype=torch.complex64))
+    holds, done = {}, []                                # plane coordinate of each buffer, lines projected
+
+    def call(name, *a):
+        if name == "ephip_gridopt_stage1_planes":
+            n = a[9]
+            x1 = (C.c_double * n).from_address(a[10])
+            out = (C.c_void_p * n).from_address(a[12])
+            holds.update({out[p]: x1[p] for p in range(n)})
+        elif name == "ephip_lane_project":
+            m = a[4]
+            op1, la, lz = ((t * m).from_address(x) for t, x in zip((C.c_void_p, C.c_int32, C.c_int32), a[5:8]))
+            assert 1 <= m <= 8
+            for p in range(m):
+                for line in range(la[p], lz[p]):
+                    k = int(go.line_start_host[line])
+                    assert holds[op1[p]] == float(loop.xk_surv[k, 0])
+                    done.append(line)
+
+    monkeypatch.setattr(eph.L, "call", call)
+    go.run(loop, 0, nk, 0, nk * nb, torch.zeros((nk * nb, 1), dtype=torch.complex64), None)
+    assert sorted(done) == list(range(len(go.line_start_host) - 1))
