@@ -986,6 +986,12 @@ def _repeats(r) -> bool:
     return len(np.unique(r, axis=0)) < len(r)
 
 
+def _differ(a, b) -> bool:
+    """Some coordinates differ by more than whole cells (and what FP32 phases resolve)."""
+    d = np.asarray(a) - b
+    return bool(np.abs(d - np.rint(d)).max(initial=0.0) > 1e-10)
+
+
 class _GridOptKR:
     """Staged RR->kR over Re (ephip_gridopt_stage1_planes + ephip_lane_project where the box is symmetric along axes
     2 and 3 and nw <= 16, else ephip_gridopt_kR_project[_mfma] or ephip_staged_project), the device
@@ -1013,9 +1019,16 @@ class _GridOptKR:
         if (len(ks) == 0 or n[0] > cls.N1_MAX or n[1] > cls.N23_MAX or n[2] > cls.N23_MAX
                 or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)):
             return None
-        return cls(st, ks, nd, r, lo, n, kg, mfma, general)
+        x = st.el.xk.index_select(0, st.ksurv).cpu().numpy()
+        i1, i2 = ks // (kg[1] * kg[2]), (ks // kg[2]) % kg[1]
+        for c, at in ((0, i1), (1, i1 * kg[1] + i2)):   # one coordinate per plane and per line
+            of = np.zeros(int(at.max()) + 1)
+            of[at] = x[:, c]
+            if _differ(x[:, c], of[at]):
+                return None
+        return cls(st, ks, nd, r, lo, n, kg, x[:, 0], mfma, general)
 
-    def __init__(self, st, ks, nd, r, lo, n, kg, mfma, general=False):
+    def __init__(self, st, ks, nd, r, lo, n, kg, x1, mfma, general=False):
         torch = _torch()
         dev = st.el.xk.device
         self.nd = self.nd_max = nd   # rows in use, and what the plane buffers hold
@@ -1054,7 +1067,6 @@ class _GridOptKR:
         nb_k = (st.el.filt.band_max.cpu().numpy()[ks] - st.el.filt.band_min.cpu().numpy()[ks] + 1).astype(np.int64)
         cum = np.concatenate([[0], np.cumsum(nb_k)])
         self.max_line_units = int((cum[starts[1:]] - cum[starts[:-1]]).max())  # units of the fullest line
-        x1 = st.el.xk.index_select(0, st.ksurv).cpu().numpy()[:, 0]
         # planes with surviving k in order of their first one, their k1 coordinates, and the stage-1 group of each
         first_line = np.sort(np.unique(self.line_plane, return_index=True)[1])
         self.planes = [int(p) for p in self.line_plane[first_line]]
@@ -1215,6 +1227,9 @@ class _GridOptKQ:
         n = hi - lo + 1
         m = np.asarray(st.qgrid, dtype=np.int64)
         if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535 or _repeats(r):
+            return None
+        xq = st.ph.xq.cpu().numpy()   # the grid's points in its order, third index fastest
+        if len(xq) != m.prod() or _differ(xq, np.stack(np.unravel_index(np.arange(len(xq)), m), axis=1) / m):
             return None
         if general and (st.nw > 32 or st.nm > 48 or n.max() <= _GridOptKR.SMALL_BOX):
             return None

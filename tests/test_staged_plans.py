@@ -103,3 +103,26 @@ def test_projection_covers_every_line_in_any_order_of_k(monkeypatch, nw, general
     monkeypatch.setattr(eph.L, "call", call)
     go.run(loop, 0, nk, 0, nk * nb, torch.zeros((nk * nb, 1), dtype=torch.complex64), None)
     assert sorted(done) == list(range(len(go.line_start_host) - 1))
+
+
+@pytest.mark.parametrize("nw,general", [(12, True), (16, False)])
+def test_points_off_the_grid_take_the_direct_sums(nw, general):
+    """kR->kq takes the q from their place in the grid, RR->kR a plane's and a line's coordinate from one k."""
+    def plans(st):
+        return _kr(st, general=general) is not None, eph._GridOptKQ.build(st, general=general) is not None
+
+    assert plans(_setup(nw)) == (True, True)
+    st = _setup(nw)
+    st.ph.xq, st.el.xk = st.ph.xq - 1.0, st.el.xk + torch.tensor([0.01, 0.02, 0.03])   # whole cells; a shift of all k
+    assert plans(st) == (True, True)
+    st = _setup(nw)
+    st.ph.xq = st.ph.xq + torch.tensor([0.0, 0.0, 0.1])
+    assert plans(st) == (True, False)
+    for some in (slice(0, 7), torch.randperm(96, generator=torch.Generator().manual_seed(0))):  # some q, another order
+        st = _setup(nw)
+        st.ph.xq = st.ph.xq[some]
+        assert plans(st) == (True, False)
+    for axis, ok in ((0, False), (1, False), (2, True)):   # one k off its plane, off its line, elsewhere on its line
+        st = _setup(nw)
+        st.el.xk[10, axis] += 0.05
+        assert plans(st) == (ok, True)
