@@ -384,7 +384,8 @@ __global__ __launch_bounds__(512) void staged_kq_kernel(SqArgs a) {
                 const int o = __shfl_up(tot, off, 64);
                 if (lane >= off) tot += o;
             }
-            // a column is taken while entries + lines <= NQ tb (so tasks <= tb) and lines <= ls: a prefix of them
+            // a column is taken while entries + lines <= NQ tb (so tasks <= tb) and lines <= ls: a prefix of them, and
+            // at least one (sq_choose)
             int taken = 0, end = 0;
             bool in[SQ_CPL];
 #pragma unroll
@@ -914,13 +915,28 @@ extern "C" int ephip_staged_project(int32_t nw, int64_t ngcol, int32_t np, int32
     return EPHIP_OK;
 }
 
-template <int N, bool SYM, int NQ, int NB>
-static int staged_kq_launch_form(SqArgs a, int nunits, double entries, hipStream_t st) {
+// Form by the mean window width w (bands per kept q): two kept q per thread while most windows hold one band
+// (a band's g is then formed for itself), else one kept q with up to 2 or 4 of its bands, which share g.
+struct SqForm {
+    int nq, nb;      // kept q of a thread, bands of each
+    double entries;  // expected entries of one (unit, q1) slab
+};
+static SqForm sq_form(int nw, double cols, double width) {
+    if (width < 1.4) return SqForm{2, 1, cols * width};
+    if (width < 1.9 || nw > 16) return SqForm{1, 2, cols * (0.5 + 0.5 * width)};
+    return SqForm{1, 4, cols * (width < 3.0 ? 1.05 : 0.3 + 0.25 * width)};
+}
+
+// The workgroup: a.tb, a.nug, a.ls and a.split; false if none fits.
+template <int N>
+static bool sq_choose(SqArgs &a, const SqForm f) {
     const size_t cu_lds = 160 * 1024, most = 152 * 1024;
     // threads of a group: NQ entries each; room for the entries and lines of most slabs (a slab past it takes a
     // second segment, which repeats stages 1 and 2)
-    const double want = (1.15 * entries + (NQ > 1 ? a.m2 : 0.0)) / NQ;
-    const int tb_want = max(16, min(128, (int)(want / 8 + 1) * 8));
+    const double want = fmin(1024.0, (1.15 * f.entries + (f.nq > 1 ? a.m2 : 0.0)) / f.nq);
+    // never fewer than the entries of one kept q with nbw bands take, and its line (17 threads of two for 32 bands)
+    const int tb_min = max(16, ((a.nbw + f.nb - 1) / f.nb + (f.nq > 1) + f.nq - 1) / f.nq);
+    const int tb_want = max((tb_min + 7) & ~7, min(128, (int)(want / 8 + 1) * 8));
     // (group size, mode groups): a workgroup is a chain of latencies, about a quarter of it per pass over nug modes,
     // so the number of workgroups a CU holds (LDS; registers: U takes 2 NQ NB nw of them) over that length counts.
     // Measured, ms per pass: 4 orbitals, 3 modes, 7^3 boxes, q 24^3: 1.38 at 6 workgroups and 3 passes, 1.77 at 4 and
@@ -929,22 +945,22 @@ static int staged_kq_launch_form(SqArgs a, int nunits, double entries, hipStream
     double best = -1.0;
     SqArgs c = a;
     const int nwt = a.nw <= 4 ? 4 : a.nw <= 8 ? 8 : a.nw <= 12 ? 12 : a.nw <= 16 ? 16 : 32;
-    const int simd_waves = max(1, min(4, 512 / (2 * NQ * NB * nwt + 72)));
-    for (int tb = tb_want; tb >= 16; tb -= 16)
+    const int simd_waves = max(1, min(4, 512 / (2 * f.nq * f.nb * nwt + 72)));
+    for (int tb = tb_want; tb >= tb_min; tb -= 16)
         for (int nug = 1; nug <= min(a.nm, 512 / tb); nug++) {
             a.tb = tb;
             a.nug = nug;
             a.ls = min(a.m2, SQ_LINES);
-            while (sq_lds_bytes<N>(a, NQ, NB) > cu_lds / 2 && a.ls > 8) a.ls--;
-            while (sq_lds_bytes<N>(a, NQ, NB) > most && a.ls > 1) a.ls--;
-            const size_t lds = sq_lds_bytes<N>(a, NQ, NB);
+            while (sq_lds_bytes<N>(a, f.nq, f.nb) > cu_lds / 2 && a.ls > 8) a.ls--;
+            while (sq_lds_bytes<N>(a, f.nq, f.nb) > most && a.ls > 1) a.ls--;
+            const size_t lds = sq_lds_bytes<N>(a, f.nq, f.nb);
             if (lds > most || N * N * nug * a.nw >= 65536) continue;
             const int rounds = (a.nm + nug - 1) / nug, waves = (tb * nug + 63) / 64;
             const int blocks = min((int)(cu_lds / lds), simd_waves / ((waves + 3) / 4) * (waves < 4 ? 4 / waves : 1));
             const double s = blocks / (1.0 + 0.25 * rounds) * tb / tb_want * (waves == 1 ? 0.8 : 1.0);
             if (s > best) best = s, c = a;
         }
-    EPHIP_REQUIRE(best > 0.0, "staged_kq: nw=%d nm=%d nbw=%d do not fit a workgroup", a.nw, a.nm, a.nbw);
+    if (best <= 0.0) return false;
     a = c;
     const int bd = (a.tb * a.nug + 63) & ~63, rows = a.nug * a.nw;
     // stage 2: (row, c) items split over the lines so that the threads have equal shares
@@ -958,6 +974,13 @@ static int staged_kq_launch_form(SqArgs a, int nunits, double entries, hipStream
             a.split = s;
         }
     }
+    return true;
+}
+
+template <int N, bool SYM, int NQ, int NB>
+static int staged_kq_launch_form(SqArgs a, int nunits, const SqForm f, hipStream_t st) {
+    EPHIP_REQUIRE(sq_choose<N>(a, f), "staged_kq: nw=%d nm=%d nbw=%d do not fit a workgroup", a.nw, a.nm, a.nbw);
+    const int bd = (a.tb * a.nug + 63) & ~63, rows = a.nug * a.nw;
     a.mg_rows = sq_magic(rows);
     a.mg_rn = sq_magic(N * rows);
     a.mg_nm = sq_magic(a.nm);
@@ -983,13 +1006,32 @@ static int lane_kq_launch(SqArgs a, int nunits, hipStream_t st) {
     return EPHIP_OK;
 }
 
-// Form by the mean window width w (bands per kept q): two kept q per thread while most windows hold one band
-// (a band's g is then formed for itself), else one kept q with up to 2 or 4 of its bands, which share g.
 template <int N, bool SYM>
 static int staged_kq_launch(const SqArgs &a, int nunits, double cols, double width, hipStream_t st) {
-    if (width < 1.4) return staged_kq_launch_form<N, SYM, 2, 1>(a, nunits, cols * width, st);
-    if (width < 1.9 || a.nw > 16) return staged_kq_launch_form<N, SYM, 1, 2>(a, nunits, cols * (0.5 + 0.5 * width), st);
-    return staged_kq_launch_form<N, SYM, 1, 4>(a, nunits, cols * (width < 3.0 ? 1.05 : 0.3 + 0.25 * width), st);
+    const SqForm f = sq_form(a.nw, cols, width);
+    if (f.nq == 2) return staged_kq_launch_form<N, SYM, 2, 1>(a, nunits, f, st);
+    if (f.nb == 2) return staged_kq_launch_form<N, SYM, 1, 2>(a, nunits, f, st);
+    return staged_kq_launch_form<N, SYM, 1, 4>(a, nunits, f, st);
+}
+
+extern "C" int ephip_staged_kq_group(int32_t nw, int32_t nm, int32_t nbw, int32_t np, int32_t m2, int32_t m3,
+                                     double cols_hint, double width_hint, int32_t *group) {
+    EPHIP_REQUIRE(nw >= 1 && nw <= 32 && nm >= 1 && nm <= 48 && nbw >= 1 && nbw <= nw && np >= 3 && np <= 8 && m2 >= 1 &&
+                      m2 <= SQ_LINES && m3 >= 1 && m3 <= 64 && group,
+                  "staged_kq_group: bad sizes");
+    SqArgs a{};
+    a.nw = nw, a.nm = nm, a.nbw = nbw, a.m2 = m2, a.m3 = m3;
+    const SqForm f = sq_form(nw, cols_hint, width_hint);
+    const bool ok = np == 3   ? sq_choose<3>(a, f)
+                    : np == 4 ? sq_choose<4>(a, f)
+                    : np == 5 ? sq_choose<5>(a, f)
+                    : np == 6 ? sq_choose<6>(a, f)
+                    : np == 7 ? sq_choose<7>(a, f)
+                              : sq_choose<8>(a, f);
+    EPHIP_REQUIRE(ok, "staged_kq: nw=%d nm=%d nbw=%d do not fit a workgroup", nw, nm, nbw);
+    const int g[5] = {f.nq, f.nb, a.tb, a.nug, a.ls};
+    for (int i = 0; i < 5; i++) group[i] = g[i];
+    return EPHIP_OK;
 }
 
 extern "C" int ephip_staged_kq(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits, int32_t n1, int32_t np,

@@ -99,6 +99,7 @@ SIGNATURES = {
     "ephip_staged_rr_to_rq": [_i64, _i32, _i32, _i32, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp],
     "ephip_staged_rq_rotate": [_i32, _i32, _i32, _i32, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp,
                                _i64, _vp, _vp, _vp, _vp],
+    "ephip_staged_kq_group": [_i32, _i32, _i32, _i32, _i32, _i32, _d, _d, _vp],
     "ephip_staged_phases": [_i32, _i32, _i32, _i32, _vp, _vp],
     "ephip_staged_kq": [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp,
                         _i64, _vp, _vp, _vp, _vp, _vp, _vp, _d, _d, _vp, _vp, _vp],

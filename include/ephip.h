@@ -340,9 +340,13 @@ int ephip_gridopt_kq_rotate(int32_t nw, int32_t nm, int32_t nbw, int32_t nunits,
  *    A[u lda + g] = sum_j g(k_u)[j, g] U_u[j], u counted from kus[k0]; units of k0 <= k < k1.
  *  - ephip_staged_kq: ephip_gridopt_kq_rotate for those shapes (arguments and output as there, no pre-pass).
  *    cols_hint, width_hint: expected kept q of one (unit, q1) slab and window bands per kept q; they size the
- *    workgroups only. e1 (m1 rows of n1), e2 (m2 rows) and e3 (m3 rows of np rounded up to even): the q grid's
+ *    workgroups only. ephip_staged_kq_group (host only) gives the workgroup for them: group[0] kept q of a thread,
+ *    group[1] bands of each, group[2] threads of a mode group, group[3] mode groups, group[4] q2 lines at a time.
+ *    It holds at least one kept q with nbw bands. e1 (m1 rows of n1), e2 (m2 rows) and e3 (m3 rows of np rounded up to even): the q grid's
  *    phases along each axis, complex64, from ephip_staged_phases.
  *  - ephip_staged_phases: out[x ne + b] = e^{2 pi i (x / m) (pmin + b)} for x < m, b < n; zero for n <= b < ne. */
+int ephip_staged_kq_group(int32_t nw, int32_t nm, int32_t nbw, int32_t np, int32_t m2, int32_t m3, double cols_hint,
+                          double width_hint, int32_t *group);
 int ephip_staged_phases(int32_t m, int32_t n, int32_t ne, int32_t pmin, void *out, void *stream);
 int ephip_staged_project(int32_t nw, int64_t ngcol, int32_t np, int32_t r2min, int32_t nplanes,
                          const void *const *op1, const int32_t *l0, const int32_t *l1, int64_t k0, int64_t k1,
