@@ -295,6 +295,11 @@ class OuterQLoop:
 
     def run_qtile(self, iq0: int, nq: int, calculators=()):
         st = self.st
+        nq_all = st.ph.xq.shape[0]
+        if nq > self.nq_tile:
+            raise L.EphipError(f"tile of {nq} q: the loop's buffers hold {self.nq_tile}")
+        if iq0 < 0 or nq < 0 or iq0 + nq > nq_all:
+            raise IndexError(f"tile of {nq} q at {iq0}: there are {nq_all} q")
         if self.staged is not None:
             self.staged.run(self, iq0, nq)
             nks = st.ksurv.shape[0]

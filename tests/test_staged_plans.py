@@ -126,3 +126,19 @@ def test_points_off_the_grid_take_the_direct_sums(nw, general):
         st = _setup(nw)
         st.el.xk[10, axis] += 0.05
         assert plans(st) == (ok, True)
+
+
+@pytest.mark.parametrize("staged", [True, False])
+def test_outer_q_tile_past_the_last_q_is_refused(monkeypatch, staged):
+    """A tile reads its q, phonons and frequencies by position: it has to lie within the list and the buffers."""
+    st = _setup(3, 3, (4, 2, 3))
+    st.epmat.op_r = torch.zeros((1, 1))
+    loop = eph.OuterQLoop(st, nq_tile=8, staged=staged)
+    assert (loop.staged is not None) == staged
+    nq, calls = st.ph.xq.shape[0], []
+    monkeypatch.setattr(eph.L, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(eph, "get_eph_RR_to_Rq_batched", lambda *a, **k: calls.append("RR_to_Rq"))
+    for iq0, n in ((nq - 3, 4), (nq, 1), (-1, 2), (0, 9), (0, -1)):
+        with pytest.raises((eph.L.EphipError, IndexError)):
+            loop.run_qtile(iq0, n)
+        assert not calls
