@@ -602,17 +602,19 @@ class OuterKLoop:
         # RR->kR as the staged (GridOpt) transform with the projection fused, in FP32 for either precision:
         # k1 planes and (k1, k2) lines of the grid share their partial sums
         ks_host = st.ksurv.cpu().numpy()
-        self.gridopt = _GridOptKR.build(st, ks_host, self.nd_el, gridopt_mfma) if (gridopt and nw in (8, 16)) \
-            else None
+        staged = bool(staged and gridopt)
+        self.gridopt = None
+        if gridopt and nw in (8, 16):
+            if nw == 8 and staged and st.nbw <= _GridOptKR.NBW_MAX:   # the general form in place of the VALU projection
+                self.gridopt = _GridOptKR.build(st, ks_host, self.nd_el, general=True)
+            if self.gridopt is None:
+                self.gridopt = _GridOptKR.build(st, ks_host, self.nd_el, gridopt_mfma)
         # kR->kq as the staged transform over the uniform q grid with the rotations and g2 fused (FP32)
         self.gridopt_q = _GridOptKQ.build(st) if (gridopt and nw == 16 and nm <= 16 and st.nbw <= 4) else None
         # the same transforms for the shapes that the two do not cover (other nw, more modes, wider windows)
-        staged = bool(staged and gridopt)
         self.staged_k = _GridOptKR.build(st, ks_host, self.nd_el, general=True) if (
             staged and self.gridopt is None) else None
         self.staged_q = _GridOptKQ.build(st, general=True) if (staged and self.gridopt_q is None) else None
-        if self.gridopt is not None and not self.gridopt.mfma and nw != 16 and staged and self.gridopt.box > 3:
-            self.gridopt.use_general()
         # the lane-private projection adds in another order than the MFMA tiles: boxes of 27 R and callers without the
         # general staged kernels keep the digits that FP64 rates are held to (_GridOptKR.SMALL_BOX)
         if self.gridopt is not None and not self.gridopt.general and (not staged or self.gridopt.box <= 3):
@@ -1079,12 +1081,6 @@ class _GridOptKR:
         self.plane_pos = {p: i for i, p in enumerate(self.planes)}
         self.cache = []  # [group, {plane: buffer}, buffers], most recent last, at most two
         self.next_k = 0  # the general form: one past the last batch's k
-
-    def use_general(self):
-        """Take the general form (ephip_staged_project) in place of the VALU projection."""
-        self.general, self._nb = True, 1
-        if self.np in (3, 5, 7) and self.nd // 8 < 1 << 25 and self.rmin[1] == self.rmin[2] == -(self.np // 2):
-            self.jl = 8
 
     def lanes(self) -> bool:
         """The lane-private projection applies (ephip_lane_project)."""

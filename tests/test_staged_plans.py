@@ -142,3 +142,15 @@ def test_outer_q_tile_past_the_last_q_is_refused(monkeypatch, staged):
         with pytest.raises((eph.L.EphipError, IndexError)):
             loop.run_qtile(iq0, n)
         assert not calls
+
+
+@pytest.mark.parametrize("nbw", [1, 3, 4])
+@pytest.mark.parametrize("edge", [4, 5])   # a face without its opposite offsets, and one with them
+def test_line_pieces_fit_the_projection(edge, nbw):
+    """ephip_staged_project takes pieces of at most 64 k and 128 units: 8 orbitals, lines of 48 k."""
+    st = _setup(8, 3, (2, 2, 48), (1, 1, 1), nbw=nbw, re=_box((edge,) * 3))
+    st.epmat.op_r = torch.zeros((1, 1))
+    rr = eph.OuterKLoop(st, nk_batch=192).rr
+    assert rr.general and rr.lanes() == (edge == 5)
+    assert rr.max_line_units <= 128 and rr.max_line_k <= 64
+    assert rr.line_start_host[0] == 0 and rr.line_start_host[-1] == 192
