@@ -221,9 +221,8 @@ __global__ __launch_bounds__(256) void bte_accumulate_tab_kernel(
     __shared__ int ciq[256], cf0[256], wsum[4];
     extern __shared__ uint16_t list[];  // [256 nbw] column | band << 8
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    // units first: with the columns first, the empty workgroups at the end of every unit all fell to the same XCDs
-    const int64_t c0 = (int64_t)(blockIdx.x / nunits) * 256;
-    const int u = (int)(blockIdx.x % nunits), cnt = count[u];
+    const int64_t c0 = units_first_tile() * 256;
+    const int u = blockIdx.x, cnt = count[u];
     if (c0 >= cnt) return;  // uniform
     const int64_t i = unit_state_index[u], row0 = (int64_t)u * cs + c0, orow0 = rowptr[u] + c0;
     int nb = 0;
@@ -635,13 +634,11 @@ extern "C" int ephip_bte_accumulate_tables(int32_t nunits, int64_t cs, int32_t n
     EPHIP_REQUIRE(count && col_index && ikq && g2 && unit_state_index && state_offset && bmin && bmax && e_state &&
                       tab_q && tab_s && Ts && etas && rowptr && S_out && S_in && row_code,
                   "bte_accumulate_tables: null device pointer");
-    const int64_t wgs = (cs + 255) / 256 * nunits;
-    EPHIP_REQUIRE(wgs <= 0x7fffffffLL, "bte_accumulate_tables: %lld workgroups", (long long)wgs);
     using K = decltype(&bte_accumulate_tab_kernel<1, 1>);
 #define BTE_ROW(m) {bte_accumulate_tab_kernel<m, 1>, bte_accumulate_tab_kernel<m, 2>, bte_accumulate_tab_kernel<m, 3>}
     static const K kern[6][3] = {BTE_ROW(1), BTE_ROW(2), BTE_ROW(3), BTE_ROW(4), BTE_ROW(5), BTE_ROW(6)};
 #undef BTE_ROW
-    kern[method - 1][nT == 1 ? 0 : nT == 2 ? 1 : 2]<<<(unsigned)wgs, 256,
+    kern[method - 1][nT == 1 ? 0 : nT == 2 ? 1 : 2]<<<units_first_grid(nunits, (cs + 255) / 256), 256,
                                                       (size_t)256 * nbw * sizeof(uint16_t), as_stream(stream)>>>(
         nunits, cs, nbw, nm, nq, count, col_index, ikq, g2, unit_state_index, state_offset, bmin, bmax, e_state, tab_q,
         tab_s, wtq, nT, Ts, etas, smearing, w_cut, nstates, rowptr, S_out, S_in, row_code,

@@ -58,6 +58,16 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+// Grid of `tiles` workgroups for each of nunits <= 65535 units, the units first: workgroups are dealt to the XCDs and
+// their shader engines in turn, and with a unit's tiles first the empty ones at its end leave the same of them idle. The
+// unit is blockIdx.x; a tile past the last one (its columns past the unit's) has nothing to do. A dimension takes at
+// most 2^32 threads, y and z 65535 workgroups.
+inline dim3 units_first_grid(int nunits, int64_t tiles) {
+    const int64_t y = tiles < 65535 ? tiles : 65535;
+    return dim3((unsigned)nunits, (unsigned)y, (unsigned)((tiles + y - 1) / y));
+}
+__device__ __forceinline__ int64_t units_first_tile() { return blockIdx.y + (int64_t)gridDim.y * blockIdx.z; }
+
 // Make this lane's LDS writes visible to the other lanes of its own wavefront and keep the
 // compiler from moving LDS accesses across the point. No cross-wave synchronisation.
 __device__ __forceinline__ void wave_lds_sync() {

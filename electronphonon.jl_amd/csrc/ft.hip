@@ -336,7 +336,7 @@ template <int RB, int TN, int KC>
 __global__ __launch_bounds__(1024) void ft32_kernel(int64_t ndata, int nr, const cplx<float> *__restrict__ op,
                                                     int64_t ldop, const int *__restrict__ irvec, int nk,
                                                     const double *__restrict__ xk, cplx<float> *__restrict__ out,
-                                                    int64_t ldout, FtBatch bt, unsigned nunits, int WR) {
+                                                    int64_t ldout, FtBatch bt, int WR) {
     extern __shared__ float ft32_lds[];
     constexpr int NF = FT_FILL, NPI = KC * TN / (64 * NF), AE = 3 * KC / NF, PB = TN + 32;
     __shared__ float2 tab[FT_TAB_MAX][TN];
@@ -344,15 +344,13 @@ __global__ __launch_bounds__(1024) void ft32_kernel(int64_t ndata, int nr, const
     const int TM = 16 * RB * WR, PA = TM + 4;
     const int stage = KC * 2 * (PA + PB);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Units first: the chip hands workgroups to its shader engines in turn, and a tail of column tiles without work in
-    // every unit would leave the same engines idle (half of the columns kept: twice the time).
-    const unsigned tile = blockIdx.x / nunits, rtiles = (unsigned)((ndata + TM - 1) / TM);
-    const int64_t d0 = (int64_t)(tile % rtiles) * TM;
-    const int j0 = (int)(tile / rtiles) * TN;
+    const unsigned tile = (unsigned)units_first_tile(), rtiles = (unsigned)((ndata + TM - 1) / TM);
+    const int64_t d0 = (int64_t)(tile % rtiles) * TM, j0l = (int64_t)(tile / rtiles) * TN;
+    const int j0 = (int)j0l;
     {
-        const int u = blockIdx.x % nunits;
+        const int u = blockIdx.x;
         if (bt.ncol) nk = bt.ncol[u];
-        if (j0 >= nk) return;  // uniform for the block: nothing of this unit in this column tile
+        if (j0l >= nk) return;  // uniform for the block: nothing of this unit in this column tile
         op += u * bt.op_stride;
         out += u * bt.out_stride;
         if (bt.col_index) bt.col_index += u * bt.col_stride;
@@ -458,10 +456,11 @@ static int launch_ft32(int WR, int nunits, int64_t ndata, int nr, const cplx<flo
     if (lds + sizeof(float2) * FT_TAB_MAX * TN + 384 > 64 * 1024)
         EPHIP_TRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ft32_kernel<RB, TN, KC>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int64_t wgs = (int64_t)((nk + TN - 1) / TN) * ((ndata + TM - 1) / TM) * nunits;
-    EPHIP_REQUIRE(wgs <= 0x7fffffffLL, "fourier_c32: %lld workgroups", (long long)wgs);
-    ft32_kernel<RB, TN, KC><<<(unsigned)wgs, 64 * waves, lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt,
-                                                                   (unsigned)nunits, WR);
+    // units first: half of the columns kept took twice the time with the column tiles first
+    const int64_t tiles = ((int64_t)nk + TN - 1) / TN * ((ndata + TM - 1) / TM);
+    EPHIP_REQUIRE(tiles <= 65535LL * 65535, "fourier_c32: %lld tiles", (long long)tiles);
+    ft32_kernel<RB, TN, KC><<<units_first_grid(nunits, tiles), 64 * waves, lds, s>>>(ndata, nr, op, ldop, irvec, nk, xk,
+                                                                                     out, ldout, bt, WR);
     return EPHIP_OK;
 }
 
@@ -471,7 +470,7 @@ static int launch_ft32(int WR, int nunits, int64_t ndata, int nr, const cplx<flo
 // units: 54 with 16 x 64, 66 with 32 x 128; 48 rows x 125 R x 4096 columns: 18 with 16 x 64, 22 with 32 x 64.
 static int ft32_run(int nunits, int64_t ndata, int nr, const cplx<float> *op, int64_t ldop, const int *irvec, int nk,
                     const double *xk, cplx<float> *out, int64_t ldout, const FtBatch &bt, hipStream_t s) {
-    auto wgs = [&](int tm, int tn) { return (ndata + tm - 1) / tm * ((nk + tn - 1) / tn) * nunits; };
+    auto wgs = [&](int tm, int tn) { return (ndata + tm - 1) / tm * (((int64_t)nk + tn - 1) / tn) * nunits; };
     auto padded = [&](int tm) { return (ndata + tm - 1) / tm * tm; };
     if (ndata > 16 && ndata <= 32 && wgs(32, 128) >= 256)
         return launch_ft32<2, 128, 8>(1, nunits, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, bt, s);

@@ -125,8 +125,8 @@ __global__ __launch_bounds__(256) void rotate_kq_g2_kernel(int nw, int nm, int n
                                                           c32 *__restrict__ ep_out) {
     extern __shared__ c32 tsh[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int u = (int)(blockIdx.x % nunits);  // units first, see rotate_kq_g2_lds_kernel
-    const int64_t c = (int64_t)(blockIdx.x / nunits) * 4 + wave;
+    const int u = blockIdx.x;
+    const int64_t c = units_first_tile() * 4 + wave;
     if (c >= count[u]) return;
     c32 *T = tsh + wave * nbw * nm;
     const int64_t row = (int64_t)u * cs + c;
@@ -192,10 +192,8 @@ __global__ __launch_bounds__(256) void rotate_kq_g2_lds_kernel(int nw, int nm, i
                                                               const double *__restrict__ omega,
                                                               float *__restrict__ g2, c32 *__restrict__ ep_out) {
     extern __shared__ __attribute__((aligned(16))) unsigned char rkq_lds[];
-    // Units first: workgroups go to the XCDs and their shader engines in turn, and with the columns first the empty
-    // ones at the end of every unit leave the same of them idle.
-    const int u = (int)(blockIdx.x % nunits);
-    const int64_t c0 = (int64_t)(blockIdx.x / nunits) * RKQ_COLS;
+    const int u = blockIdx.x;
+    const int64_t c0 = units_first_tile() * RKQ_COLS;
     const int cnt = count[u];
     if (c0 >= cnt) return;  // uniform for the block
     const int ncol = (int)min<int64_t>(RKQ_COLS, cnt - c0);
@@ -378,15 +376,14 @@ extern "C" int ephip_eph_rotate_kq_g2(int32_t nw, int32_t nm, int32_t nbw, int32
     if (nunits == 0 || cs == 0) return EPHIP_OK;
     EPHIP_REQUIRE(count && col_index && ikq && Gq && U && bmin && bmax && uph && omega && (g2 || ep),
                   "eph_rotate_kq_g2: null device pointer");
-    EPHIP_REQUIRE((cs + 3) / 4 * nunits <= 0x7fffffffLL, "eph_rotate_kq_g2: %lld columns", (long long)(cs * nunits));
     const size_t lds2 = rkq_lds_bytes(nw, nm, nbw);
     if (lds2 <= 64 * 1024) {
-        const unsigned grid = (unsigned)((cs + RKQ_COLS - 1) / RKQ_COLS * nunits);
+        const dim3 grid = units_first_grid(nunits, (cs + RKQ_COLS - 1) / RKQ_COLS);
         rotate_kq_g2_lds_kernel<<<grid, 256, lds2, as_stream(stream)>>>(
             nw, nm, nbw, nunits, cs, count, col_index, ikq, static_cast<const c32 *>(Gq), ldg, gstride,
             static_cast<const c32 *>(U), bmin, bmax, static_cast<const c32 *>(uph), omega, g2, static_cast<c32 *>(ep));
     } else {  // large nw*nm: one wave per column
-        const unsigned grid = (unsigned)((cs + 3) / 4 * nunits);
+        const dim3 grid = units_first_grid(nunits, (cs + 3) / 4);
         rotate_kq_g2_kernel<<<grid, 256, lds, as_stream(stream)>>>(nw, nm, nbw, nunits, cs, count, col_index, ikq,
                                                                   static_cast<const c32 *>(Gq), ldg, gstride,
                                                                   static_cast<const c32 *>(U), bmin, bmax,
