@@ -316,12 +316,19 @@ static Ft64Tile ft64_tile(int64_t ndata, int nr, int nk) {
     return best;
 }
 
+// Columns of a launch: a tile has up to 64 threads a column, and a grid dimension takes 2^32.
+constexpr int64_t FT64_COLS = 1 << 25;
+
 static int ft64_run(int64_t ndata, int nr, const cplx<double> *op, int64_t ldop, const int *irvec, int nk,
                     const double *xk, cplx<double> *out, int64_t ldout, hipStream_t s) {
     const Ft64Tile t = ft64_tile(ndata, nr, nk);
-    if (t.form == 0) return launch_ft64<4, 2, 8, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
-    if (t.form == 1) return launch_ft64<2, 1, 16, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
-    return launch_ft64<1, 1, 32, 8>(t.wr, t.wc, ndata, nr, op, ldop, irvec, nk, xk, out, ldout, s);
+    auto launch = t.form == 0 ? launch_ft64<4, 2, 8, 8> : t.form == 1 ? launch_ft64<2, 1, 16, 8> : launch_ft64<1, 1, 32, 8>;
+    for (int64_t j = 0; j < nk; j += FT64_COLS) {
+        const int st = launch(t.wr, t.wc, ndata, nr, op, ldop, irvec, (int)std::min<int64_t>(FT64_COLS, nk - j),
+                              xk + 3 * j, out + ldout * j, ldout, s);
+        if (st) return st;
+    }
+    return EPHIP_OK;
 }
 
 // FP32 form. As ft64_kernel: FT_FILL waves fill two LDS stages of KC complex R, WR x WC waves multiply. A wave owns

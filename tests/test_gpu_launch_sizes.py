@@ -81,3 +81,25 @@ def test_fourier_batched(backend):
                L.ptr(out), nd, 0, L.PREC_FP32, L.stream_handle())
         got.append(out)
     assert float(got[0].abs().min()) > 0 and torch.equal(*got)
+
+
+def test_fourier_c64_columns(backend):
+    """More columns than a grid dimension has room for (6 threads each); the columns repeat 1021 points."""
+    import numpy as np
+    import torch
+    from ephip import _lib as L
+    n, m = 2 ** 32 // 6 + 100000, 1021
+    op = torch.tensor([[0.6 - 0.8j]], dtype=torch.complex128, device="cuda")
+    r = torch.tensor([[2, -1, 3]], dtype=torch.int32, device="cuda")
+    x = np.random.default_rng(3).uniform(-1, 1, (m, 3))
+    period = torch.from_numpy(x).to("cuda")
+    xk = period.repeat(-(-n // m), 1)[:n].contiguous()
+    out = torch.zeros(n, dtype=torch.complex128, device="cuda")
+    L.call("ephip_fourier_c64", 1, 1, L.ptr(op), 1, L.ptr(r), n, L.ptr(xk), L.ptr(out), 1, L.stream_handle())
+    ref = torch.from_numpy((0.6 - 0.8j) * np.exp(2j * np.pi * (x @ [2, -1, 3]))).to("cuda")
+    whole = out[: n // m * m].view(-1, m)
+    for row in (0, whole.shape[0] - 1):        # |t| < 6 cycles: 6 2 pi 2^-53 in the angle, a few ulp of the rest
+        assert float((whole[row] - ref).abs().max()) <= 1e-14
+    for a in range(0, whole.shape[0], 1 << 16):   # every repetition gives the same bits
+        assert bool((torch.view_as_real(whole[a:a + (1 << 16)]) == torch.view_as_real(whole[0])).all())
+    assert torch.equal(out[n // m * m:], whole[0][: n % m])
