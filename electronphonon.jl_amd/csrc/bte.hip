@@ -607,7 +607,7 @@ extern "C" int ephip_bte_tables(int32_t nq, int32_t nm, const double *omega, int
     EPHIP_REQUIRE(method >= 1 && method <= 6, "bte_tables: method %d outside 1..6", method);
     const int64_t n = (int64_t)nm * nq + nT * nstates;
     if (n == 0) return EPHIP_OK;
-    EPHIP_REQUIRE(n <= 0x7fffffffLL * 256, "bte_tables: too many entries");
+    EPHIP_REQUIRE(n <= MAX_THREADS_X, "bte_tables: too many entries");
     EPHIP_REQUIRE(omega && e_state && mus && Ts && tab_q && tab_s, "bte_tables: null device pointer");
     bte_tables_kernel<<<nbk(n), 256, 0, as_stream(stream)>>>(nq, nm, omega, nstates, e_state, nT, mus, Ts, method, tab_q,
                                                             tab_s);

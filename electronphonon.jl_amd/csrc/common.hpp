@@ -60,8 +60,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // Grid of `tiles` workgroups for each of nunits <= 65535 units, the units first: workgroups are dealt to the XCDs and
 // their shader engines in turn, and with a unit's tiles first the empty ones at its end leave the same of them idle. The
-// unit is blockIdx.x; a tile past the last one (its columns past the unit's) has nothing to do. A dimension takes at
-// most 2^32 threads, y and z 65535 workgroups.
+// unit is blockIdx.x; a tile past the last one (its columns past the unit's) has nothing to do. y and z take 65535
+// workgroups, x MAX_THREADS_X threads: with 65535 units of 257 tiles of 256 threads side by side in x the launch
+// reported no error and left the tiles past 2^32 threads out.
+constexpr int64_t MAX_THREADS_X = 0xffffffffLL & ~255LL;
 inline dim3 units_first_grid(int nunits, int64_t tiles) {
     const int64_t y = tiles < 65535 ? tiles : 65535;
     return dim3((unsigned)nunits, (unsigned)y, (unsigned)((tiles + y - 1) / y));

@@ -267,8 +267,8 @@ extern "C" int ephip_staged_rq_rotate(int32_t nw, int32_t nm, int32_t nbw, int32
     EPHIP_REQUIRE(lda >= (int64_t)nw * nm * nq, "staged_rq_rotate: lda too small");
     const int64_t n = (int64_t)nk * nq * nm;
     if (n == 0) return EPHIP_OK;
+    EPHIP_REQUIRE(n <= MAX_THREADS_X, "staged_rq_rotate: too many (k, q, mode)");
     EPHIP_REQUIRE(ks && xk && xq && kus && A && U && bmin && bmax && omega && ikq && g2, "staged_rq_rotate: null device pointer");
-    EPHIP_REQUIRE(n <= 0x7fffffffLL * 256, "staged_rq_rotate: too many (k, q, mode)");
     staged_rq_rotate_kernel<<<(unsigned)((n + 255) / 256), 256, 0, as_stream(stream)>>>(
         nw, nm, nbw, nq, k0, nk, ks, xk, xq, ngrid[0], ngrid[1], ngrid[2], kus, static_cast<const cplx<float> *>(A), lda,
         static_cast<const cplx<float> *>(U), bmin, bmax, omega, ldk, ikq, g2, static_cast<float2 *>(ep));
