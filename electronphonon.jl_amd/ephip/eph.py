@@ -301,13 +301,16 @@ class OuterQLoop:
         if iq0 < 0 or nq < 0 or iq0 + nq > nq_all:
             raise IndexError(f"tile of {nq} q at {iq0}: there are {nq_all} q")
         if self.staged is not None:
-            self.staged.run(self, iq0, nq)
+            self.staged.transform(self, iq0, nq)
             nks = st.ksurv.shape[0]
             for t in range(nq):
+                t0 = t % self.staged.nt
+                if t0 == 0:
+                    self.staged.run(self, iq0, t, min(self.staged.nt, nq - t))
                 for c in calculators:
                     c.begin_q(iq0 + t)
                 for s in range(0, nks, self.nk_batch):
-                    payload = self.staged.payload(self, iq0, t, s, min(nks, s + self.nk_batch))
+                    payload = self.staged.payload(iq0 + t, t0, s, min(nks, s + self.nk_batch))
                     for c in calculators:
                         c.run(payload)
                 for c in calculators:
@@ -353,9 +356,13 @@ class OuterQLoop:
 
 
 class _StagedRQ:
-    """Staged Rq->kq of a tile of q (csrc/staged_q.hip): RR->Rq with the tile's q side by side, stage 1 of each k1
-    plane and the k-side projection of every unit (k, in-window band) over the rows (i, j, nu, q), then the k+q window
-    rotation and g2 of every (k, q)."""
+    """Staged Rq->kq of a tile of q (csrc/staged_q.hip): RR->Rq with the tile's q side by side; then, for nt q at a time,
+    stage 1 of each k1 plane and the k-side projection of every unit (k, in-window band) over the rows (i, j, nu, q), and
+    the k+q window rotation and g2 of every (k, q)."""
+
+    # What is held per q for all surviving k (g2, ep, k+q), for a k batch (A) and for the k1 planes: nt is the tile, or
+    # what this holds; where one q does not fit, the loop takes the direct form, whose buffers are nk_batch rows.
+    TILE_BYTES = 8 << 30
 
     @classmethod
     def build(cls, loop):
@@ -363,10 +370,23 @@ class _StagedRQ:
         ks = st.ksurv.cpu().numpy()
         if st.nw > 32 or st.nm > 48 or len(ks) == 0:
             return None
-        go = _GridOptKR.build(st, ks, loop.nq_tile * st.nw * st.nw * st.nm, general=True, small=True)
-        return None if go is None else cls(loop, ks, go)
+        nd_q = st.nw * st.nw * st.nm
+        go = _GridOptKR.build(st, ks, loop.nq_tile * nd_q, general=True, small=True)
+        if go is None:
+            return None
+        nb = (st.el.filt.band_max - st.el.filt.band_min + 1).cpu().numpy()[ks].astype(np.int64)
+        cum = np.concatenate([[0], np.cumsum(nb)])
+        nk_batch = min(loop.nk_batch, len(ks))
+        max_units = max(int(cum[min(s + nk_batch, len(ks))] - cum[s]) for s in range(0, len(ks), nk_batch))
+        per_q = (len(ks) * (st.nm * st.nbw ** 2 * (12 if loop.keep_ep else 4) + 8) + 8 * max_units * st.nw * st.nm
+                 + 8 * go.plane_buffers() * go.np ** 2 * nd_q)
+        nt = min(loop.nq_tile, cls.TILE_BYTES // per_q)
+        if nt < 1:
+            return None
+        go.nd = go.nd_max = nt * nd_q
+        return cls(loop, ks, go, cum, nk_batch, max_units, nt)
 
-    def __init__(self, loop, ks, go):
+    def __init__(self, loop, ks, go, k_unit_start, nk_batch, max_units, nt):
         import ctypes
         torch = _torch()
         st = loop.st
@@ -375,8 +395,8 @@ class _StagedRQ:
         self.go = go
         self.st = st
         f = st.el.filt
-        nb = (f.band_max - f.band_min + 1).cpu().numpy()[ks].astype(np.int64)
-        self.k_unit_start = np.concatenate([[0], np.cumsum(nb)])
+        self.k_unit_start = k_unit_start
+        nb = np.diff(k_unit_start)
         self.k_unit_start_dev = torch.from_numpy(self.k_unit_start.astype(np.int32)).to(dev)
         self.unit_kpos = torch.from_numpy(np.repeat(np.arange(len(ks)), nb).astype(np.int32)).to(dev)
         self.unit_state = torch.from_numpy(np.repeat(ks, nb).astype(np.int64)).to(dev)
@@ -385,15 +405,14 @@ class _StagedRQ:
         self.unit_band = torch.from_numpy(band.astype(np.int32)).to(dev)
         self.max_units_per_k = int(nb.max())
         self.xk_surv = loop.xk_surv
-        self.nk_batch = min(loop.nk_batch, len(ks))
-        starts = range(0, len(ks), self.nk_batch)
-        self.max_units = max(int(self.k_unit_start[min(s + self.nk_batch, len(ks))] - self.k_unit_start[s]) for s in starts)
-        nt = loop.nq_tile
+        self.nk_batch, self.max_units, self.nt = nk_batch, max_units, nt
         self.nrp = nm * nt   # go.run's columns per i: (nu, q)
         self.A = torch.empty((self.max_units, nw * nm * nt), dtype=torch.complex64, device=dev)
-        self.epmat_el = loop.eRpq.view(loop.nr_el, nt * nw * nw * nm)   # rows (i, j, nu, q) of each Re
+        self.rows = loop.eRpq.view(loop.nr_el, loop.nq_tile * nw * nw * nm)   # rows (i, j, nu, q) of each Re
+        self.epmat_el = None                                                  # those of the q in hand
         nrp = st.epmat.nr
-        self.phases = torch.empty(((nt + 15) // 16) * 16 * ((nrp + 3) // 4 * 4), dtype=torch.complex64, device=dev)
+        self.phases = torch.empty(((loop.nq_tile + 15) // 16) * 16 * ((nrp + 3) // 4 * 4), dtype=torch.complex64,
+                                  device=dev)
         shape = (nt, len(ks), nm, st.nbw, st.nbw)
         self.g2 = torch.empty(shape, dtype=torch.float32, device=dev)
         self.ep = torch.empty(shape, dtype=torch.complex64, device=dev) if loop.keep_ep else None
@@ -402,30 +421,38 @@ class _StagedRQ:
         self.uph = st.ph.u.contiguous()
         self.kgrid_c = (ctypes.c_int32 * 3)(*map(int, st.kgrid))
 
-    def run(self, loop, iq0, nq):
-        """g2, ep and ikq of the tile's q at every surviving k."""
+    def transform(self, loop, iq0, nq):
+        """RR->Rq of the tile."""
+        st = self.st
+        nw, nm = st.nw, st.nm
+        L.call("ephip_staged_rr_to_rq", nw * nw, nm, loop.nr_el, st.epmat.nr, L.ptr(st.epmat.op_r), st.epmat.op_r.stride(0),
+               L.ptr(st.epmat.irvec_dev()), nq, L.ptr(st.ph.xq[iq0:iq0 + nq]), L.ptr(self.uph[iq0:iq0 + nq]),
+               L.ptr(self.phases), L.ptr(loop.gq_work), loop.gq_work.stride(0), L.ptr(self.rows), self.rows.stride(0),
+               L.stream_handle())
+
+    def run(self, loop, iq0, t, n):
+        """g2, ep and ikq of the tile's q t .. t + n - 1 (n <= nt) at every surviving k."""
         import ctypes as C
         st, go = self.st, self.go
         nw, nm = st.nw, st.nm
+        nd_q = nw * nw * nm
         nks = st.ksurv.shape[0]
         stream = L.stream_handle()
-        xq, om = st.ph.xq[iq0:iq0 + nq], self.omega[iq0:iq0 + nq]
-        L.call("ephip_staged_rr_to_rq", nw * nw, nm, loop.nr_el, st.epmat.nr, L.ptr(st.epmat.op_r), st.epmat.op_r.stride(0),
-               L.ptr(st.epmat.irvec_dev()), nq, L.ptr(xq), L.ptr(self.uph[iq0:iq0 + nq]), L.ptr(self.phases),
-               L.ptr(loop.gq_work), loop.gq_work.stride(0), L.ptr(self.epmat_el), self.epmat_el.stride(0), stream)
-        go.nd = nq * nw * nw * nm
+        xq, om = st.ph.xq[iq0 + t:iq0 + t + n], self.omega[iq0 + t:iq0 + t + n]
+        self.epmat_el = self.rows[:, t * nd_q:(t + n) * nd_q]
+        go.nd = n * nd_q
         go.invalidate()
         for s in range(0, nks, self.nk_batch):
-            n = min(self.nk_batch, nks - s)
-            u0, u1 = int(self.k_unit_start[s]), int(self.k_unit_start[s + n])
-            go.run(self, s, n, u0, u1, self.A, stream)
-            L.call("ephip_staged_rq_rotate", nw, nm, st.nbw, nq, s, n, L.ptr(st.ksurv), L.ptr(st.el.xk), L.ptr(xq),
+            nk = min(self.nk_batch, nks - s)
+            u0, u1 = int(self.k_unit_start[s]), int(self.k_unit_start[s + nk])
+            go.run(self, s, nk, u0, u1, self.A, stream)
+            L.call("ephip_staged_rq_rotate", nw, nm, st.nbw, n, s, nk, L.ptr(st.ksurv), L.ptr(st.el.xk), L.ptr(xq),
                    C.addressof(self.kgrid_c), L.ptr(self.k_unit_start_dev), L.ptr(self.A), self.A.stride(0),
                    L.ptr(st.el.U), L.ptr(st.el.filt.band_min), L.ptr(st.el.filt.band_max), L.ptr(om), nks,
                    L.ptr(self.ikq), L.ptr(self.g2), L.ptr(self.ep), stream)
 
-    def payload(self, loop, iq0, t, s, e):
-        return EPDataKWindowed(iq0 + t, self.st.ksurv[s:e], self.ikq[t, s:e], self.g2[t, s:e],
+    def payload(self, iq, t, s, e):
+        return EPDataKWindowed(iq, self.st.ksurv[s:e], self.ikq[t, s:e], self.g2[t, s:e],
                                None if self.ep is None else self.ep[t, s:e], self.st.nbw)
 
 
@@ -1099,6 +1126,15 @@ class _GridOptKR:
         for entry in self.cache:
             entry[0], entry[1] = None, {}
 
+    def _groups(self) -> tuple[int, int]:
+        """Groups whose planes are held at a time (two, where there are as many), and the planes of one."""
+        return min(2, -(-len(self.planes) // self.PLANES)), min(self.PLANES, len(self.planes))
+
+    def plane_buffers(self) -> int:
+        """Plane buffers held at most."""
+        groups, planes = self._groups()
+        return groups * planes
+
     def _plane_buffer(self, plane, epmat_el, stream):
         import ctypes as C
         torch = _torch()
@@ -1107,9 +1143,10 @@ class _GridOptKR:
                 return entry[1][plane]
         g = self.plane_pos[plane] // self.PLANES
         members = self.planes[g * self.PLANES:(g + 1) * self.PLANES]
-        if len(self.cache) < 2:
+        held, size = self._groups()
+        if len(self.cache) < held:
             bufs = [torch.empty((self.np * self.np, self.nd_max), dtype=torch.complex64, device=epmat_el.device)
-                    for _ in range(self.PLANES)]
+                    for _ in range(size)]
         else:  # reuse the older group's buffers (stream order: its projections are already queued)
             bufs = self.cache.pop(0)[2]
         self.cache.append([g, dict(zip(members, bufs)), bufs])

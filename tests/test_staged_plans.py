@@ -154,3 +154,27 @@ def test_line_pieces_fit_the_projection(edge, nbw):
     assert rr.general and rr.lanes() == (edge == 5)
     assert rr.max_line_units <= 128 and rr.max_line_k <= 64
     assert rr.line_start_host[0] == 0 and rr.line_start_host[-1] == 192
+
+
+def _outer_q(st, **kw):
+    st.epmat.op_r = torch.zeros((1, 1))
+    return eph.OuterQLoop(st, **kw)
+
+
+@pytest.mark.parametrize("keep_ep", [False, True])
+@pytest.mark.parametrize("tile,budget", [(8, 1 << 33), (8, 3 << 20), (8, 1 << 20), (5, 1 << 18)])
+def test_outer_q_buffers_stay_within_their_budget(monkeypatch, keep_ep, tile, budget):
+    """What the staged form holds for every surviving k of a tile is bounded: fewer q at a time, or the direct form,
+    whose buffers are nk_batch rows."""
+    monkeypatch.setattr(eph._StagedRQ, "TILE_BYTES", budget)
+    st = _setup(4, 6, (6, 5, 4), nbw=3)
+    loop = _outer_q(st, nq_tile=tile, nk_batch=50, keep_ep=keep_ep)
+    s = loop.staged
+    per_q = 120 * (6 * 9 * (12 if keep_ep else 4) + 8) + 8 * 150 * 4 * 6 + 8 * 6 * 25 * 4 * 4 * 6   # 6 planes of k1
+    if per_q > budget:
+        assert s is None
+        return
+    assert s.nt == min(tile, budget // per_q)
+    held = [s.g2, s.ikq, s.A] + ([s.ep] if keep_ep else [])
+    held = sum(t.numel() * t.element_size() for t in held) + 8 * 6 * 25 * s.go.nd_max
+    assert held <= budget and s.go.nd_max == s.nt * 4 * 4 * 6
