@@ -608,39 +608,31 @@ class OuterKLoop:
         order of the additions, about 3e-8 of a scattering rate."""
         torch = _torch()
         self.st = st
-        if nk_batch is None:  # memory-adaptive width (plan_batch), the e-ph tensor already resident
-            per_k, _ = core.outer_k_staging_bytes(st.nw, st.nm, st.irvec_el_dev.shape[0], st.epmat.nr,
-                                                  st.el.xk.shape[0], st.ph.xq.shape[0], st.nbw)
-            nre_b = 8 * st.epmat.op_r.numel()  # the "el" copy is allocated below
-            nk_batch = core.plan_batch(core.free_bytes(None), per_k, nre_b, nk_batch_cap, what="outer-k")
-        self.nk_batch = int(nk_batch)
-        self.precision = precision
         dev = st.el.xk.device
         nw, nm = st.nw, st.nm
         self.nre = st.irvec_el_dev.shape[0]
         self.nrp = st.epmat.nr
         self.nd_el = nw * nw * nm * self.nrp
-        # "el" layout copy of the e-ph tensor: rows (i, j, nu, Rp), one column per Re
-        self.epmat_el = torch.empty((self.nre, self.nd_el), dtype=torch.complex64, device=dev)
-        L.call("ephip_eph_ph_to_el", nw * nw * nm, self.nre, self.nrp, L.ptr(st.epmat.op_r), L.ptr(self.epmat_el),
-               L.stream_handle())
-        self.el_obj = _RqObject(self.epmat_el, st.irvec_el_dev, self.nd_el)
-        self.irvec_ep_dev = st.epmat.irvec_dev()
+        el_bytes = 8 * st.epmat.op_r.numel()  # the "el" copy is allocated below
         # RR->kR as the staged (GridOpt) transform with the projection fused, in FP32 for either precision:
         # k1 planes and (k1, k2) lines of the grid share their partial sums
         ks_host = st.ksurv.cpu().numpy()
         staged = bool(staged and gridopt)
+
+        def staged_kr(**kw):
+            go = _GridOptKR.build(st, ks_host, self.nd_el, **kw)
+            return go if go is not None and go.fit_planes(el_bytes) else None
+
         self.gridopt = None
         if gridopt and nw in (8, 16):
             if nw == 8 and staged and st.nbw <= _GridOptKR.NBW_MAX:   # the general form in place of the VALU projection
-                self.gridopt = _GridOptKR.build(st, ks_host, self.nd_el, general=True)
+                self.gridopt = staged_kr(general=True)
             if self.gridopt is None:
-                self.gridopt = _GridOptKR.build(st, ks_host, self.nd_el, gridopt_mfma)
+                self.gridopt = staged_kr(mfma=gridopt_mfma)
         # kR->kq as the staged transform over the uniform q grid with the rotations and g2 fused (FP32)
         self.gridopt_q = _GridOptKQ.build(st) if (gridopt and nw == 16 and nm <= 16 and st.nbw <= 4) else None
         # the same transforms for the shapes that the two do not cover (other nw, more modes, wider windows)
-        self.staged_k = _GridOptKR.build(st, ks_host, self.nd_el, general=True) if (
-            staged and self.gridopt is None) else None
+        self.staged_k = staged_kr(general=True) if (staged and self.gridopt is None) else None
         self.staged_q = _GridOptKQ.build(st, general=True) if (staged and self.gridopt_q is None) else None
         # the lane-private projection adds in another order than the MFMA tiles: boxes of 27 R and callers without the
         # general staged kernels keep the digits that FP64 rates are held to (_GridOptKR.SMALL_BOX)
@@ -648,6 +640,18 @@ class OuterKLoop:
             self.gridopt.jl = 0
         self.rr = self.gridopt if self.gridopt is not None else self.staged_k
         self.kq = self.gridopt_q if self.gridopt_q is not None else self.staged_q
+        if nk_batch is None:  # memory-adaptive width (plan_batch), the e-ph tensor already resident
+            per_k, _ = core.outer_k_staging_bytes(nw, nm, self.nre, self.nrp, st.el.xk.shape[0], st.ph.xq.shape[0], st.nbw)
+            planes = 0 if self.rr is None else self.rr.plane_bytes()
+            nk_batch = core.plan_batch(core.free_bytes(None), per_k, el_bytes + planes, nk_batch_cap, what="outer-k")
+        self.nk_batch = int(nk_batch)
+        self.precision = precision
+        # "el" layout copy of the e-ph tensor: rows (i, j, nu, Rp), one column per Re
+        self.epmat_el = torch.empty((self.nre, self.nd_el), dtype=torch.complex64, device=dev)
+        L.call("ephip_eph_ph_to_el", nw * nw * nm, self.nre, self.nrp, L.ptr(st.epmat.op_r), L.ptr(self.epmat_el),
+               L.stream_handle())
+        self.el_obj = _RqObject(self.epmat_el, st.irvec_el_dev, self.nd_el)
+        self.irvec_ep_dev = st.epmat.irvec_dev()
         # split-BF16: the contractions that are not staged run on pre-packed operands. The "el" tensor is
         # split once (same bytes as complex64) and its complex64 copy released; the q-grid phase table is
         # built once; k phases and unit operands are packed per batch.
@@ -1031,11 +1035,12 @@ class _GridOptKR:
     2 and 3 and nw <= 16, else ephip_gridopt_kR_project[_mfma] or ephip_staged_project), the device
     GridOpt of src/wannier/GridOpt.jl: Re embedded in its bounding box, the surviving k (grid order,
     third index fastest) grouped into k1 planes and (k1, k2) lines. Stage 1 runs for a group of PLANES
-    consecutive planes at once (one pass over the operand for all of them); the two most recent groups
-    are kept, so a pass over the k batches in order computes each plane once."""
+    consecutive planes at once (one pass over the operand for all of them; fewer where memory is short); the
+    two most recent groups are kept, so a pass over the k batches in order computes each plane once."""
 
     N1_MAX, N23_MAX, KLINE_MAX, NBW_MAX = 32, 8, 64, 4
     PLANES = 8
+    PLANE_BYTES = 8 << 30   # plane buffers up to this are held without a look at the free memory
     LINE_UNITS = 128   # units of a line piece of the general form (ephip_staged_project)
     # boxes of 27 R stay with the direct kernels: the staged ones are 1.0 to 5.5 times as fast there (7.1 -> 2.4 ms
     # at 10 orbitals, 9 modes; 3.7 -> 3.6 at 16, 12), but their other order of the FP32 additions would move the FP64
@@ -1125,6 +1130,19 @@ class _GridOptKR:
         batch recomputes every plane it needs."""
         for entry in self.cache:
             entry[0], entry[1] = None, {}
+
+    def plane_bytes(self) -> int:
+        return 8 * self.plane_buffers() * self.np ** 2 * self.nd_max
+
+    def fit_planes(self, committed: int) -> bool:
+        """Take groups of fewer planes where the buffers would pass PLANE_BYTES and a quarter of the device memory left
+        beside ``committed``; False if those of one plane would."""
+        if self.plane_bytes() <= self.PLANE_BYTES:
+            return True
+        room = max(0, core.free_bytes(None) - committed) // 4
+        if self.plane_bytes() > room:
+            self.PLANES = min(self.PLANES, room // (2 * 8 * self.np ** 2 * self.nd_max))
+        return self.PLANES >= 1
 
     def _groups(self) -> tuple[int, int]:
         """Groups whose planes are held at a time (two, where there are as many), and the planes of one."""

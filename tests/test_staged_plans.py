@@ -178,3 +178,40 @@ def test_outer_q_buffers_stay_within_their_budget(monkeypatch, keep_ep, tile, bu
     held = [s.g2, s.ikq, s.A] + ([s.ep] if keep_ep else [])
     held = sum(t.numel() * t.element_size() for t in held) + 8 * 6 * 25 * s.go.nd_max
     assert held <= budget and s.go.nd_max == s.nt * 4 * 4 * 6
+
+
+@pytest.mark.parametrize("quarter,planes", [(100, 8), (13, 6), (2, 1), (1, 0)])
+def test_outer_k_planes_leave_room(monkeypatch, quarter, planes):
+    """Plane buffers take at most a quarter of what the "el" tensor leaves: smaller groups, or the direct form; the
+    batch is planned on what they leave."""
+    st = _setup(9, 3, (19, 2, 3))
+    st.epmat.op_r = torch.zeros((125, st.epmat.ndata // 125))
+    nd = 9 * 9 * 3 * 125
+    one, el = 8 * 25 * nd, 8 * st.epmat.op_r.numel()
+    monkeypatch.setattr(eph._GridOptKR, "PLANE_BYTES", 1 << 20, raising=False)
+    free = el + 4 * quarter * one + 3
+    monkeypatch.setattr(eph.core, "free_bytes", lambda _: free)
+    seen = []
+    plan = eph.core.plan_batch
+    monkeypatch.setattr(eph.core, "plan_batch", lambda *a, **k: seen.append(a) or plan(*a, **k))
+    loop = eph.OuterKLoop(st, nk_batch=None, nk_batch_cap=4)
+    if planes == 0:
+        assert loop.rr is None and loop.G is not None
+        assert seen[0][2] == el
+        return
+    assert loop.rr.PLANES == planes
+    held = 2 * planes * one
+    assert loop.rr.plane_buffers() == 2 * planes and held <= quarter * one
+    assert seen[0][0] == free and seen[0][2] == el + held
+    assert eph._GridOptKR.PLANES == 8
+
+
+def test_outer_k_planes_of_a_usual_size_ask_for_no_memory(monkeypatch):
+    st = _setup(9, 3, (19, 2, 3))
+    st.epmat.op_r = torch.zeros((125, 1))
+
+    def never(_):
+        raise AssertionError("free memory asked for")
+
+    monkeypatch.setattr(eph.core, "free_bytes", never)
+    assert eph.OuterKLoop(st, nk_batch=4).rr.PLANES == 8
