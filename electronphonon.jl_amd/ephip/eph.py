@@ -283,15 +283,34 @@ class OuterQLoop:
         self.eRpq = torch.empty((self.nq_tile, st.epmat.ndata), dtype=torch.complex64, device=dev)
         self.xk_surv = st.el.xk.index_select(0, st.ksurv).contiguous()
         self.staged = _StagedRQ.build(self) if staged else None
-        if self.staged is None:
+        # arithmetic each contraction runs in: the staged kernels are FP32 whatever ``precision`` asks for
+        self.precision_requested = precision
+        used = L.PREC_FP32 if self.staged is not None else precision
+        self.stage_precision = {"RR->Rq": used, "Rq->kq": used}
+        self.precision_overridden = used != precision
+        if self.staged is not None:   # g(k, q) is not stored; the payloads are views of g2 and ep
+            self.gk, self.g2, self.ep = None, self.staged.g2, self.staged.ep
+        else:
             self.gk = torch.empty((self.nk_batch, nd_q), dtype=torch.complex64, device=dev)
             self.g2 = torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.float32, device=dev)
             self.ep = (torch.empty((self.nk_batch, st.nm, st.nbw, st.nbw), dtype=torch.complex64, device=dev)
                        if keep_ep else None)
         self.xq_host = st.ph.xq.cpu().numpy()
-        # optional list collecting (start event, end event, columns) around each Rq->kq Fourier launch;
+        # optional list collecting (start event, end event, columns) around each Rq->kq Fourier launch (the staged
+        # form: each k batch's launches for the columns (k, q) of a tile);
         # the events are recorded on the current stream, which is the stream the kernels run on
         self.ft_timer = None
+
+    def _timed(self, columns: int, fn):
+        """fn(), between two events in ft_timer if that is set."""
+        if self.ft_timer is None:
+            return fn()
+        torch = _torch()
+        ev0, ev1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        ev0.record()
+        fn()
+        ev1.record()
+        self.ft_timer.append((ev0, ev1, columns))
 
     def run_qtile(self, iq0: int, nq: int, calculators=()):
         st = self.st
@@ -331,15 +350,8 @@ class OuterQLoop:
                 e = min(nks, s + self.nk_batch)
                 ik = st.ksurv[s:e]
                 ikq = core.kq_index(self.xk_surv[s:e], self.xq_host[iq], st.kgrid)
-                if self.ft_timer is not None:
-                    torch = _torch()
-                    ev0 = torch.cuda.Event(enable_timing=True)
-                    ev1 = torch.cuda.Event(enable_timing=True)
-                    ev0.record()
-                core.fourier_batched(obj, self.xk_surv[s:e], out=self.gk[: e - s], precision=self.precision)
-                if self.ft_timer is not None:
-                    ev1.record()
-                    self.ft_timer.append((ev0, ev1, e - s))
+                self._timed(e - s, lambda: core.fourier_batched(obj, self.xk_surv[s:e], out=self.gk[: e - s],
+                                                                precision=self.precision))
                 g2 = eph_rotate_rqkq_g2(self.gk[: e - s], ik, ikq, st.el, st.ph.omega[iq], st.nbw,
                                         g2=self.g2[: e - s], ep=None if self.ep is None else self.ep[: e - s])
                 payload = EPDataKWindowed(iq, ik, ikq, g2, None if self.ep is None else self.ep[: e - s], st.nbw)
@@ -445,7 +457,7 @@ class _StagedRQ:
         for s in range(0, nks, self.nk_batch):
             nk = min(self.nk_batch, nks - s)
             u0, u1 = int(self.k_unit_start[s]), int(self.k_unit_start[s + nk])
-            go.run(self, s, nk, u0, u1, self.A, stream)
+            loop._timed(nk * n, lambda: go.run(self, s, nk, u0, u1, self.A, stream))
             L.call("ephip_staged_rq_rotate", nw, nm, st.nbw, n, s, nk, L.ptr(st.ksurv), L.ptr(st.el.xk), L.ptr(xq),
                    C.addressof(self.kgrid_c), L.ptr(self.k_unit_start_dev), L.ptr(self.A), self.A.stride(0),
                    L.ptr(st.el.U), L.ptr(st.el.filt.band_min), L.ptr(st.el.filt.band_max), L.ptr(om), nks,

@@ -215,3 +215,35 @@ def test_outer_k_planes_of_a_usual_size_ask_for_no_memory(monkeypatch):
 
     monkeypatch.setattr(eph.core, "free_bytes", never)
     assert eph.OuterKLoop(st, nk_batch=4).rr.PLANES == 8
+
+
+def test_outer_q_reports_its_arithmetic_and_times_its_transforms(monkeypatch):
+    """The staged loop keeps what the direct one has: the payload buffers, ft_timer and, as the outer-k loop, the
+    arithmetic that the transforms run in beside the one asked for."""
+    st = _setup(3, 3, (4, 2, 3))
+    L = eph.L
+    for staged, prec, used in ((True, L.PREC_FP32, L.PREC_FP32), (True, L.PREC_BF16X3, L.PREC_FP32),
+                               (False, L.PREC_BF16X3, L.PREC_BF16X3)):
+        loop = _outer_q(st, nq_tile=5, nk_batch=10, precision=prec, staged=staged, keep_ep=True)
+        assert loop.precision_requested == loop.precision == prec
+        assert loop.stage_precision == {"RR->Rq": used, "Rq->kq": used}
+        assert loop.precision_overridden == (prec != used)
+        assert loop.g2.shape[-3:] == (3, 2, 2) and loop.ep.shape == loop.g2.shape and loop.ep.is_complex()
+        assert (loop.gk is None) == staged
+
+    class Event:
+        now = 0
+
+        def __init__(self, enable_timing):
+            assert enable_timing
+
+        def record(self):
+            Event.now += 1
+            self.at = Event.now
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    loop = _outer_q(st, nq_tile=5, nk_batch=10)
+    loop.ft_timer = []
+    loop.run_qtile(0, 5)
+    assert [n for _, _, n in loop.ft_timer] == [50, 50, 20]   # (k, q) of each of the three k batches: 24 k, 5 q
+    assert all(a.at + 1 == b.at for a, b, _ in loop.ft_timer)
