@@ -170,6 +170,8 @@ class BandSurrogate:
         """loss_and_grad in three launches; ga and gz of the returned buffers hold dL/dz of the two hidden layers."""
         torch = _torch()
         n, O, H = xk.shape[0], self.nout, self.hidden
+        if n == 0:
+            raise ZeroDivisionError("mean squared error of no points")
         a = acts if acts is not None else self._alloc_acts(n)
         nparts = max(1, min(256, (n + 31) // 32))   # workgroups of the weight gradients, at least 32 points each
         gw = grads if grads is not None else dict(gy=torch.empty((n, O), dtype=torch.float32, device=self.dev),
