@@ -126,6 +126,19 @@ class BandSurrogate:
         L.call("ephip_gemm_f32_splitk", 1, 0, o, 1, n, L.ptr(gz), o, L.ptr(ones), 1, L.ptr(part), 1, nsplit, st)
         L.call("ephip_colsum", nsplit, o, L.ptr(part), o, L.ptr(self.view(self.g, out_name)), st)
 
+    def _grads(self, n, npart, grads):
+        """Gradient buffers of n points with a workspace of npart floats: those given, completed where they come from
+        the other form of the step."""
+        torch = _torch()
+        O, H = self.nout, self.hidden
+        mk = lambda *s: torch.empty(s, dtype=torch.float32, device=self.dev)
+        if grads is None:
+            return dict(gy=mk(n, O), ga=mk(n, H), gz=mk(n, H), part=mk(npart),
+                        partial=torch.empty((n * O + 255) // 256, dtype=torch.float64, device=self.dev))
+        if grads["part"].numel() < npart:
+            grads["part"] = mk(npart)
+        return grads
+
     def loss_and_grad(self, xk, target, acts=None, grads=None):
         """Mean squared error over points and outputs; fills self.g. Returns (loss tensor (device), acts)."""
         torch = _torch()
@@ -135,14 +148,9 @@ class BandSurrogate:
         a = self.forward(xk, acts)
         st = L.stream_handle()
         O, H = self.nout, self.hidden
-        gw = grads if grads is not None else dict(gy=torch.empty((n, O), dtype=torch.float32, device=self.dev),
-                                                  ga=torch.empty((n, H), dtype=torch.float32, device=self.dev),
-                                                  gz=torch.empty((n, H), dtype=torch.float32, device=self.dev),
-                                                  part=torch.empty(64 * H * max(H, self.nf), dtype=torch.float32,
-                                                                   device=self.dev),
-                                                  partial=torch.empty((n * O + 255) // 256, dtype=torch.float64,
-                                                                      device=self.dev),
-                                                  ones=torch.ones(n, dtype=torch.float32, device=self.dev))
+        gw = self._grads(n, 64 * H * max(H, self.nf), grads)
+        if "ones" not in gw:
+            gw["ones"] = torch.ones(n, dtype=torch.float32, device=self.dev)
         L.call("ephip_mse_grad", n * O, L.ptr(a["y"]), L.ptr(target), 1.0 / (n * O), L.ptr(gw["gy"]),
                L.ptr(gw["partial"]), st)
         # layer 3
@@ -163,8 +171,10 @@ class BandSurrogate:
         return gw["partial"], a, gw
 
     def _fused(self) -> bool:
-        """Sizes of ephip_mlp_train_step: features and hidden multiples of 16 up to 128, outputs up to 64."""
-        return self.nf % 16 == 0 and self.nf <= 128 and self.hidden % 16 == 0 and self.hidden <= 128 and self.nout <= 64
+        """What ephip_mlp_train_step takes: features and hidden multiples of 16 up to 128, outputs up to 64, and
+        parameters that start at 16 bytes (a program may hold them as a part of another vector)."""
+        return (self.nf % 16 == 0 and self.nf <= 128 and self.hidden % 16 == 0 and self.hidden <= 128 and self.nout <= 64
+                and self.p.data_ptr() % 16 == 0)
 
     def _loss_and_grad_fused(self, xk, target, acts, grads):
         """loss_and_grad in three launches; ga and gz of the returned buffers hold dL/dz of the two hidden layers."""
@@ -174,13 +184,7 @@ class BandSurrogate:
             raise ZeroDivisionError("mean squared error of no points")
         a = acts if acts is not None else self._alloc_acts(n)
         nparts = max(1, min(256, (n + 31) // 32))   # workgroups of the weight gradients, at least 32 points each
-        gw = grads if grads is not None else dict(gy=torch.empty((n, O), dtype=torch.float32, device=self.dev),
-                                                  ga=torch.empty((n, H), dtype=torch.float32, device=self.dev),
-                                                  gz=torch.empty((n, H), dtype=torch.float32, device=self.dev),
-                                                  part=torch.empty(nparts * self.nparam, dtype=torch.float32,
-                                                                   device=self.dev),
-                                                  partial=torch.empty((n * O + 255) // 256, dtype=torch.float64,
-                                                                      device=self.dev))
+        gw = self._grads(n, nparts * self.nparam, grads)
         L.call("ephip_mlp_train_step", n, L.ptr(xk), self.nf2, L.ptr(self.mvec), H, O, L.ptr(self.p), L.ptr(target),
                L.ptr(a["f"]), L.ptr(a["z1"]), L.ptr(a["a1"]), L.ptr(a["z2"]), L.ptr(a["a2"]), L.ptr(a["y"]),
                L.ptr(gw["gy"]), L.ptr(gw["ga"]), L.ptr(gw["gz"]), L.ptr(gw["partial"]), nparts, L.ptr(gw["part"]),
