@@ -591,13 +591,17 @@ class QBatchedAdapter(AbstractCalculator):
 class BatchGraph:
     """A captured sequence of outer-k batches (OuterKLoop.capture): ``replay()`` launches the recorded
     graph on the current stream. ``payloads`` are the batches' payload views into the loop's buffers as
-    the capture built them (after a replay, the last batch's is current)."""
+    the capture built them (after a replay, the last batch's is current). A replay writes the loop's stage-1 planes
+    by the graph's own plan, so the planes that eager batches left there are dropped."""
     graph: object
     starts: list
     n: int
     payloads: list
+    rr: object = None   # the loop's staged RR->kR
 
     def replay(self):
+        if self.rr is not None:
+            self.rr.invalidate()
         self.graph.replay()
 
 
@@ -801,7 +805,7 @@ class OuterKLoop:
             self.ft_timer = timer
             if self.rr is not None:
                 self.rr.invalidate()
-        return BatchGraph(graph, starts, n, payloads)
+        return BatchGraph(graph, starts, n, payloads, self.rr)
 
     def run_pipelined(self, starts, n: int, calculators=()):
         """Run the k batches starting at the surviving-k positions ``starts`` (n k each) on two streams of
