@@ -1035,9 +1035,10 @@ class OuterKLoop:
             self.run_kbatch(i0, min(self.nk_batch, k_stop - i0), calculators)
 
 
-def _repeats(r) -> bool:
-    """The list names an R more than once. The direct sums add both; a box's index map holds one column per R."""
-    return len(np.unique(r, axis=0)) < len(r)
+def _repeats(r, lo, n) -> bool:
+    """The list names an R of its box (n from lo) more than once. The direct sums add both; a box's index map holds one
+    column per R."""
+    return bool(np.bincount(np.ravel_multi_index((r - lo).T, n)).max() > 1)
 
 
 def _differ(a, b) -> bool:
@@ -1069,10 +1070,9 @@ class _GridOptKR:
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         kg = np.asarray(st.kgrid, dtype=np.int64)
-        if _repeats(r):
-            return None
         if (len(ks) == 0 or n[0] > cls.N1_MAX or n[1] > cls.N23_MAX or n[2] > cls.N23_MAX
-                or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)):
+                or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)
+                or _repeats(r, lo, n)):
             return None
         x = st.el.xk.index_select(0, st.ksurv).cpu().numpy()
         i1, i2 = ks // (kg[1] * kg[2]), (ks // kg[2]) % kg[1]
@@ -1298,7 +1298,7 @@ class _GridOptKQ:
         lo, hi = r.min(0), r.max(0)
         n = hi - lo + 1
         m = np.asarray(st.qgrid, dtype=np.int64)
-        if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535 or _repeats(r):
+        if n[0] > 32 or n[1] > 8 or n[2] > 8 or m[1] > 64 or m[2] > 64 or m[0] > 65535 or _repeats(r, lo, n):
             return None
         xq = st.ph.xq.cpu().numpy()   # the grid's points in its order, third index fastest
         if len(xq) != m.prod() or _differ(xq, np.stack(np.unravel_index(np.arange(len(xq)), m), axis=1) / m):
