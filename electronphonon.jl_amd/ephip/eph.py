@@ -1044,7 +1044,7 @@ def _repeats(r, lo, n) -> bool:
 def _differ(a, b) -> bool:
     """Some coordinates differ by more than whole cells (and what FP32 phases resolve)."""
     d = np.asarray(a) - b
-    return bool(np.abs(d - np.rint(d)).max(initial=0.0) > 1e-10)
+    return bool(d.any() and np.abs(d - np.rint(d)).max() > 1e-10)
 
 
 class _GridOptKR:
@@ -1074,16 +1074,10 @@ class _GridOptKR:
                 or (st.nbw > cls.NBW_MAX and not general) or st.nw > 32 or (general and not small and n.max() <= cls.SMALL_BOX)
                 or _repeats(r, lo, n)):
             return None
-        x = st.el.xk.index_select(0, st.ksurv).cpu().numpy()
-        i1, i2 = ks // (kg[1] * kg[2]), (ks // kg[2]) % kg[1]
-        for c, at in ((0, i1), (1, i1 * kg[1] + i2)):   # one coordinate per plane and per line
-            of = np.zeros(int(at.max()) + 1)
-            of[at] = x[:, c]
-            if _differ(x[:, c], of[at]):
-                return None
-        return cls(st, ks, nd, r, lo, n, kg, x[:, 0], mfma, general)
+        go = cls(st, ks, nd, r, lo, n, kg, mfma, general)
+        return go if go.regular else None
 
-    def __init__(self, st, ks, nd, r, lo, n, kg, x1, mfma, general=False):
+    def __init__(self, st, ks, nd, r, lo, n, kg, mfma, general=False):
         torch = _torch()
         dev = st.el.xk.device
         self.nd = self.nd_max = nd   # rows in use, and what the plane buffers hold
@@ -1125,8 +1119,14 @@ class _GridOptKR:
         # planes with surviving k in order of their first one, their k1 coordinates, and the stage-1 group of each
         first_line = np.sort(np.unique(self.line_plane, return_index=True)[1])
         self.planes = [int(p) for p in self.line_plane[first_line]]
-        self.plane_x1 = {p: float(x1[starts[l]]) for p, l in zip(self.planes, first_line)}
+        x1, x2 = st.el.xk.index_select(0, st.ksurv).cpu().numpy().T[:2]
+        at1 = x1[starts[:-1]]
+        self.plane_x1 = {p: float(at1[l]) for p, l in zip(self.planes, first_line)}
         self.plane_pos = {p: i for i, p in enumerate(self.planes)}
+        # one coordinate per plane and per line, as the points of a grid (shifted or not) have
+        k_of_line = np.diff(starts)
+        self.regular = not (_differ(x1, np.repeat(at1, k_of_line)) or _differ(x2, np.repeat(x2[starts[:-1]], k_of_line))
+                            or _differ(at1, [self.plane_x1[p] for p in self.line_plane.tolist()]))
         self.cache = []  # [group, {plane: buffer}, buffers], most recent last, at most two
         self.next_k = 0  # the general form: one past the last batch's k
 
