@@ -354,7 +354,7 @@ def main():
         results["plain"] = dict(value=nks * args.qtile * steps / el, ms_per_step=1e3 * el / steps, steps=steps,
                                 ft_tflops=sum(flops) / sum(durs) / 1e12, ft_avg_ms=1e3 * sum(durs) / len(durs),
                                 ft_flop_per_launch=sum(flops) / len(flops),
-                                kernel="ft_mfma_kernel<float,128> (Rq->kq Fourier over Re)")
+                                kernel="ft32_kernel (Rq->kq Fourier over Re, FP32 MFMA)")
         log(f"[bench] plain outer-q fp32: {results['plain']['value']:.3e} pairs/s, FT "
             f"{results['plain']['ft_tflops']:.1f} TFLOP/s")
         del loop
@@ -559,7 +559,7 @@ def main():
                 name = KERNEL_NAMES.get((stage, var[stage])) or (
                     f"ft_bf16p_kernel (packed split-BF16, variant {var[stage]}), RR->kR Fourier over Re")
             else:
-                name = "ft_mfma_kernel<float,128>, RR->kR Fourier over Re"
+                name = "ft32_kernel, RR->kR Fourier over Re"
             dom = (name + " (k batch)", r["rrkr_tflops"], r["rrkr_avg_ms"], r["rrkr_flop_per_launch"], stage)
         else:
             if _staged(var[stage]) or r.get("fused_rotation"):

@@ -213,8 +213,8 @@ __global__ __launch_bounds__(256) void heev_c32_kernel(int n, int64_t nb, const 
             const float f = s * de.im, bb = c * de.im;
             float r, y;
             if (fminf(fabsf(f), fabsf(g)) > 0x1p-60f && fmaxf(fabsf(f), fabsf(g)) < 0x1p60f) {
-                // what hypotf and the divisions give where nothing has to be scaled: the quotients by Newton's
-                // iteration and Markstein's correction, which rounds them correctly, from one reciprocal
+                // nothing has to be scaled: r by the hardware's square root, about an ulp from hypotf's, and f / r and
+                // g / r for that r by Newton's iteration and Markstein's correction from one reciprocal
                 r = __builtin_amdgcn_sqrtf(fma(f, f, g * g));
                 y = __builtin_amdgcn_rcpf(r);
                 y = fma(fma(-r, y, 1.f), y, y);

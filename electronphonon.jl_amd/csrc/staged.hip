@@ -209,8 +209,8 @@ __host__ inline size_t sp_lds_bytes(int n, int nwave, int max_pairs) {
 // each (band, mode) from memory it took most of the kernel's time).
 // Against the direct sums and the rotation kernel (g(k, q) stored and read back), ms: 4 orbitals, 3 modes, 7^3 boxes,
 // q 24^3, 2794 units 17.5 -> 1.0; 12 orbitals, 9 modes, 5^3, q 18 x 15 x 12, 1260 units 3.7 -> 1.0; 16 orbitals, 12
-// modes, 5 window bands, 5^3, q 8^3, 10505 units 19.0 (split-BF16) -> 8.6. The VALU is 40% busy: what bounds it is the
-// chain of latencies and barriers of a workgroup whose slab is small.
+// modes, 5 window bands, 5^3, q 8^3, 10505 units 19.0 (split-BF16) -> 8.6. Bound by the chain of latencies and
+// barriers of a workgroup whose slab is small: waves wait 55% of their time, the VALU is 57% busy (4 orbitals).
 // Kept q are taken in segments: at most NQ tb entries and lines together and at most ls non-empty lines (the size
 // of B2); a line may be cut. The pitch of a line in B2 is 16 bytes over a multiple of 16, so the lines that the
 // lanes of a wave read lie in different banks.
@@ -640,8 +640,8 @@ __global__ __launch_bounds__(512) void staged_kq_kernel(SqArgs a) {
 // ms, staged_kq_kernel -> this: 16 orbitals, 12 modes, 5^3 boxes, 5 window bands, q 8^3, 10505 units 8.7 -> 5.0 (5.9 with
 // parts of 64 and the row of u_ph read as it was used; 5.5 at four waves a SIMD, which spill); 12 orbitals, 9 modes,
 // q 18 x 15 x 12, 1260 units 1.09 -> 0.82. Whole passes: 12, 12, 5^3, q 16^3, 3 bands 12.3 -> 4.5; 10, 15, q 20^3
-// 5.6 -> 2.7; 12, 12, 7^3, q 12^3 3.56 -> 3.25. Waves wait for the staging and its barriers 55% of their time; VALU
-// 45% busy, MFMAs 9%.
+// 5.6 -> 2.7; 12, 12, 7^3, q 12^3 3.56 -> 3.25. Waves wait for the staging and its barriers 54% of their time; VALU
+// 46% busy, MFMAs 9% (5 window bands; 42%, 53%, 13% at 12 orbitals).
 constexpr int LQ_ENT = 96, LQ_TP = 18, LQ_SLAB = 4096;  // LQ_SLAB: words of the tables of a slab
 
 __host__ inline size_t lq_lds_bytes(const SqArgs &a, int jl) {

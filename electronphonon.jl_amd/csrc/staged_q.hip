@@ -6,8 +6,8 @@
 //     ephip_staged_project with columns g = i + nw (nu + nm q)), where the phase sums over Re cost 8 nw^2 nm nr flops
 //     per (k, q);
 //   * the k+q-window rotation and g2 of every (k, q) of the tile (staged_rq_rotate_kernel).
-// 16 q, 5735 k, 16 orbitals, 12 modes, 7^3 boxes: 11.5 ms with the phase sums at every k, 1.45 here (0.65 RR->Rq, 0.71
-// stages 1 to 3, 0.06 window rotation).
+// 16 q, 5735 k, 16 orbitals, 12 modes, 7^3 boxes: 11.5 ms with the phase sums at every k, 1.33 here (0.71 RR->Rq, 0.61
+// stages 1 to 3, 0.07 window rotation).
 #include "common.hpp"
 
 namespace ephip {

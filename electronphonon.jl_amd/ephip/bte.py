@@ -568,8 +568,8 @@ def run_transport(model, kgrid, qgrid, window, params: ElectronTransportParams, 
     core.synchronize(backend)
     t["setup"] = time.perf_counter() - t0
     t0 = time.perf_counter()
-    # without the general staged kernels: the FP64 rates and conductivities keep the digits that the FP32 elements
-    # of the direct kernels give (another order of the FP32 sums moves them by 3e-8)
+    # without the general staged kernels: the FP64 rates and conductivities keep the digits that the FP32 elements of
+    # the direct kernels give (another order of the FP32 sums moves them by 3e-8; these are 8e-8 from 64 bits)
     loop = eph.OuterKLoop(st, nk_batch=nk_batch, precision=precision, staged=False)
     calc = BoltzmannCalculator(params, smearing=smearing, occupation_method=occupation_method)
     run_boltzmann(loop, calc)

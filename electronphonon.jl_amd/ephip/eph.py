@@ -620,8 +620,10 @@ class OuterKLoop:
                  nk_batch_cap: int = 512, fuse_rotation: bool = True, fuse_projection: bool = True,
                  gridopt: bool = True, gridopt_mfma: bool = True, with_ep: bool = False, staged: bool = True):
         """``gridopt``: the staged transforms (GridOpt) of the shapes that csrc/gridopt.hip covers. ``staged``: with
-        it, those of every other shape (csrc/staged.hip). Both evaluate the same sums in FP32; they differ in the
-        order of the additions, about 3e-8 of a scattering rate."""
+        it, those of every other shape (csrc/staged.hip). Staged and direct forms evaluate the same sums in FP32 and
+        differ in the order of the additions: g2 is about 2e-7 from the 64-bit result by the staged ones, 3e-7 to 7e-7
+        by the direct ones, and FP64 rates formed from the two differ by about 3e-8. Points or R that are no grid or box
+        (a list of q, a repeated R) take the direct sums."""
         torch = _torch()
         self.st = st
         dev = st.el.xk.device
@@ -645,13 +647,18 @@ class OuterKLoop:
                 self.gridopt = staged_kr(general=True)
             if self.gridopt is None:
                 self.gridopt = staged_kr(mfma=gridopt_mfma)
-        # kR->kq as the staged transform over the uniform q grid with the rotations and g2 fused (FP32)
+        # kR->kq as the staged transform over the uniform q grid with the rotations and g2 fused (FP32). 16 orbitals, up to
+        # four bands; the general form in its place, ms: 5.85 -> 11.1 (12 modes, 7^3 boxes, k = q = 20^3), 4.65 -> 5.8
+        # (5^3), 1.06 -> 1.72 and 0.78 -> 0.77 (three bands, 10^3)
         self.gridopt_q = _GridOptKQ.build(st) if (gridopt and nw == 16 and nm <= 16 and st.nbw <= 4) else None
         # the same transforms for the shapes that the two do not cover (other nw, more modes, wider windows)
         self.staged_k = staged_kr(general=True) if (staged and self.gridopt is None) else None
         self.staged_q = _GridOptKQ.build(st, general=True) if (staged and self.gridopt_q is None) else None
         # the lane-private projection adds in another order than the MFMA tiles: boxes of 27 R and callers without the
-        # general staged kernels keep the digits that FP64 rates are held to (_GridOptKR.SMALL_BOX)
+        # general staged kernels keep the digits of the tiles (_GridOptKR.SMALL_BOX). Elsewhere 16 orbitals take the lanes,
+        # whose g2 is nearer to 64 bits (1.8e-7 to 2.2e-7 for 2.1e-7 to 2.5e-7). RR->kR of 12 modes, 7^3 boxes, 1152-k
+        # batches, lanes / tiles, ms: 4.3 / 6.3 at 3.5 units a line, 5.6 / 6.6 at 9, 8.1 / 8.1 at 18; longer lines fill
+        # the tiles: 10.4 / 9.7 at 27, 15.4 / 13.2 at 47 (but 0.147 / 0.170 whole passes of 3 modes, 5^3, at 40)
         if self.gridopt is not None and not self.gridopt.general and (not staged or self.gridopt.box <= 3):
             self.gridopt.jl = 0
         self.rr = self.gridopt if self.gridopt is not None else self.staged_k
@@ -1059,9 +1066,11 @@ class _GridOptKR:
     PLANES = 8
     PLANE_BYTES = 8 << 30   # plane buffers up to this are held without a look at the free memory
     LINE_UNITS = 128   # units of a line piece of the general form (ephip_staged_project)
-    # boxes of 27 R stay with the direct kernels: the staged ones are 1.0 to 5.5 times as fast there (7.1 -> 2.4 ms
-    # at 10 orbitals, 9 modes; 3.7 -> 3.6 at 16, 12), but their other order of the FP32 additions would move the FP64
-    # rates that consumers form from these payloads by 3e-8, where results are held to 1e-9
+    # The outer-k loop's boxes of 27 R stay with the direct kernels, to keep the digits that FP64 rates formed from their
+    # payloads have had: another order of the FP32 additions moves them by 3e-8. That is a choice, not a bound: larger
+    # boxes took the staged order, which is 1.0 to 5.5 times as fast here too (7.1 -> 2.4 ms at 10 orbitals, 9 modes;
+    # 3.7 -> 3.6 at 16, 12). run_transport asks for the same by staged=False at any box; the outer-q loop, whose g2 is its
+    # result, does not (small).
     SMALL_BOX = 3
 
     @classmethod
