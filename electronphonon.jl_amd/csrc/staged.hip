@@ -210,7 +210,7 @@ __host__ inline size_t sp_lds_bytes(int n, int nwave, int max_pairs) {
 // Against the direct sums and the rotation kernel (g(k, q) stored and read back), ms: 4 orbitals, 3 modes, 7^3 boxes,
 // q 24^3, 2794 units 17.5 -> 1.0; 12 orbitals, 9 modes, 5^3, q 18 x 15 x 12, 1260 units 3.7 -> 1.0; 16 orbitals, 12
 // modes, 5 window bands, 5^3, q 8^3, 10505 units 19.0 (split-BF16) -> 8.6. Bound by the chain of latencies and
-// barriers of a workgroup whose slab is small: waves wait 55% of their time, the VALU is 57% busy (4 orbitals).
+// barriers of a workgroup whose slab is small: waves wait 55% of their time, the VALU is 58% busy (4 orbitals).
 // Kept q are taken in segments: at most NQ tb entries and lines together and at most ls non-empty lines (the size
 // of B2); a line may be cut. The pitch of a line in B2 is 16 bytes over a multiple of 16, so the lines that the
 // lanes of a wave read lie in different banks.
