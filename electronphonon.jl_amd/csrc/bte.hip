@@ -184,7 +184,8 @@ struct BtePair {
             d = occ_boson(ek - ekq, T) + si;
         }
     }
-    // n: the mode's occupation factor; so = d1 f1o + d2 f2o, si = d2 f1i + d1 f2i (vanishing deltas left out)
+    // n: the mode's occupation factor; so = d1 f1o + d2 f2o, si = d2 f1i + d1 f2i (vanishing deltas left out, and g2 where
+    // both vanish, whatever the factors and g2 are)
     __device__ void add(double n, double d1, double d2, double pref, double &so, double &si) const {
         double f1o, f2o, f1i, f2i;
         if constexpr (METHOD == 1) {
@@ -200,8 +201,9 @@ struct BtePair {
         } else {
             f1o = c, f2o = -c, f1i = d, f2i = -d;
         }
-        so += ((d1 == 0.0 ? 0.0 : d1 * f1o) + (d2 == 0.0 ? 0.0 : d2 * f2o)) * pref;
-        si += ((d2 == 0.0 ? 0.0 : d2 * f1i) + (d1 == 0.0 ? 0.0 : d1 * f2i)) * pref;
+        const double pg = d1 == 0.0 && d2 == 0.0 ? 0.0 : pref;
+        so += ((d1 == 0.0 ? 0.0 : d1 * f1o) + (d2 == 0.0 ? 0.0 : d2 * f2o)) * pg;
+        si += ((d2 == 0.0 ? 0.0 : d2 * f1i) + (d1 == 0.0 ? 0.0 : d1 * f2i)) * pg;
     }
 };
 
@@ -295,7 +297,7 @@ __global__ __launch_bounds__(256) void bte_accumulate_tab_kernel(
 #pragma unroll
                 for (int y = 0; y < 4; y++) {
                     const bool in = nu0 + y < nm && !(w[y] < w_cut);  // else both deltas zero: nothing added
-                    const double pref = in ? pre2 * (double)g[y] : 0.0;
+                    const double pref = pre2 * (double)g[y];
                     double d1 = 0.0, d2 = 0.0;
 #pragma unroll
                     for (int x = 0; x < NT; x++) {
