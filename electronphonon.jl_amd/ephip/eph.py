@@ -720,7 +720,7 @@ class OuterKLoop:
         self.max_units_per_k = int(nb.max()) if len(nb) else 1
         self.unit_kpos = torch.from_numpy(np.repeat(np.arange(len(ks)), nb).astype(np.int32)).to(dev)
         self.unit_state = torch.from_numpy(np.repeat(ks, nb).astype(np.int64)).to(dev)
-        band = np.concatenate([np.arange(bmin[k] - 1, bmax[k]) for k in ks]) if len(ks) else np.zeros(0)
+        band = np.arange(self.k_unit_start[-1]) - np.repeat(self.k_unit_start[:-1] - (bmin[ks] - 1), nb)
         self.unit_band = torch.from_numpy(band.astype(np.int32)).to(dev)
         self.xk_surv = st.el.xk.index_select(0, st.ksurv).contiguous()
         self.nq = st.ph.xq.shape[0]
