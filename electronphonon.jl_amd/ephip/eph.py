@@ -261,6 +261,11 @@ def setup_outer_q(model, kgrid, qgrid, window, backend: core.GPUBackend, epmat_d
     return OuterQSetup(el, ph, ksurv, nbw, epmat_dev, irvec_el_dev, nw, nm, tuple(kgrid), tuple(qgrid))
 
 
+def _check_precision(precision):
+    if precision not in (L.PREC_FP32, L.PREC_BF16X3):
+        raise L.EphipError(f"unknown precision {precision}")
+
+
 class OuterQLoop:
     """The per-q body of _loop_eph_over_q_and_k_batched (src/calculator/run_eph_over_q_and_k.jl:
     526-610): RR->Rq for a tile of q, then for each q and k-batch: Fourier over Re at the surviving
@@ -271,6 +276,7 @@ class OuterQLoop:
         """``staged``: Rq->kq by per-axis partial sums over the grid (FP32, csrc/staged_q.hip) where the Re box fits;
         False, and other boxes, run the phase sums over Re at every k."""
         torch = _torch()
+        _check_precision(precision)
         self.st = st
         self.nk_batch = int(nk_batch)
         self.nq_tile = int(nq_tile)
@@ -625,6 +631,7 @@ class OuterKLoop:
         by the direct ones, and FP64 rates formed from the two differ by about 3e-8. Points or R that are no grid or box
         (a list of q, a repeated R) take the direct sums."""
         torch = _torch()
+        _check_precision(precision)
         self.st = st
         dev = st.el.xk.device
         nw, nm = st.nw, st.nm

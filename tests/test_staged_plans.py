@@ -247,3 +247,14 @@ def test_outer_q_reports_its_arithmetic_and_times_its_transforms(monkeypatch):
     loop.run_qtile(0, 5)
     assert [n for _, _, n in loop.ft_timer] == [50, 50, 20]   # (k, q) of each of the three k batches: 24 k, 5 q
     assert all(a.at + 1 == b.at for a, b, _ in loop.ft_timer)
+
+
+def test_unknown_precision_is_refused():
+    """The staged kernels run in FP32 whatever is asked for, but what is asked for has to exist, as for the direct ones."""
+    for nw in (5, 8):
+        st = _setup(nw, 3, (4, 2, 3))
+        st.epmat.op_r = torch.zeros((1, 1))
+        for make in (lambda p: eph.OuterQLoop(st, nq_tile=2, precision=p), lambda p: eph.OuterKLoop(st, precision=p)):
+            make(eph.L.PREC_BF16X3)
+            with pytest.raises(eph.L.EphipError, match="precision"):
+                make(7)
